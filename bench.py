@@ -509,21 +509,18 @@ def main():
     slab_b = slab_bytes(prob, info["nstick"], nb, 4)
     slab_fl = slab_flops(prob, info["kxmax"], nb)
     achieved = slab_b / (slab_ms * 1e-3) / 1e9
-    # FP32 square grids of the register-FFT sizes take k_slab_xy_reg (8 bands
-    # per z plane), others the LDS kernel k_slab_xy
-    reg = prob.grid[0] == prob.grid[1] and prob.grid[0] in (24, 30, 32, 36, 40, 48, 60, 64, 72)
-    # the autotuner's FP32 choice names the variant ("slab reg <lanes per y
-    # transform> <bands per plane>"): k_slab_xy_reg<float, n, n, bands, 2
-    # waves/SIMD, lanes[, 512 threads for the 16-band variant]>
-    # (" p": the persistent grid, k_slab_xy_reg_p)
-    mly = re.search(r"slab reg (\d) (\d+)( p)?", out["autotune"]["f32"])
-    reg = reg and (mly is not None or "slab lds" not in out["autotune"]["f32"])
-    ly, sb = (mly.group(1), int(mly.group(2))) if mly else ("1", 0)
-    # (a name prefix: the traced name carries the thread count too)
-    tail = ", 512" if sb == 16 else ""
-    kbase = "k_slab_xy_reg_p" if mly and mly.group(3) else "k_slab_xy_reg"
-    kname = (f"{kbase}<float, {prob.grid[0]}, {prob.grid[1]}, {sb or 8}, 2, {ly}{tail}" if reg
-             else f"k_slab_xy<float, {prob.grid[0]}, {prob.grid[1]}")
+    # the autotuner's FP32 choice names the kernel: "slab mm" the matrix-core
+    # transform k_slab_mm, "slab reg <lanes per y transform> 0" the register
+    # FFTs k_slab_xy_reg, "slab lds ..." the LDS kernel k_slab_xy (a name
+    # prefix: the traced name carries the other template arguments too)
+    tuned = out["autotune"]["f32"]
+    mly = re.search(r"slab reg (\d)", tuned)
+    if "slab mm" in tuned:
+        kname = "k_slab_mm<float"
+    elif mly:
+        kname = f"k_slab_xy_reg<float, {prob.grid[0]}, {prob.grid[1]}, 8, 2, {mly.group(1)}"
+    else:
+        kname = f"k_slab_xy<float, {prob.grid[0]}, {prob.grid[1]}"
     traffic, full = pmc_traffic(os.path.join(ROOT, "profiles", f"pmc_traffic_{prob.name}.md"), kname)
     kname = full or kname + ">"
 

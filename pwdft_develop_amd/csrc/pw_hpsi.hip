@@ -179,26 +179,15 @@ k_slab_xy(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restric
 // by scheduling barriers so that the compiler does not hoist all of them next
 // to the spectrum (that spills past the 256 VGPRs of two waves per SIMD).
 // Same arithmetic, in the same order, as k_slab_xy.
-// LY lanes per y column transform (1, 2 or 4); NT threads per workgroup.
-template <typename T, int N1, int N2, int SB, int LB, int LY, int NT = 256>
-__global__ void __launch_bounds__(NT, LB)  // LB waves per SIMD: <= 512 / LB registers
+// LY lanes per y column transform (1, 2 or 4).
+template <typename T, int N1, int N2, int SB, int LB, int LY>
+__global__ void __launch_bounds__(256, LB)  // LB waves per SIMD: <= 512 / LB registers
 k_slab_xy_reg(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restrict__ t2, int n3, int nstick,
               int kxmax, int nb, const int* __restrict__ pos, const int* __restrict__ mpos,
               const T* __restrict__ vtot) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  slab_xy_reg_body<T, N1, N2, SB, LY, NT>(blockIdx.x, blockIdx.y * SB, t1, t2, n3, nstick, kxmax, nb, pos, mpos,
+  slab_xy_reg_body<T, N1, N2, SB, LY>(blockIdx.x, blockIdx.y * SB, t1, t2, n3, nstick, kxmax, nb, pos, mpos,
                                           vtot, smem_raw);
-}
-
-// The same transform as a persistent grid over (plane, band group) items
-// with the next item prefetched (slab_xy_reg_persistent).
-template <typename T, int N1, int N2, int SB, int LB, int LY>
-__global__ void __launch_bounds__(256, LB)
-k_slab_xy_reg_p(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restrict__ t2, int n3, int nstick,
-                int kxmax, int nb, const int* __restrict__ pos, const int* __restrict__ mpos,
-                const T* __restrict__ vtot) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  slab_xy_reg_persistent<T, N1, N2, SB, LY, 256>(t1, t2, n3, nstick, kxmax, nb, pos, mpos, vtot, smem_raw);
 }
 
 // ---------------------------------------------------------------- kernel 3
@@ -358,34 +347,14 @@ auto slab_kernel(int n1, int n2) -> decltype(&k_slab_xy<T, 0, 0>) {
 // second workgroup either), two waves up to 48 points, one beyond (the
 // 60-point double FFT pair needs about 350 registers)
 template <typename T> struct SlabCfg { static constexpr int SB = 8; };
-constexpr int kSlabWideSB = 16;  // the wide FP32 variant: 16 bands per plane, 512 threads
 template <> struct SlabCfg<double> { static constexpr int SB = 4; };
 template <typename T, int N> constexpr int slab_lb() { return (sizeof(T) == 4 || N <= 48) ? 2 : 1; }
-// lanes per y column transform when no plan chooses
-template <typename T> static int default_slab_ly(int n) {
-  (void)n;
-  return 1;
-}
 #define PW_REG_SIZES(X) X(24) X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72)
 template <typename T>
 using slab_reg_fn = decltype(&k_slab_xy_reg<T, 24, 24, SlabCfg<T>::SB, 2, 1>);
 template <typename T, int N>
-static slab_reg_fn<T> slab_reg_ly(int ly, int sb, bool persist) {
+static slab_reg_fn<T> slab_reg_ly(int ly) {
   constexpr int SB = SlabCfg<T>::SB, LB = slab_lb<T, N>();
-  if (persist) {
-    // persistent variant: FP32 only (the FP64 prefetch registers spill),
-    // the default band count, one lane per column
-    if constexpr (sizeof(T) == 4) {
-      if (ly == 1 && sb == SB) return &k_slab_xy_reg_p<T, N, N, SB, LB, 1>;
-    }
-    return nullptr;
-  }
-  if (sb == kSlabWideSB) {
-    // FP32 planes up to 64 points: 16 bands per z plane, 512 threads
-    if constexpr (sizeof(T) == 4 && N <= 64)
-      if (ly == 1) return &k_slab_xy_reg<T, N, N, kSlabWideSB, 2, 1, 512>;
-    return nullptr;
-  }
   if (ly == 1) return &k_slab_xy_reg<T, N, N, SB, LB, 1>;
   if (ly == 2) return &k_slab_xy_reg<T, N, N, SB, LB, 2>;
   if constexpr (N % 4 == 0)
@@ -393,24 +362,22 @@ static slab_reg_fn<T> slab_reg_ly(int ly, int sb, bool persist) {
   return nullptr;
 }
 // the register slab kernel of an n1 x n2 plane with ly lanes per y column
-// transform and sb bands per z plane (<= 0: the defaults for the precision),
-// or null if there is none
+// transform (<= 0: one), or null if there is none
 template <typename T>
-static slab_reg_fn<T> slab_reg_kernel(int n1, int n2, int ly = 0, int sb = 0, bool persist = false) {
+static slab_reg_fn<T> slab_reg_kernel(int n1, int n2, int ly = 0) {
   if (n1 != n2) return nullptr;
-  if (ly <= 0) ly = default_slab_ly<T>(n1);
-  if (sb <= 0) sb = SlabCfg<T>::SB;
+  if (ly <= 0) ly = 1;
   switch (n1) {
 #define PW_CASE(n) \
   case n:          \
-    return slab_reg_ly<T, n>(ly, sb, persist);
+    return slab_reg_ly<T, n>(ly);
     PW_REG_SIZES(PW_CASE)
 #undef PW_CASE
     default:
       return nullptr;
   }
 }
-// LDS bytes of the register slab kernel at sb bands per plane
+// LDS bytes of the register slab kernel
 static size_t slab_reg_lds(const pw_ctx* c, size_t csz, int sb) {
   return csz * ((size_t)sb * (c->sp.kxmax + 1) * c->n2) + csz * (size_t)(c->n2 / 2) * (c->n1 + 1) +
          sizeof(int) * 2 * (size_t)c->sp.nstick;
@@ -664,15 +631,10 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
     const char* sl = getenv("PW_SLAB");
     for (auto& pl : c->plan) {
       pl.reg = !(sl && std::string(sl).compare(0, 3, "lds") == 0);
-      // "reg:<ly>[:<sb>][:p]": the register kernel with ly lanes per y
-      // column transform (sb bands per z plane; 16: the wide FP32 variant;
-      // p: on a persistent grid)
-      if (sl && std::string(sl).compare(0, 4, "reg:") == 0) {
-        pl.ly = std::max(1, atoi(sl + 4));
-        const char* b = strchr(sl + 4, ':');
-        if (b) pl.sb = std::max(0, atoi(b + 1));
-        pl.persist = strstr(sl + 4, ":p") != nullptr;  // ":p": the persistent grid
-      }
+      pl.mm = pl.reg;
+      // "reg[:<ly>...]": the transforms held in registers (on matrix cores or
+      // as register FFTs with ly lanes per y column), as by default
+      if (sl && std::string(sl).compare(0, 4, "reg:") == 0) pl.ly = std::max(1, atoi(sl + 4));
       // "lds:<g>[:<r>]": the LDS kernel with its large-plane layout, g y
       // columns per group (and r x row pairs per step)
       if (sl && std::string(sl).compare(0, 4, "lds:") == 0) {
@@ -738,35 +700,48 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
     pw_ctx_destroy(c);
     return rc;
   }
-#define UP(d, h, n)                                       \
-  if ((rc = upload(&(d), (h), (n))) != PW_OK) {           \
-    pw_ctx_destroy(c);                                    \
-    return rc;                                            \
-  }
-  UP(c->d_pt_idx, c->sp.pt_idx.data(), c->sp.pt_idx.size());
-  UP(c->d_pt_sz, c->sp.pt_sz.data(), c->sp.pt_sz.size());
-  UP(c->d_chunk_off, c->sp.chunk_off.data(), c->sp.chunk_off.size());
-  UP(c->d_gpt_idx, c->sp.gpt_idx.data(), c->sp.gpt_idx.size());
-  UP(c->d_gpt_sz, c->sp.gpt_sz.data(), c->sp.gpt_sz.size());
-  UP(c->d_gchunk_off, c->sp.gchunk_off.data(), c->sp.gchunk_off.size());
-  UP(c->d_zs, c->sp.zs.data(), c->sp.zs.size());
-  UP(c->d_pos, c->sp.pos.data(), c->sp.pos.size());
-  UP(c->d_mpos, c->sp.mpos.data(), c->sp.mpos.size());
-  UP(c->d_ekin, ekin, (size_t)npw);
-  UP(c->d_teter, teter, (size_t)npw);
+  // the context's index tables and vectors: one device allocation, one copy
   {
-    std::vector<float> ef(ekin, ekin + npw), tf(teter, teter + npw);
-    UP(c->d_ekin_f, ef.data(), ef.size());
-    UP(c->d_teter_f, tf.data(), tf.size());
+    std::vector<unsigned char> host;
+    std::vector<std::pair<void**, size_t>> place;
+    auto add = [&](auto** d, const auto* h, size_t n) {
+      const size_t at = (host.size() + 255) / 256 * 256, bytes = sizeof(*h) * n;
+      host.resize(at + std::max<size_t>(bytes, 1));
+      if (bytes) memcpy(host.data() + at, h, bytes);
+      place.push_back({(void**)d, at});
+    };
+    add(&c->d_pt_idx, c->sp.pt_idx.data(), c->sp.pt_idx.size());
+    add(&c->d_pt_sz, c->sp.pt_sz.data(), c->sp.pt_sz.size());
+    add(&c->d_chunk_off, c->sp.chunk_off.data(), c->sp.chunk_off.size());
+    add(&c->d_gpt_idx, c->sp.gpt_idx.data(), c->sp.gpt_idx.size());
+    add(&c->d_gpt_sz, c->sp.gpt_sz.data(), c->sp.gpt_sz.size());
+    add(&c->d_gchunk_off, c->sp.gchunk_off.data(), c->sp.gchunk_off.size());
+    add(&c->d_zs, c->sp.zs.data(), c->sp.zs.size());
+    add(&c->d_pos, c->sp.pos.data(), c->sp.pos.size());
+    add(&c->d_mpos, c->sp.mpos.data(), c->sp.mpos.size());
+    add(&c->d_ekin, ekin, (size_t)npw);
+    add(&c->d_teter, teter, (size_t)npw);
+    const std::vector<float> ef(ekin, ekin + npw), tf(teter, teter + npw);
+    add(&c->d_ekin_f, ef.data(), ef.size());
+    add(&c->d_teter_f, tf.data(), tf.size());
     std::vector<double> tw;
     roots(c->n1, tw);
     roots(c->n2, tw);
     roots(c->n3, tw);
-    std::vector<float> twf(tw.begin(), tw.end());
-    UP(c->d_tw64, tw.data(), tw.size());
-    UP(c->d_tw32, twf.data(), twf.size());
+    const std::vector<float> twf(tw.begin(), tw.end());
+    add(&c->d_tw64, tw.data(), tw.size());
+    add(&c->d_tw32, twf.data(), twf.size());
+    if (hipMalloc(&c->d_tables, host.size()) != hipSuccess ||
+        hipMemcpy(c->d_tables, host.data(), host.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      pw_ctx_destroy(c);
+      return fail(PW_ERR_HIP, "pw_ctx_create: cannot upload %zu bytes of tables", host.size());
+    }
+    for (const auto& e : place) *e.first = (unsigned char*)c->d_tables + e.second;
   }
-#undef UP
+  if ((rc = mm_plan(c)) != PW_OK) {
+    pw_ctx_destroy(c);
+    return rc;
+  }
   c->tbytes = sizeof(double2) * (size_t)max_bands * c->n3 * c->sp.nstick;
   if (hipMalloc(&c->d_t1, c->tbytes) != hipSuccess || hipMalloc(&c->d_t2, c->tbytes) != hipSuccess) {
     pw_ctx_destroy(c);
@@ -785,10 +760,9 @@ extern "C" int pw_ctx_destroy(pw_ctx* c) {
   if (!c) return PW_OK;
   pw_free_workspace(c);
   exx_free(c);
+  mm_free(c);
   if (c->d_gemm_ws) (void)hipFree(c->d_gemm_ws);
-  void* ptrs[] = {c->d_pt_idx, c->d_pt_sz, c->d_chunk_off, c->d_gpt_idx, c->d_gpt_sz, c->d_gchunk_off, c->d_zs,
-                  c->d_pos, c->d_mpos, c->d_ekin, c->d_teter, c->d_ekin_f, c->d_teter_f, c->d_tw64,
-                  c->d_tw32, c->d_vtot, c->d_vtot_f, c->d_beta, c->d_betaw, c->d_W, c->d_beta_f,
+  void* ptrs[] = {c->d_tables, c->d_vtot, c->d_vtot_f, c->d_beta, c->d_betaw, c->d_W, c->d_beta_f,
                   c->d_betaw_f, c->d_W_f, c->d_t1, c->d_t2, c->d_betaw_bf, c->d_W_bf};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -830,6 +804,7 @@ extern "C" int pw_set_vtot(pw_ctx* c, const double* vtot) {
   }
   PW_HIP(hipMemcpy(c->d_vtot, v.data(), sizeof(double) * c->N, hipMemcpyHostToDevice));
   PW_HIP(hipMemcpy(c->d_vtot_f, vf.data(), sizeof(float) * c->N, hipMemcpyHostToDevice));
+  PW_TRY(mm_potential(c));
   c->have_vtot = true;
   return PW_OK;
 }
@@ -914,6 +889,28 @@ static size_t slab_lds(const pw_ctx* c, int esz, int rp, int cg) {
   return esz * (n1 + n2 + nk * n2 + std::max((size_t)cg * n2, 2 * (size_t)rp * n1));
 }
 
+// Whether the matrix-core slab kernel is the faster one for nb bands; it is
+// against the LDS kernel (no register FFT for the plane) on every plane tried:
+// 45 x 45 FP32 207 -> 47 us, FP64 259 -> 81 us at 256 bands.  Against the
+// register FFT (us at 256 / 32 / 8 bands, FFT -> matrix cores):
+//   FP32 24: 19 -> 15 / - / 16 -> 7      FP64 38 -> 22 / - / 17 -> 8
+//        32: 24 -> 27 / 17 -> 9 / 17 -> 8     66 -> 44 / 18 -> 11 / 18 -> 10
+//        36: 30 -> 35 / 17 -> 12 / 17 -> 9    83 -> 55 / 22 -> 16 / 18 -> 11
+//        40: 40 -> 42                        103 -> 69
+//        48: 58 -> 49 / 22 -> 13 / 20 -> 10  141 -> 82 / 29 -> 20 / 22 -> 12
+//        60: 94 -> 71 / 26 -> 17 / 24 -> 11  348 -> 124 / 54 -> 26 / 28 -> 14
+//        64: 201 -> 121                      438 -> 224
+//        72: 309 -> 250 / 72 -> 51 / 39 -> 22   655 -> 675 / 117 -> 125 / 41 -> 46
+// The quarter plane is padded to 16-row tiles: 32..40 points (17..21 rows)
+// pay most for it, which only FP32 with the whole chip busy loses, and at 72
+// FP64 points (37 rows, 18 columns) one wave per SIMD holds the tiles.
+template <typename T>
+static bool mm_wins(const pw_ctx* c, int nb) {
+  if (!slab_reg_kernel<T>(c->n1, c->n2)) return true;
+  if (sizeof(T) == 4) return !(c->n1 >= 32 && c->n1 <= 40 && (long)nb * c->n3 >= 5000);
+  return c->n1 < 72;
+}
+
 template <typename T>
 static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
   typedef typename cx<T>::t C;
@@ -965,52 +962,35 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
     }
     if (!found) { rp = 1; cg = 1; }
   }
-  // one or two bands (the Lanczos steps): the LDS kernel with all y columns
-  // in one group and all x row pairs in one step at 512 threads spreads each
-  // plane's transforms over the workgroup, where the register kernel leaves
-  // most of its threads idle (si64_60, one band: FP32 13.6 us against 24.0,
-  // FP64 15.7 against 29.3)
+  const bool mm = pl.mm && mm_slab_ready<T>(c) && (pl.mm_only || mm_wins<T>(c, nb));
+  // one or two bands (the Lanczos steps) where the plane has no matrix-core
+  // kernel: the LDS kernel with all y columns in one group and all x row
+  // pairs in one step at 512 threads spreads each plane's transforms over the
+  // workgroup, where the register kernel leaves most of its threads idle
+  // (si64_60, one band: FP32 13.6 us against 24.0, FP64 15.7 against 29.3)
   const int nkc = c->sp.kxmax + 1, npr = (c->n2 + 1) / 2;
-  const bool few = nb <= 2 && slab_lds(c, esz, npr, nkc) <= 160 * 1024;
+  const bool few = !mm && nb <= 2 && slab_lds(c, esz, npr, nkc) <= 160 * 1024;
   if (few) {
     cg = nkc;
     rp = npr;
   }
   const size_t lds2 = slab_lds(c, esz, rp, cg);
+  const slab_reg_fn<T> kreg = pl.reg && !few ? slab_reg_kernel<T>(c->n1, c->n2, pl.ly) : nullptr;
   if (lds2 > 160 * 1024)
     return fail(PW_ERR_UNSUPPORTED, "H*psi slab needs %zu bytes of LDS (> 160 KiB)", lds2);
   const size_t lds1 = (size_t)esz * (c->n3 + 2 * (size_t)sc * c->n3);
   PW_TRY(mark(c, 0));
   PW_TRY(launch_inv_z<T>(c, nb, (const C*)psi, t1, tw3));
   PW_TRY(mark(c, 1));
-  // the wide variant only where its y-space fits the LDS
-  const bool wide = pl.sb == kSlabWideSB && slab_reg_lds(c, sizeof(C), kSlabWideSB) <= 160 * 1024;
-  // the persistent grid where that variant exists, else the one-item grid
-  slab_reg_fn<T> kreg =
-      pl.reg && !few && pl.persist && !wide ? slab_reg_kernel<T>(c->n1, c->n2, pl.ly, 0, true) : nullptr;
-  const bool persist = kreg != nullptr;
-  if (pl.reg && !few && !kreg) kreg = slab_reg_kernel<T>(c->n1, c->n2, wide ? 1 : pl.ly, wide ? kSlabWideSB : 0);
-  if (kreg) {
-    // one z plane of SB bands per workgroup (or per item of the persistent
-    // grid), V plane + y-space in LDS
-    const int SB = wide ? kSlabWideSB : SlabCfg<T>::SB;
+  if (mm) {
+    PW_TRY(mm_slab<T>(c, nb, t1, t2));
+  } else if (kreg) {
+    // one z plane of SB bands per workgroup, V plane + y-space in LDS
+    constexpr int SB = SlabCfg<T>::SB;
     const size_t ldsr = slab_reg_lds(c, sizeof(C), SB);
     PW_TRY(ensure_lds((const void*)kreg, ldsr));
-    dim3 grid(c->n3, (nb + SB - 1) / SB);
-    if (persist) {
-      // as many workgroups as the device holds at once
-      pw_ctx::Plan& pm = c->plan[sizeof(T) == 8 ? PW_F64 : PW_F32];
-      if (pm.pkern != (const void*)kreg || pm.plds != ldsr) {
-        int per_cu = 0, ncu = 0;
-        PW_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kreg, 256, ldsr));
-        PW_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
-        pm.pkern = (const void*)kreg;
-        pm.plds = ldsr;
-        pm.pgrid = std::max(1, per_cu) * std::max(1, ncu);
-      }
-      grid = dim3((unsigned)std::min<long>((long)grid.x * grid.y, pm.pgrid));
-    }
-    hipLaunchKernelGGL(kreg, grid, dim3(wide ? 512 : 256), ldsr, c->stream, (const C*)t1, (C*)t2, c->n3,
+    const dim3 grid(c->n3, (nb + SB - 1) / SB);
+    hipLaunchKernelGGL(kreg, grid, dim3(256), ldsr, c->stream, (const C*)t1, (C*)t2, c->n3,
                        c->sp.nstick, c->sp.kxmax, nb, c->d_pos, c->d_mpos, (const T*)vt);
   } else {
     auto kslab = slab_kernel<T>(c->n1, c->n2);
@@ -1032,10 +1012,12 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
   return PW_OK;
 }
 
-bool has_reg_slab(const pw_ctx* c, int dtype, int ly, int sb, bool persist) {
-  if (sb == kSlabWideSB && slab_reg_lds(c, dtype == PW_F64 ? 16 : 8, sb) > 160 * 1024) return false;
-  return dtype == PW_F64 ? slab_reg_kernel<double>(c->n1, c->n2, ly, sb, persist) != nullptr
-                         : slab_reg_kernel<float>(c->n1, c->n2, ly, sb, persist) != nullptr;
+bool has_reg_slab(const pw_ctx* c, int dtype, int ly) {
+  return dtype == PW_F64 ? slab_reg_kernel<double>(c->n1, c->n2, ly) != nullptr
+                         : slab_reg_kernel<float>(c->n1, c->n2, ly) != nullptr;
+}
+bool has_mm_slab(const pw_ctx* c, int dtype) {
+  return dtype == PW_F64 ? mm_slab_ready<double>(c) : mm_slab_ready<float>(c);
 }
 size_t slab_lds_bytes(const pw_ctx* c, int esz, int rp, int cg) { return slab_lds(c, esz, rp, cg); }
 

@@ -211,11 +211,11 @@ template <typename T>
 int sticks_to_sphere_add(pw_ctx* c, int nb, const void* t2, void* out);
 // Slab-kernel facts for the autotuner (pw_hpsi.hip): whether the
 // register-FFT kernel exists for the context's planes in dtype with ly
-// lanes per y column transform and sb bands per plane (<= 0: the defaults;
-// sb = 16: the wide FP32 variant, where its LDS fits; persist: the
-// persistent-grid variant), and the LDS bytes of
-// the LDS kernel at (rp, cg) for complex elements of esz bytes.
-bool has_reg_slab(const pw_ctx* c, int dtype, int ly = 0, int sb = 0, bool persist = false);
+// lanes per y column transform (<= 0: one), whether the matrix-core kernel
+// does, and the LDS bytes of the LDS kernel at (rp, cg) for complex elements
+// of esz bytes.
+bool has_reg_slab(const pw_ctx* c, int dtype, int ly = 0);
+bool has_mm_slab(const pw_ctx* c, int dtype);
 // the context's second stream and fork / join events (created on first use)
 int side_stream(pw_ctx* c);
 size_t slab_lds_bytes(const pw_ctx* c, int esz, int rp, int cg);
@@ -224,6 +224,17 @@ size_t slab_lds_bytes(const pw_ctx* c, int esz, int rp, int cg);
 // (d_coef / d_coef_f) at 3 step; Yp == null for the first step.  HY is
 // scratch (the local, kinetic and exchange terms).
 int cheb_step_apply(pw_ctx* c, int dtype, int nb, const void* Y, void* HY, const void* Yp, void* Ynew, int step);
+// The xy slab transform on matrix cores (pw_slab_mm.hip): per-context plan
+// (created with the context where it covers the sphere), the potential in
+// its operand order (after every pw_set_vtot), the launch t1 -> t2.
+struct SlabMm;
+int mm_plan(pw_ctx* c);
+int mm_potential(pw_ctx* c);
+void mm_free(pw_ctx* c);
+template <typename T>
+bool mm_slab_ready(const pw_ctx* c);
+template <typename T>
+int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2);
 // Exact exchange (pw_exx.hip): a3 += V_x psi when the context holds an
 // exchange operator; state freed with the context.
 struct ExxState;
@@ -237,6 +248,7 @@ void exx_free(pw_ctx* c);
 }  // namespace pw
 
 struct pw_ctx {
+  pw::SlabMm* mm = nullptr;     // matrix-core slab plan, where there is one
   pw::ExxState* exx = nullptr;  // screened exchange operator, when set
   void* d_gemm_ws = nullptr;  // split-K partial tiles
   size_t gemm_ws_bytes = 0;
@@ -256,7 +268,8 @@ struct pw_ctx {
   std::vector<int> h_idx;       // idxCoarseCut, host copy
   std::vector<double> h_wgt;    // projector weights, host copy
   std::vector<int> f1, f2, f3;  // radix plans
-  // device arrays
+  // device arrays (d_pt_idx ... d_tw32 lie in d_tables)
+  void* d_tables = nullptr;
   int *d_pt_idx = nullptr, *d_pt_sz = nullptr, *d_chunk_off = nullptr;
   int *d_gpt_idx = nullptr, *d_gpt_sz = nullptr, *d_gchunk_off = nullptr;
   int* d_zs = nullptr;  // StickPlan::zs
@@ -304,20 +317,17 @@ struct pw_ctx {
   int bf16_split = 3;
   bool zreg = false;  // PW_ZREG=1: the register z kernels where the z length has one
   // Plans per precision ([PW_F64], [PW_F32]), set by PW_SLAB or pw_autotune:
-  //   reg: the register-FFT slab kernel where compiled (PW_SLAB=lds: the LDS
-  //   kernel); cg / rp / threads: the LDS kernel's y column groups (0 = two
+  //   mm, reg: the matrix-core slab kernel, else the register-FFT one where
+  //   compiled (PW_SLAB=lds: the LDS kernel); cg / rp / threads: the LDS kernel's y column groups (0 = two
   //   y buffers), x row pairs per step, threads per workgroup (0 = the
   //   built-in rule; PW_SLAB=lds:<cg>:<rp>:<threads>); tn_tm / tn_cap: the
   //   split-K TN product's tile (1: 64 x 64, 2: 128 x 128) and the number of
   //   partial workgroups aimed at (0 = the built-in rule)
   struct Plan {
     bool reg = true;
-    int ly = 0;  // register kernel: lanes per y column transform (0: default)
-    int sb = 0;  // register kernel: bands per z plane (0: default; 16: wide FP32 variant)
-    bool persist = false;          // register kernel on a persistent grid (next item prefetched)
-    const void* pkern = nullptr;   // persistent grid size, for this kernel and LDS size
-    size_t plds = 0;
-    int pgrid = 0;
+    bool mm = true;        // the matrix-core slab kernel where it wins
+    bool mm_only = false;  // ... and wherever the context has its plan (the autotuner's choice)
+    int ly = 0;  // register kernel: lanes per y column transform (0: one)
     int cg = 0, rp = 0, threads = 0;
     int tn_tm = 0, tn_cap = 0;
   } plan[2];

@@ -1,0 +1,291 @@
+// The xy slab transform on matrix cores: one wavefront takes one z plane of
+// one band from its sticks to its sticks, every intermediate in registers.
+//
+// r(x, y) real is split by parity in x and in y.  With th_x = 2 pi / n1,
+// th_y = 2 pi / n2, E = Y(kx, ky) + Y(kx, -ky), O = Y(kx, ky) - Y(kx, -ky)
+// and c = 1 for kx = 0 and kx = n1 / 2, else 2, the four class matrices
+//   ee = c Re E,  oe = -c Im E,  eo = -c Im O,  oo = -c Re O   (x, y parity)
+// over 0 <= kx <= kxmax, 0 <= ky <= kymax give r as four REAL products
+//   r_ab = Ca_x A_ab Cb_y^T,   Ce = cos(th h k), Co = sin(th h k),
+//   r(+-x, +-y) = r_ee (+-)x r_oe (+-)y r_eo (+-)x(+-)y r_oo
+// over the quarter plane 0 <= x <= n1/2, 0 <= y <= n2/2, and the forward
+// transform is the transpose.  Against a dense transform that is a quarter
+// of the multiplications, and the sphere's pruning (kmax about n / 4) halves
+// the inner lengths again: at 60 x 60 with kmax 14 the padded products are
+// 394 kflop per plane against 167 kflop of butterflies, on units that do
+// twice (FP32) to eight times what the butterflies reached.
+//
+// Chain of v_mfma_*_16x16x4 per 16-row y tile, no LDS and no barrier between
+// the products: an accumulator (register i, lane group g) is the operand of
+// the next product's k-step i as it stands, as B operand or, transposed, as
+// A operand (both put the inner index in the lane group).
+//   1  D1[kx][y]  = A[kx][ky]   C_y[ky][y]      A = the class matrix
+//   2  D2[x][y]   = C_x[x][kx]  D1[kx][y]       B = D1
+//      pointwise: times V, itself split into its classes W (the product of
+//      classes a and b is of class a b, so out_a = sum_b W_ab r_b: 16
+//      multiply-adds per point of the quarter plane)
+//   3  D3[y][kx] += D2^T[y][x]  C_x[x][kx]      A = D2, over the x tiles
+//   4  D4[ky][kx] += C_y[ky][y] D3[y][kx]       B = D3, over the y tiles
+// Row r of an accumulator sits at (i, g) = (r / 4, r % 4) in FP64 but
+// (r % 4, r / 4) in FP32, so FP32 lanes carry the indices in the permuted
+// order perm(): then (i, g) holds index 4 i + g of its tile in both.
+//
+// Bound by the matrix pipes.  Constants (tables of {cos, sin}) come from LDS,
+// one read per four products; V from a copy in operand order.
+#pragma once
+#include <type_traits>
+
+#include "pw_fft.h"
+#include "pw_internal.h"
+
+namespace pw {
+
+template <typename T> struct MmV;
+template <> struct MmV<double> { typedef double t __attribute__((ext_vector_type(4))); };
+template <> struct MmV<float> { typedef float t __attribute__((ext_vector_type(4))); };
+
+__device__ __forceinline__ MmV<double>::t mm16(double a, double b, MmV<double>::t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ MmV<float>::t mm16(float a, float b, MmV<float>::t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// index within a 16-tile carried by lane c % 16
+template <typename T>
+__host__ __device__ __forceinline__ int mm_perm(int c) {
+  return sizeof(T) == 8 ? c : 4 * (c & 3) + (c >> 2);
+}
+
+// Stick entry of (kx, ky >= 0): x = stick of +ky, y = stick of -ky; kMmNone
+// where there is none, kMmConj set where the value is the conjugate of that
+// stick (the kx = 0 column, which stores one of each pair).
+constexpr int kMmNone = -1;
+constexpr int kMmConj = 1 << 30;
+
+// Device pointers and lengths of one context's plan in one precision.
+template <typename T>
+struct MmArgs {
+  const typename cx<T>::t *kx_t, *hx_t;  // x: [TX][KS][64] (k inner), [TK][4 TX][64] (h inner)
+  const typename cx<T>::t *ky_t, *hy_t;  // y, the same pointers where the tables agree
+  const int2* sp;                        // [TK][KS][64]
+  const typename MmV<T>::t* v;           // [z][TY][TX][4][64]: V / N as W_ee, W_oe, W_eo, W_oo
+  int TX, TY, XS, YS;                    // tiles and k-steps of the quarter plane
+  int n3, nstick, nb, half;              // half: n1 / 2 where n1 is even, else -1 (the kx with weight 1)
+  int shared;                            // the y tables are the x tables
+};
+
+// LDS bytes of the tables
+template <typename T>
+inline size_t mm_lds(int KS, int TX, int TY, bool shared) {
+  const int TK = (KS + 3) / 4;
+  const size_t tab = (size_t)(KS + 4 * TK) * (TX + (shared ? 0 : TY));
+  return 64 * (sizeof(typename cx<T>::t) * tab + sizeof(int2) * TK * KS);
+}
+
+// KS: k-steps (of 4) that cover kxmax + 1 and kymax + 1; NW waves per
+// workgroup, each with its own band of plane z.  A workgroup walks over
+// (plane, band group) items; a wave asks for the sticks of its next item
+// before the last products of the current one, when the registers of the
+// first products are free.
+template <typename T, int KS, int NW, int LB>
+__global__ void __launch_bounds__(64 * NW, LB)
+k_slab_mm(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restrict__ t2, const MmArgs<T> g_) {
+  typedef typename cx<T>::t C;
+  typedef typename MmV<T>::t V;
+  constexpr int TK = (KS + 3) / 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  C* kxt = reinterpret_cast<C*>(smem_raw);
+  C* hxt = kxt + 64 * KS * g_.TX;
+  C* kyt = g_.shared ? kxt : hxt + 64 * 4 * TK * g_.TX;
+  C* hyt = g_.shared ? hxt : kyt + 64 * KS * g_.TY;
+  int2* spt = reinterpret_cast<int2*>(hyt + 64 * 4 * TK * g_.TY);
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, c = lane & 15;
+  // consecutive items: the band groups of one plane.  XCD x takes one
+  // contiguous run of items (one L2 copy of a plane of V) and its blocks step
+  // through that run together.
+  const int ngrp = (g_.nb + NW - 1) / NW, items = g_.n3 * ngrp;
+  const int xcd = blockIdx.x & 7, step = (gridDim.x + 7 - xcd) >> 3;
+  const int q8 = items >> 3, r8 = items & 7;
+  const int last = (xcd + 1) * q8 + min(xcd + 1, r8);
+  int item = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
+  {
+    const int nk = 64 * KS * g_.TX, nh = 64 * 4 * TK * g_.TX;
+    for (int e = t; e < nk; e += 64 * NW) kxt[e] = g_.kx_t[e];
+    for (int e = t; e < nh; e += 64 * NW) hxt[e] = g_.hx_t[e];
+    if (!g_.shared) {
+      const int mk = 64 * KS * g_.TY, mh = 64 * 4 * TK * g_.TY;
+      for (int e = t; e < mk; e += 64 * NW) kyt[e] = g_.ky_t[e];
+      for (int e = t; e < mh; e += 64 * NW) hyt[e] = g_.hy_t[e];
+    }
+    for (int e = t; e < 64 * TK * KS; e += 64 * NW) spt[e] = g_.sp[e];
+  }
+  __syncthreads();
+
+  // the sticks +-ky of this lane, as loaded (absent ones: any stick)
+  C rp[TK][KS], rm[TK][KS];
+  auto fetch = [&](int it) {
+    const int z = it / ngrp, band = min((it - z * ngrp) * NW + w, g_.nb - 1);
+    const C* src = t1 + ((size_t)band * g_.n3 + z) * g_.nstick;
+#pragma unroll
+    for (int k = 0; k < TK; k++)
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const int2 e = spt[(k * KS + s) * 64 + lane];
+        rp[k][s] = src[e.x == kMmNone ? 0 : (e.x & ~kMmConj)];
+        rm[k][s] = src[e.y == kMmNone ? 0 : (e.y & ~kMmConj)];
+      }
+  };
+  if (item < last) fetch(item);
+
+  for (; item < last; item += step) {
+  const int z = item / ngrp, band = (item - z * ngrp) * NW + w;
+  // the plane's sticks into the four class matrices
+  T ee[TK][KS], oe[TK][KS], eo[TK][KS], oo[TK][KS];
+#pragma unroll
+  for (int k = 0; k < TK; k++) {
+    const int kx = 16 * k + mm_perm<T>(c);
+    const T wt = (kx == 0 || kx == g_.half) ? (T)1 : (T)2;
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      const int2 e = spt[(k * KS + s) * 64 + lane];
+      C p = rp[k][s], m = rm[k][s];
+      if (e.x & kMmConj) p.y = -p.y;
+      if (e.y & kMmConj) m.y = -m.y;
+      if (e.x == kMmNone) p = C{0, 0};
+      if (e.y == kMmNone) m = C{0, 0};
+      ee[k][s] = wt * (p.x + m.x);
+      oe[k][s] = -wt * (p.y + m.y);
+      eo[k][s] = -wt * (p.y - m.y);
+      oo[k][s] = -wt * (p.x - m.x);
+    }
+  }
+
+  const V zero = {0, 0, 0, 0};
+  V zee[TK][TK], zoe[TK][TK], zeo[TK][TK], zoo[TK][TK];  // [ky tile][kx tile]
+#pragma unroll
+  for (int a = 0; a < TK; a++)
+#pragma unroll
+    for (int b = 0; b < TK; b++) zee[a][b] = zoe[a][b] = zeo[a][b] = zoo[a][b] = zero;
+
+  auto ytile = [&](int yt, bool prefetch) {
+    V dee[TK], doe[TK], deo[TK], doo[TK];
+#pragma unroll
+    for (int k = 0; k < TK; k++) dee[k] = doe[k] = deo[k] = doo[k] = zero;
+    {
+      C q[KS];
+#pragma unroll
+      for (int s = 0; s < KS; s++) q[s] = kyt[(yt * KS + s) * 64 + lane];
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int k = 0; k < TK; k++) {
+          dee[k] = mm16(ee[k][s], q[s].x, dee[k]);
+          deo[k] = mm16(eo[k][s], q[s].y, deo[k]);
+          doe[k] = mm16(oe[k][s], q[s].x, doe[k]);
+          doo[k] = mm16(oo[k][s], q[s].y, doo[k]);
+        }
+    }
+    V fee[TK], foe[TK], feo[TK], foo[TK];  // D3
+#pragma unroll
+    for (int k = 0; k < TK; k++) fee[k] = foe[k] = feo[k] = foo[k] = zero;
+    const V* vp = g_.v + ((size_t)(z * g_.TY + yt) * g_.TX * 4) * 64 + lane;
+    // one x tile of NI k-steps in its second product.  Everything it reads is
+    // issued first (left alone, the compiler sinks the loads behind the
+    // products and waits for each)
+    auto tile = [&](int xt, auto ni) {
+      constexpr int NI = decltype(ni)::value;
+      V v[4];
+      C q[KS], h[TK][NI];
+#pragma unroll
+      for (int i = 0; i < NI; i++) v[i] = vp[(xt * 4 + i) * 64];
+#pragma unroll
+      for (int s = 0; s < KS; s++) q[s] = kxt[(xt * KS + s) * 64 + lane];
+      if constexpr (TK == 1) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) h[0][i] = hxt[(4 * xt + i) * 64 + lane];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      V ree = zero, roe = zero, reo = zero, roo = zero;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        ree = mm16(q[s].x, dee[s / 4][s % 4], ree);
+        roe = mm16(q[s].y, doe[s / 4][s % 4], roe);
+        reo = mm16(q[s].x, deo[s / 4][s % 4], reo);
+        roo = mm16(q[s].y, doo[s / 4][s % 4], roo);
+      }
+      if constexpr (TK > 1) {
+#pragma unroll
+        for (int k = 0; k < TK; k++)
+#pragma unroll
+          for (int i = 0; i < NI; i++) h[k][i] = hxt[(k * 4 * g_.TX + 4 * xt + i) * 64 + lane];
+      }
+#pragma unroll
+      for (int i = 0; i < NI; i++) {
+        const T e0 = ree[i], e1 = roe[i], e2 = reo[i], e3 = roo[i];
+        const T w0 = v[i][0], w1 = v[i][1], w2 = v[i][2], w3 = v[i][3];
+        ree[i] = w0 * e0 + w1 * e1 + w2 * e2 + w3 * e3;
+        roe[i] = w1 * e0 + w0 * e1 + w3 * e2 + w2 * e3;
+        reo[i] = w2 * e0 + w3 * e1 + w0 * e2 + w1 * e3;
+        roo[i] = w3 * e0 + w2 * e1 + w1 * e2 + w0 * e3;
+#pragma unroll
+        for (int k = 0; k < TK; k++) {
+          fee[k] = mm16(ree[i], h[k][i].x, fee[k]);
+          foe[k] = mm16(roe[i], h[k][i].y, foe[k]);
+          feo[k] = mm16(reo[i], h[k][i].x, feo[k]);
+          foo[k] = mm16(roo[i], h[k][i].y, foo[k]);
+        }
+      }
+    };
+    const int full = g_.XS >> 2;
+    for (int xt = 0; xt < full; xt++) tile(xt, std::integral_constant<int, 4>{});
+    switch (g_.XS & 3) {
+      case 1: tile(full, std::integral_constant<int, 1>{}); break;
+      case 2: tile(full, std::integral_constant<int, 2>{}); break;
+      case 3: tile(full, std::integral_constant<int, 3>{}); break;
+      default: break;
+    }
+    if (prefetch) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(min(item + step, last - 1));  // unconditional: a branch would keep the old values in registers
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int a = 0; a < TK; a++) {
+      C q[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) q[i] = hyt[(a * 4 * g_.TY + 4 * yt + i) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i == 0 || 4 * yt + i < g_.YS) {
+#pragma unroll
+          for (int k = 0; k < TK; k++) {
+            zee[a][k] = mm16(q[i].x, fee[k][i], zee[a][k]);
+            zeo[a][k] = mm16(q[i].y, feo[k][i], zeo[a][k]);
+            zoe[a][k] = mm16(q[i].x, foe[k][i], zoe[a][k]);
+            zoo[a][k] = mm16(q[i].y, foo[k][i], zoo[a][k]);
+          }
+        }
+    }
+  };
+  for (int yt = 0; yt + 1 < g_.TY; yt++) ytile(yt, false);
+  ytile(g_.TY - 1, true);
+  if (band >= g_.nb) continue;
+  // Z(kx, +-ky): Re = ee -+ oo, Im = -(oe +- eo)
+  C* dst = t2 + ((size_t)band * g_.n3 + z) * g_.nstick;
+#pragma unroll
+  for (int k = 0; k < TK; k++) {
+    int2 e[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) e[s] = spt[(k * KS + s) * 64 + lane];
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      const T a = zee[s / 4][k][s % 4], b = zoo[s / 4][k][s % 4], p = zoe[s / 4][k][s % 4], q = zeo[s / 4][k][s % 4];
+      if (e[s].x >= 0 && !(e[s].x & kMmConj)) dst[e[s].x] = C{a - b, -(p + q)};
+      if (e[s].y >= 0 && !(e[s].y & kMmConj)) dst[e[s].y] = C{a + b, q - p};
+    }
+  }
+  }
+}
+
+}  // namespace pw

@@ -1,0 +1,240 @@
+// Host side of the matrix-core slab transform (pw_slab_mm.h): tables, stick
+// entries and the potential in operand order per context, and the launch.
+#include "pw_slab_mm.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <vector>
+
+#include "pw_internal.h"
+
+namespace pw {
+
+struct SlabMm {
+  int KS = 0, TX = 0, TY = 0, XS = 0, YS = 0, half = -1, shared = 0;
+  struct Grid { int blocks = 0; } grid[2];  // resident workgroups, asked for once
+  size_t off_hx = 0, off_ky = 0, off_hy = 0;
+  void* buf = nullptr;                // tables and stick entries of both precisions
+  const void* tab[2];                 // [PW_F64], [PW_F32]: x and y tables
+  const int2* sp[2];
+  void* v[2] = {nullptr, nullptr};    // V / N in operand order (one allocation, at v[PW_F64])
+};
+
+// {cos, sin} of 2 pi m / n, m = 0 .. n - 1, the quadrant taken exactly
+static std::vector<double2> roots_of(int n) {
+  std::vector<double2> w(n);
+  for (long m = 0; m < n; m++) {
+    const long q = 4 * m / n, rem = 4 * m - q * n;
+    const long double a = (long double)rem / (long double)n * 1.57079632679489661923132169163975144L;
+    const double c = (double)cosl(a), s = (double)sinl(a);
+    w[m] = q == 0 ? double2{c, s} : q == 1 ? double2{-s, c} : q == 2 ? double2{-c, -s} : double2{s, -c};
+  }
+  return w;
+}
+
+// The two tables of one axis: kt [T][KS][64] = {cos, sin}(2 pi h k / n) at
+// k = 4 s + lane / 16, h = 16 tile + perm(lane % 16); ht [TK][4 T][64] at h =
+// 4 u + lane / 16, k = 16 tile + perm(lane % 16); zero beyond kmax and n / 2.
+template <typename T>
+static typename cx<T>::t* axis_tables(int n, int kmax, int KS, int tiles, typename cx<T>::t* out) {
+  const int TK = (KS + 3) / 4, H = n / 2 + 1;
+  const std::vector<double2> w = roots_of(n);
+  auto put = [&](int k, int h) {
+    const double2 e = k <= kmax && h < H ? w[(long)k * h % n] : double2{0, 0};
+    *out++ = typename cx<T>::t{(T)e.x, (T)e.y};
+  };
+  for (int a = 0; a < tiles; a++)
+    for (int s = 0; s < KS; s++)
+      for (int l = 0; l < 64; l++) put(4 * s + l / 16, 16 * a + mm_perm<T>(l % 16));
+  for (int a = 0; a < TK; a++)
+    for (int u = 0; u < 4 * tiles; u++)
+      for (int l = 0; l < 64; l++) put(16 * a + mm_perm<T>(l % 16), 4 * u + l / 16);
+  return out;
+}
+
+// V / N in operand order: [z][y tile][x tile][i][lane], the four classes
+// W = sum over the signs of (x, y) of V(+-x, +-y) times the class's signs at
+// (x, y) = (16 xt + 4 i + lane / 16, 16 yt + perm(lane % 16)); a point that is
+// its own mirror counts once.  Formed in FP64 in both precisions.
+template <typename T>
+__global__ void k_mm_potential(const double* __restrict__ vtot, typename MmV<T>::t* __restrict__ out, int n1, int n2,
+                               int TX, int TY, long total) {
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
+    const int lane = (int)(e & 63), i = (int)(e >> 6) & 3;
+    const long q = e >> 8;
+    const int xt = (int)(q % TX), yt = (int)(q / TX % TY);
+    const long z = q / TX / TY;
+    const int x = 16 * xt + 4 * i + lane / 16, y = 16 * yt + mm_perm<T>(lane % 16);
+    typename MmV<T>::t w = {0, 0, 0, 0};
+    if (x <= n1 / 2 && y <= n2 / 2) {
+      const double* p = vtot + z * n1 * n2;
+      const bool mx = x != 0 && 2 * x != n1, my = y != 0 && 2 * y != n2;
+      const double a = p[(long)y * n1 + x];
+      const double b = mx ? p[(long)y * n1 + n1 - x] : 0.0;
+      const double c = my ? p[(long)(n2 - y) * n1 + x] : 0.0;
+      const double d = mx && my ? p[(long)(n2 - y) * n1 + n1 - x] : 0.0;
+      w[0] = (T)((a + b) + (c + d));
+      w[1] = (T)((a - b) + (c - d));
+      w[2] = (T)((a + b) - (c + d));
+      w[3] = (T)((a - b) - (c - d));
+    }
+    out[e] = w;
+  }
+}
+
+void mm_free(pw_ctx* c) {
+  if (!c->mm) return;
+  if (c->mm->buf) (void)hipFree(c->mm->buf);
+  if (c->mm->v[PW_F64]) (void)hipFree(c->mm->v[PW_F64]);
+  delete c->mm;
+  c->mm = nullptr;
+}
+
+// one precision's tables and stick entries at host (and their device place)
+template <typename T>
+static void fill_plan(const pw_ctx* c, SlabMm* m, int kymax, const std::vector<int>& plus,
+                      const std::vector<int>& minus, unsigned char* host, size_t tab_bytes, const unsigned char* dev) {
+  typedef typename cx<T>::t C;
+  const int d = sizeof(T) == 8 ? PW_F64 : PW_F32, TK = (m->KS + 3) / 4, nk = 16 * TK;
+  C* end = axis_tables<T>(c->n1, c->sp.kxmax, m->KS, m->TX, (C*)host);
+  if (!m->shared) axis_tables<T>(c->n2, kymax, m->KS, m->TY, end);
+  int2* sp = (int2*)(host + tab_bytes);
+  for (int k = 0; k < TK; k++)
+    for (int s = 0; s < m->KS; s++)
+      for (int l = 0; l < 64; l++) {
+        const int kx = 16 * k + mm_perm<T>(l % 16), ky = 4 * s + l / 16;
+        *sp++ = int2{plus[ky * nk + kx], minus[ky * nk + kx]};
+      }
+  m->tab[d] = dev;
+  m->sp[d] = (const int2*)(dev + tab_bytes);
+}
+
+// The plan of a context, where the transform covers its sphere: at most 32
+// kx and 32 ky, and one stick of each conjugate pair of the kx = 0 column.
+int mm_plan(pw_ctx* c) {
+  const StickPlan& st = c->sp;
+  int kymax = 0;
+  for (int s = 0; s < st.nstick; s++) kymax = std::max(kymax, std::abs(kgrid(st.ky[s], c->n2)));
+  const int K = std::max(st.kxmax, kymax) + 1, KS = (K + 3) / 4;
+  if (KS > 8) return PW_OK;
+  SlabMm* m = new SlabMm();
+  m->KS = KS <= 2 ? 2 : (KS == 7 ? 8 : KS);
+  m->TX = (c->n1 / 2 + 16) / 16;
+  m->TY = (c->n2 / 2 + 16) / 16;
+  m->XS = (c->n1 / 2 + 4) / 4;
+  m->YS = (c->n2 / 2 + 4) / 4;
+  m->half = c->n1 % 2 == 0 ? c->n1 / 2 : -1;
+  m->shared = c->n1 == c->n2 && st.kxmax == kymax;
+  const int TK = (m->KS + 3) / 4, nk = 16 * TK;
+  std::vector<int> plus((size_t)nk * 4 * m->KS, kMmNone), minus(plus);
+  bool ok = true;
+  for (int s = 0; s < st.nstick; s++) {
+    const int ky = kgrid(st.ky[s], c->n2), at = std::abs(ky) * nk + st.kx[s];
+    (ky >= 0 ? plus : minus)[at] = s;
+  }
+  for (int s = 0; s < st.nstick; s++) {
+    const int ky = kgrid(st.ky[s], c->n2), at = std::abs(ky) * nk;
+    if (st.kx[s] != 0 || ky == 0 || 2 * ky == c->n2) continue;
+    int& other = (ky > 0 ? minus : plus)[at];
+    if (other != kMmNone && !(other & kMmConj)) ok = false;
+    else other = s | kMmConj;
+  }
+  m->off_hx = 64 * (size_t)m->KS * m->TX;
+  m->off_ky = m->shared ? 0 : m->off_hx + 64 * (size_t)4 * TK * m->TX;
+  m->off_hy = m->shared ? m->off_hx : m->off_ky + 64 * (size_t)m->KS * m->TY;
+  if (!ok) {
+    delete m;
+    return PW_OK;
+  }
+  c->mm = m;
+  const size_t entries = 64 * (size_t)(m->KS + 4 * TK) * (m->TX + (m->shared ? 0 : m->TY));
+  const size_t sp_bytes = sizeof(int2) * 64 * TK * m->KS, tab64 = sizeof(double2) * entries, tab32 = tab64 / 2;
+  std::vector<unsigned char> host(tab64 + tab32 + 2 * sp_bytes);
+  PW_HIP(hipMalloc(&m->buf, host.size()));
+  unsigned char* dev = (unsigned char*)m->buf;
+  fill_plan<double>(c, m, kymax, plus, minus, host.data(), tab64, dev);
+  const size_t second = tab64 + sp_bytes;
+  fill_plan<float>(c, m, kymax, plus, minus, host.data() + second, tab32, dev + second);
+  PW_HIP(hipMemcpy(m->buf, host.data(), host.size(), hipMemcpyHostToDevice));
+  const size_t vn = 4 * 64 * 4 * (size_t)m->TX * m->TY * c->n3;
+  PW_HIP(hipMalloc(&m->v[PW_F64], (sizeof(double) + sizeof(float)) * vn));
+  m->v[PW_F32] = (double*)m->v[PW_F64] + vn;
+  return PW_OK;
+}
+
+// After the potential has been set (on the context's stream, waited for).
+int mm_potential(pw_ctx* c) {
+  if (!c->mm) return PW_OK;
+  SlabMm* m = c->mm;
+  const long total = 256L * m->TX * m->TY * c->n3;
+  const int blocks = (int)std::min<long>((total + 255) / 256, 8192);
+  hipLaunchKernelGGL(k_mm_potential<double>, dim3(blocks), dim3(256), 0, c->stream, c->d_vtot,
+                     (MmV<double>::t*)m->v[PW_F64], c->n1, c->n2, m->TX, m->TY, total);
+  hipLaunchKernelGGL(k_mm_potential<float>, dim3(blocks), dim3(256), 0, c->stream, c->d_vtot,
+                     (MmV<float>::t*)m->v[PW_F32], c->n1, c->n2, m->TX, m->TY, total);
+  PW_HIP(hipGetLastError());
+  PW_HIP(hipStreamSynchronize(c->stream));
+  return PW_OK;
+}
+
+constexpr int kMmWaves = 4;
+
+// waves per SIMD of an instantiation: the registers of its accumulators
+template <typename T, int KS> constexpr int mm_lb() {
+  return sizeof(T) == 8 ? (KS <= 4 ? 2 : 1) : (KS <= 4 ? 4 : 2);
+}
+template <typename T>
+using mm_fn = decltype(&k_slab_mm<T, 4, kMmWaves, mm_lb<T, 4>()>);
+template <typename T>
+static mm_fn<T> mm_kernel(int KS) {
+  switch (KS) {
+    case 2: return &k_slab_mm<T, 2, kMmWaves, mm_lb<T, 2>()>;
+    case 3: return &k_slab_mm<T, 3, kMmWaves, mm_lb<T, 3>()>;
+    case 4: return &k_slab_mm<T, 4, kMmWaves, mm_lb<T, 4>()>;
+    case 5: return &k_slab_mm<T, 5, kMmWaves, mm_lb<T, 5>()>;
+    case 6: return &k_slab_mm<T, 6, kMmWaves, mm_lb<T, 6>()>;
+    case 8: return &k_slab_mm<T, 8, kMmWaves, mm_lb<T, 8>()>;
+    default: return nullptr;
+  }
+}
+
+template <typename T>
+bool mm_slab_ready(const pw_ctx* c) {
+  if (!c->mm) return false;
+  const SlabMm* m = c->mm;
+  return mm_lds<T>(m->KS, m->TX, m->TY, m->shared) <= 160 * 1024;
+}
+
+template <typename T>
+int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
+  typedef typename cx<T>::t C;
+  const SlabMm* m = c->mm;
+  const int d = sizeof(T) == 8 ? PW_F64 : PW_F32;
+  const C* tab = (const C*)m->tab[d];
+  MmArgs<T> a{tab, tab + m->off_hx, tab + m->off_ky, tab + m->off_hy, m->sp[d], (const typename MmV<T>::t*)m->v[d],
+              m->TX, m->TY, m->XS, m->YS, c->n3, c->sp.nstick, nb, m->half, m->shared};
+  const auto kern = mm_kernel<T>(m->KS);
+  const size_t lds = mm_lds<T>(m->KS, m->TX, m->TY, m->shared);
+  PW_TRY(ensure_lds((const void*)kern, lds));
+  // as many workgroups as the device holds at once, at most one per item
+  SlabMm::Grid& gr = c->mm->grid[d];
+  if (gr.blocks == 0) {
+    int per_cu = 0, ncu = 0;
+    PW_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kern, 64 * kMmWaves, lds));
+    PW_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+    gr.blocks = std::max(1, per_cu) * std::max(8, ncu);
+  }
+  const int items = c->n3 * ((nb + kMmWaves - 1) / kMmWaves);
+  // (8 at least: every XCD's run of items needs a workgroup)
+  hipLaunchKernelGGL(kern, dim3((unsigned)std::max(8, std::min(items, gr.blocks))), dim3(64 * kMmWaves), lds,
+                     c->stream, (const C*)t1, (C*)t2, a);
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+template bool mm_slab_ready<double>(const pw_ctx*);
+template bool mm_slab_ready<float>(const pw_ctx*);
+template int mm_slab<double>(pw_ctx*, int, const void*, void*);
+template int mm_slab<float>(pw_ctx*, int, const void*, void*);
+
+}  // namespace pw

@@ -1,10 +1,7 @@
 // The xy slab transform with every 1D FFT in one thread's registers, as
 // workgroup-level device code: slab_xy_reg_body (one z plane of SB bands;
 // the body of pw_hpsi.hip's k_slab_xy_reg, also run by the batched
-// persistent kernel) and slab_xy_reg_persistent (a workgroup loops over
-// (plane, band group) items and prefetches the next item's sticks and V
-// plane into registers while it transforms the current one), both built
-// from the phases of SlabReg.
+// persistent kernel), built from the phases of SlabReg.
 //
 // For compile-time N1 = N2: one z plane of SB bands per call (bands b0 ..).
 // V's plane is staged once in LDS as (row 2q, row 2q + 1) pairs, one 64-bit
@@ -32,8 +29,8 @@ struct SlabReg {
   static_assert(N1 % 2 == 0 && N2 % 2 == 0, "even N1 and N2");
   typedef typename cx<T>::t C;
   static constexpr int H1 = N1 / 2, NPAIR = N2 / 2, LV = N1 + 1, KC = 8;
-  static constexpr int KS = 16;                        // prefetched sticks per thread
-  static constexpr int VB = (N1 * N2 + NT - 1) / NT;   // prefetched V values per thread
+  static constexpr int KS = 16;                        // sticks per thread loaded up front
+  static constexpr int VB = (N1 * N2 + NT - 1) / NT;   // V values per thread
   C* Y;        // SB x nk x N2
   C* vp;       // NPAIR x LV pairs (v[2q][x], v[2q+1][x])
   T* vs;
@@ -256,34 +253,6 @@ __device__ __forceinline__ void slab_xy_reg_body(int z, int b0, const typename c
   sl.stage(z, b0, t1, r);
   sl.compute(min(SB, nb - b0));
   sl.gather(z, b0, t2);
-}
-
-// Items i = blockIdx.x, blockIdx.x + gridDim.x, ... < n3 ceil(nb / SB),
-// item i = (plane i % n3, bands SB (i / n3) ..): while the workgroup
-// transforms item i, the sticks and V plane of its next item are already in
-// flight into registers, and the stores of item i drain during the next
-// item's phases.
-template <typename T, int N1, int N2, int SB, int LY = 1, int NT = 256>
-__device__ __forceinline__ void slab_xy_reg_persistent(const typename cx<T>::t* t1, typename cx<T>::t* t2, int n3,
-                                                       int nstick, int kxmax, int nb, const int* __restrict__ pos,
-                                                       const int* __restrict__ mpos, const T* __restrict__ vtot,
-                                                       unsigned char* smem_raw) {
-  typedef SlabReg<T, N1, N2, SB, LY, NT> S;
-  const S sl(smem_raw, n3, nstick, kxmax, nb);
-  const int items = n3 * ((nb + SB - 1) / SB);
-  int i = blockIdx.x;
-  if (i >= items) return;  // uniform over the workgroup
-  typename S::Pre r;
-  sl.load(i % n3, (i / n3) * SB, t1, vtot, r);
-  sl.stage_pos(pos, mpos);
-  for (; i < items; i += gridDim.x) {
-    const int z = i % n3, b0 = (i / n3) * SB;
-    sl.stage(z, b0, t1, r);
-    const int in = i + gridDim.x;
-    if (in < items) sl.load(in % n3, (in / n3) * SB, t1, vtot, r);
-    sl.compute(min(SB, nb - b0));
-    sl.gather(z, b0, t2);
-  }
 }
 
 }  // namespace pw
