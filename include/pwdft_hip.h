@@ -95,9 +95,18 @@ int pw_ctx_info(const pw_ctx* ctx, int* npw, int* nstick, int* kxmax, long* ngri
 /* Local potential vtot_[:, spinswitch_] (src/SCF/hamiltonian.cpp:3333-3334),
  * host array of N doubles. */
 int pw_set_vtot(pw_ctx* ctx, const double* vtot);
+/* The same from a DEVICE array of N doubles, read on the context's stream
+ * (done with it on return). */
+int pw_set_vtot_device(pw_ctx* ctx, const double* vtot);
 
 /* vnlc_[0] = (beta, w) (src/SCF/hamiltonian.cpp:693-797), host arrays. */
 int pw_set_nonlocal(pw_ctx* ctx, int nbeta, const double* beta, const double* w);
+
+/* pw_gaussian_projectors for the context's sphere followed by
+ * pw_set_nonlocal, formed on the device (host arrays pos, wgt_channel): the
+ * projectors of atoms that move, natom (lmax + 1)^2 of them. */
+int pw_set_gaussian_projectors(pw_ctx* ctx, int natom, const double* pos, double sigma, int lmax,
+                               const double* wgt_channel);
 
 /* KohnSham::MultSpinor(Spinor&, NumTns<Complex>&, Fourier&)
  * (src/SCF/hamiltonian.cpp:3270-3452) with Spinor::AddMultSpinorFineR2C

@@ -56,6 +56,8 @@ def lib():
         "pw_ctx_set_stream": [_vp, _vp],
         "pw_ctx_info": [_vp, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_long)],
         "pw_set_vtot": [_vp, _dp],
+        "pw_set_vtot_device": [_vp, _vp],
+        "pw_set_gaussian_projectors": [_vp, C.c_int, _dp, C.c_double, C.c_int, _dp],
         "pw_set_nonlocal": [_vp, C.c_int, _dp, _dp],
         "pw_mult_spinor": [_vp, C.c_int, C.c_int, _vp, _vp],
         "pw_nonlocal_multx": [_vp, C.c_int, C.c_int, _vp, _vp],

@@ -25,7 +25,7 @@ import torch
 class BandEnergy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, vtot, pos, pwctx, psi, f):
-        pwctx.set_vtot(vtot.detach().cpu().numpy())
+        pwctx.set_vtot(vtot.detach())
         pos_np = np.array(pos.detach().cpu().numpy(), dtype=np.float64)
         pwctx.set_atoms(pos_np)
         E = pwctx.band_energy(psi, f)

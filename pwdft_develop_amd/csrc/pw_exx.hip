@@ -848,18 +848,19 @@ __global__ void k_scale(double* __restrict__ x, long n, double s) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) x[i] *= s;
 }
 
-// F[a][d] = -2 sum_i f_i sum_{p in a} w_p W[p,i] D_d[p,i]; one block per
-// (a, d), summed in FP64 whatever the precision of W and D
+// F[a][d] = -2 sum_i f_i sum_{p in a} w_p W[p,i] D_d[p,i] with W, D_x, D_y,
+// D_z the four column blocks of P ([4][nc] x nb) and atom a = a0 + blockIdx.x;
+// one block per (a, d), summed in FP64 whatever the precision of P
 template <typename T>
-__global__ void k_force_reduce(const T* __restrict__ W, const T* __restrict__ D, const double* __restrict__ w,
-                               const double* __restrict__ f, int nbeta, int nb, int npa, double* __restrict__ F) {
-  const int a = blockIdx.x, d = blockIdx.y;
-  const T* Dd = D + (size_t)d * nbeta * nb;
+__global__ void k_force_reduce(const T* __restrict__ P, const double* __restrict__ w, const double* __restrict__ f,
+                               int nc, int nb, int npa, int a0, double* __restrict__ F) {
+  const int a = a0 + blockIdx.x, d = blockIdx.y;
+  const size_t ld = 4 * (size_t)nc;
   double s = 0.0;
   for (int t = threadIdx.x; t < npa * nb; t += blockDim.x) {
     const int q = t % npa, i = t / npa;
-    const int p = a * npa + q;
-    s += f[i] * w[p] * (double)W[p + (size_t)nbeta * i] * (double)Dd[p + (size_t)nbeta * i];
+    const size_t at = blockIdx.x * npa + q + ld * i;
+    s += f[i] * w[a * npa + q] * (double)P[at] * (double)P[at + (size_t)(d + 1) * nc];
   }
   __shared__ double red[256];
   red[threadIdx.x] = s;
@@ -1130,50 +1131,72 @@ extern "C" int pw_add_exx(pw_ctx* c, int dtype, int nb, const void* psi, void* a
 
 namespace pw {
 
+// The context's scratch of the energy, density and force calls: at least
+// `bytes`, kept for the next call (an allocation and a free, which waits for
+// the device, cost more than the kernels here on small cells).
+static int adjoint_ws(pw_ctx* c, size_t bytes) {
+  if (bytes <= c->adj_ws_bytes) return PW_OK;
+  if (c->d_adj_ws) (void)hipFree(c->d_adj_ws);
+  c->d_adj_ws = nullptr;
+  c->adj_ws_bytes = 0;
+  if (hipMalloc(&c->d_adj_ws, bytes) != hipSuccess)
+    return fail(PW_ERR_NOMEM, "cannot allocate %zu bytes of scratch", bytes);
+  c->adj_ws_bytes = bytes;
+  return PW_OK;
+}
+static size_t pad256(size_t b) { return (b + 255) / 256 * 256; }
+
+// On matrix cores where the sphere has that plan (k_density_mm), else through
+// the LDS transforms (48^3, 128 bands, FP64: 135 us against 35 us).
 template <typename T>
 static int density_impl(pw_ctx* c, int nb, const void* psi, const double* f, double* rho, int accumulate) {
   typedef typename cx<T>::t C;
   const long N = c->N;
-  const int nsplit = 16;
-  double *df = nullptr, *part = nullptr;
-  auto done = [&](int rc) {
-    if (df) (void)hipFree(df);
-    if (part) (void)hipFree(part);
-    return rc;
-  };
-  if (hipMalloc((void**)&df, sizeof(double) * nb) != hipSuccess ||
-      hipMalloc((void**)&part, sizeof(double) * N * nsplit) != hipSuccess)
-    return done(fail(PW_ERR_NOMEM, "pw_density: scratch allocation failed"));
-  if (hipMemcpy(df, f, sizeof(double) * nb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemsetAsync(part, 0, sizeof(double) * N * nsplit, c->stream) != hipSuccess)
-    return done(fail(PW_ERR_HIP, "pw_density: copy failed"));
-  int rc = sphere_to_sticks<T>(c, nb, psi, c->d_t1);
-  if (rc) return done(rc);
-  const C* tw = (const C*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32);
-  SlabGeom g{c->n1, c->n2, c->n3, c->sp.nstick, c->sp.kxmax, 0, 0};
-  const int thr = pick_wfn_layout(c, sizeof(C), g);
-  const size_t lds = slab_bytes(c, sizeof(C), g.kxmax, g.rp, g.cg);
-  if ((rc = set_lds(k_density_acc<T>, lds)) != PW_OK) return done(rc);
-  hipLaunchKernelGGL(k_density_acc<T>, dim3(c->n3, nsplit), dim3(thr), lds, c->stream, (const C*)c->d_t1,
-                     (const double*)df, 0, nb, nsplit, part, c->d_pos, c->d_mpos, g, 1.0 / (double)N, tw,
-                     tw + c->n1);
+  const int mm = mm_density_splits(c, nb), nsplit = mm > 0 ? mm : 16;
+  const size_t fb = pad256(sizeof(double) * nb);
+  PW_TRY(adjoint_ws(c, fb + sizeof(double) * N * nsplit));
+  double* df = (double*)c->d_adj_ws;
+  double* part = (double*)((unsigned char*)c->d_adj_ws + fb);
+  PW_HIP(hipMemcpyAsync(df, f, sizeof(double) * nb, hipMemcpyHostToDevice, c->stream));
+  PW_TRY(sphere_to_sticks<T>(c, nb, psi, c->d_t1));
+  if (mm > 0) {
+    PW_TRY(mm_density<T>(c, nb, c->d_t1, df, nsplit, part));
+  } else {
+    hipLaunchKernelGGL(k_fill_zero<double>, dim3(grid_of(N * nsplit)), dim3(256), 0, c->stream, part, N * nsplit);
+    const C* tw = (const C*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32);
+    SlabGeom g{c->n1, c->n2, c->n3, c->sp.nstick, c->sp.kxmax, 0, 0};
+    const int thr = pick_wfn_layout(c, sizeof(C), g);
+    const size_t lds = slab_bytes(c, sizeof(C), g.kxmax, g.rp, g.cg);
+    PW_TRY(set_lds(k_density_acc<T>, lds));
+    hipLaunchKernelGGL(k_density_acc<T>, dim3(c->n3, nsplit), dim3(thr), lds, c->stream, (const C*)c->d_t1,
+                       (const double*)df, 0, nb, nsplit, part, c->d_pos, c->d_mpos, g, 1.0 / (double)N, tw,
+                       tw + c->n1);
+  }
   hipLaunchKernelGGL(k_sum_partials, dim3((int)std::min<long>((N + 255) / 256, 4096)), dim3(256), 0, c->stream,
                      (const double*)part, nsplit, N, rho, accumulate);
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
-    return done(fail(PW_ERR_HIP, "pw_density: kernel failed"));
-  return done(PW_OK);
+  PW_HIP(hipGetLastError());
+  PW_HIP(hipStreamSynchronize(c->stream));
+  return PW_OK;
 }
 
+// beta of nc columns from p0 beside -i G_d beta, d = x, y, z: [4][nc] columns
+struct GVectors {
+  double recip[9];
+  int n1, n2, n3, h1, npw;
+};
 template <typename C>
-__global__ void k_make_dbeta(const C* __restrict__ beta, const double* __restrict__ G, int npw, int nbeta,
+__global__ void k_make_dbeta(const C* __restrict__ beta, const int* __restrict__ idx, GVectors v, int nc,
                              C* __restrict__ out) {
-  const long total = (long)npw * nbeta;
+  const long total = (long)v.npw * nc;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
-    const int i = (int)(e % npw);
+    const int g = idx[e % v.npw], kx = g % v.h1, ky = g / v.h1 % v.n2, kz = g / (v.h1 * v.n2);
+    const int m0 = kx <= v.n1 / 2 ? kx : kx - v.n1, m1 = ky <= v.n2 / 2 ? ky : ky - v.n2,
+              m2 = kz <= v.n3 / 2 ? kz : kz - v.n3;
     const C b = beta[e];
+    out[e] = b;
     for (int d = 0; d < 3; d++) {
-      const double gd = G[3 * i + d];
-      out[(size_t)d * total + e] = C{(decltype(b.x))(gd * b.y), (decltype(b.x))(-gd * b.x)};  // -i G_d beta
+      const double gd = v.recip[d] * m0 + v.recip[3 + d] * m1 + v.recip[6 + d] * m2;
+      out[(size_t)(d + 1) * total + e] = C{(decltype(b.x))(gd * b.y), (decltype(b.x))(-gd * b.x)};
     }
   }
 }
@@ -1235,24 +1258,15 @@ namespace pw {
 template <typename T>
 static int band_energy_impl(pw_ctx* c, int dtype, int nb, const void* X, const double* f, double* E) {
   const long m = 2L * c->npw;
-  T* HX = nullptr;
-  double* dots = nullptr;
-  if (hipMalloc((void**)&HX, sizeof(T) * m * nb) != hipSuccess ||
-      hipMalloc((void**)&dots, sizeof(double) * nb) != hipSuccess) {
-    if (HX) (void)hipFree(HX);
-    return fail(PW_ERR_NOMEM, "pw_band_energy: scratch allocation failed");
-  }
-  int rc = pw_apply_h(c, dtype, nb, X, HX);
+  const size_t db = pad256(sizeof(double) * nb);
+  PW_TRY(adjoint_ws(c, db + sizeof(T) * m * nb));
+  double* dots = (double*)c->d_adj_ws;
+  T* HX = (T*)((unsigned char*)c->d_adj_ws + db);
+  PW_TRY(pw_apply_h(c, dtype, nb, X, HX));
   std::vector<double> h(nb);
-  if (rc == PW_OK) {
-    hipLaunchKernelGGL(k_band_dots<T>, dim3(nb), dim3(256), 0, c->stream, (const T*)X, (const T*)HX, m, dots);
-    if (hipMemcpyAsync(h.data(), dots, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-        hipStreamSynchronize(c->stream) != hipSuccess)
-      rc = fail(PW_ERR_HIP, "pw_band_energy: reduction failed");
-  }
-  (void)hipFree(HX);
-  (void)hipFree(dots);
-  if (rc != PW_OK) return rc;
+  hipLaunchKernelGGL(k_band_dots<T>, dim3(nb), dim3(256), 0, c->stream, (const T*)X, (const T*)HX, m, dots);
+  PW_HIP(hipMemcpyAsync(h.data(), dots, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
+  PW_HIP(hipStreamSynchronize(c->stream));
   double e = 0.0;
   for (int i = 0; i < nb; i++) e += f[i] * h[i];
   *E = e;
@@ -1260,57 +1274,43 @@ static int band_energy_impl(pw_ctx* c, int dtype, int nb, const void* X, const d
 }
 
 // Nonlocal force in the precision of the block (T): the projections
-// W = Re(beta^H X) and D_d = Re((-i G_d beta)^H X) are T GEMMs on MFMA, the
-// force sums are FP64.
+// W = Re(beta^H X) and D_d = Re((-i G_d beta)^H X) are one T product on MFMA
+// over the four column blocks (one split-K launch of 4 nc columns where four
+// of nc left most of the chip idle: 48^3, 64 projectors, 128 bands 94 -> 25
+// us), the force sums are FP64.  Atoms go through in groups that keep the four
+// blocks within 256 MiB.
 template <typename T>
 static int nonlocal_force_impl(pw_ctx* c, int nb, const void* X, const double* f, int natom, int npa,
                                double* force) {
   typedef typename cx<T>::t Cx;
-  const int npw = c->npw, nbeta = c->nbeta, m = 2 * npw;
+  const int npw = c->npw, m = 2 * npw;
   const T* beta = sizeof(T) == 8 ? (const T*)(const void*)c->d_beta : (const T*)(const void*)c->d_beta_f;
   if (!beta) return fail(PW_ERR_STATE, "pw_nonlocal_force: no projectors set");
-  // G vectors of the sphere
-  std::vector<double> G(3 * (size_t)npw);
-  for (int i = 0; i < npw; i++) {
-    const int g = c->h_idx[i];
-    const int kx = g % c->h1, ky = (g / c->h1) % c->n2, kz = g / (c->h1 * c->n2);
-    const int m0 = kgrid(kx, c->n1), m1 = kgrid(ky, c->n2), m2 = kgrid(kz, c->n3);
-    for (int d = 0; d < 3; d++) G[3 * i + d] = c->recip[d] * m0 + c->recip[3 + d] * m1 + c->recip[6 + d] * m2;
+  const size_t per_atom = sizeof(T) * 4 * (size_t)m * npa;
+  const int na = (int)std::max<size_t>(1, std::min<size_t>(natom, ((size_t)256 << 20) / per_atom)), nc = na * npa;
+  const size_t fb = pad256(sizeof(double) * nb), Fb = pad256(sizeof(double) * 3 * natom),
+               Pb = pad256(sizeof(T) * 4 * (size_t)nc * nb);
+  PW_TRY(adjoint_ws(c, fb + Fb + Pb + per_atom * na));
+  unsigned char* ws = (unsigned char*)c->d_adj_ws;
+  double *dfv = (double*)ws, *dF = (double*)(ws + fb);
+  T *dP = (T*)(ws + fb + Fb), *dB = (T*)(ws + fb + Fb + Pb);
+  PW_HIP(hipMemcpyAsync(dfv, f, sizeof(double) * nb, hipMemcpyHostToDevice, c->stream));
+  GVectors v;
+  for (int i = 0; i < 9; i++) v.recip[i] = c->recip[i];
+  v.n1 = c->n1; v.n2 = c->n2; v.n3 = c->n3; v.h1 = c->h1; v.npw = npw;
+  for (int a0 = 0; a0 < natom; a0 += na) {
+    const int nat = std::min(na, natom - a0), cols = nat * npa;
+    const long total = (long)npw * cols;
+    hipLaunchKernelGGL(k_make_dbeta<Cx>, dim3(grid_of(total)), dim3(256), 0, c->stream,
+                       (const Cx*)beta + (size_t)npw * a0 * npa, (const int*)c->d_idx, v, cols, (Cx*)dB);
+    PW_TRY(gemm_tn<T>(c, m, 4 * cols, nb, dB, m, (const T*)X, m, dP, 4 * cols, nullptr, (T)0));
+    hipLaunchKernelGGL(k_force_reduce<T>, dim3(nat, 3), dim3(256), 0, c->stream, (const T*)dP,
+                       (const double*)c->d_wgt, (const double*)dfv, cols, nb, npa, a0, dF);
   }
-  double *dG = nullptr, *dw = nullptr, *dfv = nullptr, *dF = nullptr;
-  T *dB = nullptr, *dW = nullptr, *dD = nullptr;
-  auto done = [&](int rc) {
-    void* p[] = {dG, dB, dW, dD, dw, dfv, dF};
-    for (void* q : p)
-      if (q) (void)hipFree(q);
-    return rc;
-  };
-  const size_t blk = (size_t)m * nbeta;
-  if (hipMalloc((void**)&dG, sizeof(double) * 3 * npw) != hipSuccess ||
-      hipMalloc((void**)&dB, sizeof(T) * 3 * blk) != hipSuccess ||
-      hipMalloc((void**)&dW, sizeof(T) * (size_t)nbeta * nb) != hipSuccess ||
-      hipMalloc((void**)&dD, sizeof(T) * 3 * (size_t)nbeta * nb) != hipSuccess ||
-      hipMalloc((void**)&dw, sizeof(double) * nbeta) != hipSuccess ||
-      hipMalloc((void**)&dfv, sizeof(double) * nb) != hipSuccess ||
-      hipMalloc((void**)&dF, sizeof(double) * 3 * natom) != hipSuccess)
-    return done(fail(PW_ERR_NOMEM, "pw_nonlocal_force: scratch allocation failed"));
-  if (hipMemcpy(dG, G.data(), sizeof(double) * 3 * npw, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(dw, c->h_wgt.data(), sizeof(double) * nbeta, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(dfv, f, sizeof(double) * nb, hipMemcpyHostToDevice) != hipSuccess)
-    return done(fail(PW_ERR_HIP, "pw_nonlocal_force: upload failed"));
-  hipLaunchKernelGGL(k_make_dbeta<Cx>, dim3(4096), dim3(256), 0, c->stream, (const Cx*)beta, (const double*)dG, npw,
-                     nbeta, (Cx*)dB);
-  int rc = gemm_tn<T>(c, m, nbeta, nb, beta, m, (const T*)X, m, dW, nbeta, nullptr, (T)0);
-  for (int d = 0; d < 3 && rc == PW_OK; d++)
-    rc = gemm_tn<T>(c, m, nbeta, nb, dB + d * blk, m, (const T*)X, m, dD + (size_t)d * nbeta * nb, nbeta, nullptr,
-                    (T)0);
-  if (rc != PW_OK) return done(rc);
-  hipLaunchKernelGGL(k_force_reduce<T>, dim3(natom, 3), dim3(256), 0, c->stream, (const T*)dW, (const T*)dD,
-                     (const double*)dw, (const double*)dfv, nbeta, nb, npa, dF);
-  if (hipMemcpyAsync(force, dF, sizeof(double) * 3 * natom, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-      hipStreamSynchronize(c->stream) != hipSuccess)
-    return done(fail(PW_ERR_HIP, "pw_nonlocal_force: reduction failed"));
-  return done(PW_OK);
+  PW_HIP(hipGetLastError());
+  PW_HIP(hipMemcpyAsync(force, dF, sizeof(double) * 3 * natom, hipMemcpyDeviceToHost, c->stream));
+  PW_HIP(hipStreamSynchronize(c->stream));
+  return PW_OK;
 }
 }  // namespace pw
 

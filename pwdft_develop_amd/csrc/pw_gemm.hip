@@ -1057,14 +1057,16 @@ int gemm_nn_ep(pw_ctx* c, int m, int n, int k, const T* A, int lda, const T* B, 
 
 // A (m x k, column-major, ld lda) split ahead of time into *out (the tile
 // layout of k_gemm_nn_pre; allocated here, freed by the caller).
-int split_a_operand(pw_ctx* c, const float* A, int lda, int m, int k, unsigned short** out) {
-  *out = nullptr;
+size_t split_a_bytes(int m, int k) {
+  return sizeof(unsigned short) * (size_t)((m + 15) / 16) * ((k + 31) / 32) * kSplitTerms * 512;
+}
+
+int split_a_operand(pw_ctx* c, const float* A, int lda, int m, int k, unsigned short* out) {
   if (m <= 0 || k <= 0) return PW_OK;
   const int nrt = (m + 15) / 16, nkc = (k + 31) / 32;
   const long ng = (long)nrt * nkc;
-  PW_HIP(hipMalloc((void**)out, sizeof(unsigned short) * (size_t)ng * kSplitTerms * 512));
   hipLaunchKernelGGL(k_split_operand<false>, dim3((unsigned)((ng + 3) / 4)), dim3(256), 0, c->stream, A, lda, m, k,
-                     nkc, *out, ng);
+                     nkc, out, ng);
   PW_HIP(hipGetLastError());
   return PW_OK;
 }

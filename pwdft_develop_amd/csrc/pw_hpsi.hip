@@ -594,13 +594,6 @@ static void build_stick_plan(pw_ctx* c, const int* idx) {
   }
 }
 
-template <typename X>
-static int upload(X** d, const X* h, size_t n) {
-  PW_HIP(hipMalloc((void**)d, sizeof(X) * (n > 0 ? n : 1)));
-  if (n) PW_HIP(hipMemcpy(*d, h, sizeof(X) * n, hipMemcpyHostToDevice));
-  return PW_OK;
-}
-
 static void roots(int n, std::vector<double>& out) {
   for (int m = 0; m < n; m++) {
     long double a = 2.0L * 3.14159265358979323846264338327950288L * (long double)m / (long double)n;
@@ -717,6 +710,7 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
     add(&c->d_gpt_sz, c->sp.gpt_sz.data(), c->sp.gpt_sz.size());
     add(&c->d_gchunk_off, c->sp.gchunk_off.data(), c->sp.gchunk_off.size());
     add(&c->d_zs, c->sp.zs.data(), c->sp.zs.size());
+    add(&c->d_idx, idx, (size_t)npw);
     add(&c->d_pos, c->sp.pos.data(), c->sp.pos.size());
     add(&c->d_mpos, c->sp.mpos.data(), c->sp.mpos.size());
     add(&c->d_ekin, ekin, (size_t)npw);
@@ -763,7 +757,7 @@ extern "C" int pw_ctx_destroy(pw_ctx* c) {
   mm_free(c);
   if (c->d_gemm_ws) (void)hipFree(c->d_gemm_ws);
   void* ptrs[] = {c->d_tables, c->d_vtot, c->d_vtot_f, c->d_beta, c->d_betaw, c->d_W, c->d_beta_f,
-                  c->d_betaw_f, c->d_W_f, c->d_t1, c->d_t2, c->d_betaw_bf, c->d_W_bf};
+                  c->d_betaw_f, c->d_W_f, c->d_t1, c->d_t2, c->d_betaw_bf, c->d_W_bf, c->d_wgt, c->d_adj_ws};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->blas) rocblas_destroy_handle(c->blas);
@@ -788,55 +782,6 @@ extern "C" int pw_ctx_info(const pw_ctx* c, int* npw, int* nstick, int* kxmax, l
   if (nstick) *nstick = c->sp.nstick;
   if (kxmax) *kxmax = c->sp.kxmax;
   if (ngrid) *ngrid = c->N;
-  return PW_OK;
-}
-
-extern "C" int pw_set_vtot(pw_ctx* c, const double* vtot) {
-  if (!c || !vtot) return fail(PW_ERR_ARG, "pw_set_vtot: null argument");
-  std::vector<double> v(vtot, vtot + c->N);
-  const double inv = 1.0 / (double)c->N;
-  for (auto& x : v) x *= inv;  // fold the C2R normalisation of spinor.cpp:620-621
-  std::vector<float> vf(v.begin(), v.end());
-  if (!c->d_vtot) {
-    invalidate_graph(c);
-    PW_HIP(hipMalloc((void**)&c->d_vtot, sizeof(double) * c->N));
-    PW_HIP(hipMalloc((void**)&c->d_vtot_f, sizeof(float) * c->N));
-  }
-  PW_HIP(hipMemcpy(c->d_vtot, v.data(), sizeof(double) * c->N, hipMemcpyHostToDevice));
-  PW_HIP(hipMemcpy(c->d_vtot_f, vf.data(), sizeof(float) * c->N, hipMemcpyHostToDevice));
-  PW_TRY(mm_potential(c));
-  c->have_vtot = true;
-  return PW_OK;
-}
-
-extern "C" int pw_set_nonlocal(pw_ctx* c, int nbeta, const double* beta, const double* w) {
-  if (!c || nbeta < 0 || (nbeta > 0 && (!beta || !w))) return fail(PW_ERR_ARG, "pw_set_nonlocal: bad argument");
-  invalidate_graph(c);
-  void* ptrs[] = {c->d_beta, c->d_betaw, c->d_W, c->d_beta_f, c->d_betaw_f, c->d_W_f, c->d_betaw_bf, c->d_W_bf};
-  for (void* p : ptrs)
-    if (p) (void)hipFree(p);
-  c->d_beta = c->d_betaw = c->d_W = nullptr;
-  c->d_beta_f = c->d_betaw_f = c->d_W_f = nullptr;
-  c->d_betaw_bf = c->d_W_bf = nullptr;
-  c->nbeta = nbeta;
-  c->h_wgt.assign(w ? w : (const double*)nullptr, w ? w + nbeta : (const double*)nullptr);
-  if (nbeta == 0) return PW_OK;
-  const size_t m = 2 * (size_t)c->npw;
-  std::vector<double> bw(beta, beta + m * nbeta);
-  for (int p = 0; p < nbeta; p++)
-    for (size_t r = 0; r < m; r++) bw[m * p + r] *= w[p];
-  std::vector<float> bf(beta, beta + m * nbeta), bwf(bw.begin(), bw.end());
-  int rc;
-  if ((rc = upload(&c->d_beta, beta, m * nbeta)) != PW_OK) return rc;
-  if ((rc = upload(&c->d_betaw, bw.data(), m * nbeta)) != PW_OK) return rc;
-  if ((rc = upload(&c->d_beta_f, bf.data(), m * nbeta)) != PW_OK) return rc;
-  if ((rc = upload(&c->d_betaw_f, bwf.data(), m * nbeta)) != PW_OK) return rc;
-  PW_HIP(hipMalloc((void**)&c->d_W, sizeof(double) * (size_t)nbeta * c->max_bands));
-  PW_HIP(hipMalloc((void**)&c->d_W_f, sizeof(float) * (size_t)nbeta * c->max_bands));
-  // the FP32 filter's projector apply on split BF16 products: betaw split once
-  PW_TRY(split_a_operand(c, c->d_betaw_f, (int)m, (int)m, nbeta, &c->d_betaw_bf));
-  PW_HIP(hipMalloc((void**)&c->d_W_bf, split_b_bytes(c->max_bands, nbeta)));
-  PW_HIP(hipStreamSynchronize(c->stream));
   return PW_OK;
 }
 

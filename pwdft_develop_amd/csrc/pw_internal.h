@@ -169,11 +169,12 @@ template <typename T>
 int gemm_nn_ep(pw_ctx* c, int m, int n, int k, const T* A, int lda, const T* B, int ldb, const T* H, const T* Yc,
                const T* Yp, T* out, int ld, const T* coef, int step, bool cheb, int split = 0);
 // The FP32 projector apply on products split ahead of time (pw_gemm.hip):
-// split_a_operand allocates *out and splits A (m x k) into BF16 terms in the
-// operand-tile layout; gemm_nn_pre splits B (k x n) into Bws
+// split_a_operand splits A (m x k) into BF16 terms in the
+// operand-tile layout (split_a_bytes(m, k) bytes at out); gemm_nn_pre splits B (k x n) into Bws
 // (split_b_bytes(n, k) bytes) and forms out = epilogue(A B) like gemm_nn_ep
 // with split (2 or 3) terms.
-int split_a_operand(pw_ctx* c, const float* A, int lda, int m, int k, unsigned short** out);
+size_t split_a_bytes(int m, int k);
+int split_a_operand(pw_ctx* c, const float* A, int lda, int m, int k, unsigned short* out);
 size_t split_b_bytes(int n, int k);
 int gemm_nn_pre(pw_ctx* c, int m, int n, int k, const unsigned short* Ab, const float* B, int ldb,
                 unsigned short* Bws, const float* H, const float* Yc, const float* Yp, float* out, int ld,
@@ -235,6 +236,11 @@ template <typename T>
 bool mm_slab_ready(const pw_ctx* c);
 template <typename T>
 int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2);
+// part[split] (N doubles each) = sum over the split's bands of f r^2 / N from
+// the sticks t1; splits: how many, 0 where the context has no plan.
+int mm_density_splits(const pw_ctx* c, int nb);
+template <typename T>
+int mm_density(pw_ctx* c, int nb, const void* t1, const double* f, int nsplit, double* part);
 // Exact exchange (pw_exx.hip): a3 += V_x psi when the context holds an
 // exchange operator; state freed with the context.
 struct ExxState;
@@ -266,13 +272,13 @@ struct pw_ctx {
   int npw, npad, max_bands;
   pw::StickPlan sp;
   std::vector<int> h_idx;       // idxCoarseCut, host copy
-  std::vector<double> h_wgt;    // projector weights, host copy
   std::vector<int> f1, f2, f3;  // radix plans
   // device arrays (d_pt_idx ... d_tw32 lie in d_tables)
   void* d_tables = nullptr;
   int *d_pt_idx = nullptr, *d_pt_sz = nullptr, *d_chunk_off = nullptr;
   int *d_gpt_idx = nullptr, *d_gpt_sz = nullptr, *d_gchunk_off = nullptr;
   int* d_zs = nullptr;  // StickPlan::zs
+  int* d_idx = nullptr; // idxCoarseCut
   int *d_pos = nullptr, *d_mpos = nullptr;
   double *d_ekin = nullptr, *d_teter = nullptr;
   float *d_ekin_f = nullptr, *d_teter_f = nullptr;
@@ -284,6 +290,11 @@ struct pw_ctx {
   int nbeta = 0;
   double *d_beta = nullptr, *d_betaw = nullptr, *d_W = nullptr;
   float *d_beta_f = nullptr, *d_betaw_f = nullptr, *d_W_f = nullptr;
+  double* d_wgt = nullptr;  // projector weights
+  // scratch of the energy, density and force entry points, grown on demand
+  // (adjoint_ws), freed by pw_free_workspace
+  void* d_adj_ws = nullptr;
+  size_t adj_ws_bytes = 0;
   // betaw (FP32) split into BF16 terms ahead of time, and the per-call split
   // of W (max_bands columns), for the projector apply on split products
   unsigned short *d_betaw_bf = nullptr, *d_W_bf = nullptr;

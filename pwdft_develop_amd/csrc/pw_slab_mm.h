@@ -288,4 +288,90 @@ k_slab_mm(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restric
   }
 }
 
+// Density of nb bands on one 16 x 16 tile of the quarter plane: products 1 and
+// 2 of k_slab_mm per band, then acc += f r(+-x, +-y)^2 in FP64 registers.  A
+// wave takes (plane, tile, every nsplit-th band) and writes its tile once to
+// part[split] (N doubles each), so the sums over splits are in a fixed order.
+// The first product is repeated for each x tile (16 products beside the 16 of
+// the second): with the tile fixed the sums stay in 32 registers at any size.
+template <typename T, int KS, int NW>
+__global__ void __launch_bounds__(64 * NW, sizeof(T) == 8 && KS > 4 ? 1 : 2)
+k_density_mm(const typename cx<T>::t* __restrict__ t1, const MmArgs<T> g_, const double* __restrict__ f, double invN,
+             int nsplit, int n1, int n2, double* __restrict__ part) {
+  typedef typename cx<T>::t C;
+  typedef typename MmV<T>::t V;
+  constexpr int TK = (KS + 3) / 4;
+  const int lane = threadIdx.x & 63, c = lane & 15, gq = lane >> 4;
+  const int per_z = g_.TX * g_.TY * nsplit;
+  const int unit = blockIdx.x * NW + (threadIdx.x >> 6);
+  if (unit >= per_z * g_.n3) return;
+  const int z = unit / per_z, r = unit - z * per_z, split = r / (g_.TX * g_.TY);
+  const int xt = r % g_.TX, yt = r / g_.TX % g_.TY;
+  C ky[KS], kx[KS];
+#pragma unroll
+  for (int s = 0; s < KS; s++) {
+    ky[s] = g_.ky_t[(yt * KS + s) * 64 + lane];
+    kx[s] = g_.kx_t[(xt * KS + s) * 64 + lane];
+  }
+  double acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int s = 0; s < 4; s++) acc[i][s] = 0.0;
+  const V zero = {0, 0, 0, 0};
+  for (int band = split; band < g_.nb; band += nsplit) {
+    const C* src = t1 + ((size_t)band * g_.n3 + z) * g_.nstick;
+    const double fb = f[band] * invN;
+    V dee[TK], doe[TK], deo[TK], doo[TK];
+#pragma unroll
+    for (int k = 0; k < TK; k++) {
+      dee[k] = doe[k] = deo[k] = doo[k] = zero;
+      const int kxi = 16 * k + mm_perm<T>(c);
+      const T wt = (kxi == 0 || kxi == g_.half) ? (T)1 : (T)2;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const int2 e = g_.sp[(k * KS + s) * 64 + lane];
+        C p = src[e.x == kMmNone ? 0 : (e.x & ~kMmConj)], m = src[e.y == kMmNone ? 0 : (e.y & ~kMmConj)];
+        if (e.x & kMmConj) p.y = -p.y;
+        if (e.y & kMmConj) m.y = -m.y;
+        if (e.x == kMmNone) p = C{0, 0};
+        if (e.y == kMmNone) m = C{0, 0};
+        dee[k] = mm16(wt * (p.x + m.x), ky[s].x, dee[k]);
+        doe[k] = mm16(-wt * (p.y + m.y), ky[s].x, doe[k]);
+        deo[k] = mm16(-wt * (p.y - m.y), ky[s].y, deo[k]);
+        doo[k] = mm16(-wt * (p.x - m.x), ky[s].y, doo[k]);
+      }
+    }
+    V ree = zero, roe = zero, reo = zero, roo = zero;
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      ree = mm16(kx[s].x, dee[s / 4][s % 4], ree);
+      roe = mm16(kx[s].y, doe[s / 4][s % 4], roe);
+      reo = mm16(kx[s].x, deo[s / 4][s % 4], reo);
+      roo = mm16(kx[s].y, doo[s / 4][s % 4], roo);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const T ep = ree[i] + reo[i], em = ree[i] - reo[i], op = roe[i] + roo[i], om = roe[i] - roo[i];
+      const double r0 = ep + op, r1 = ep - op, r2 = em + om, r3 = em - om;
+      acc[i][0] += r0 * r0 * fb;
+      acc[i][1] += r1 * r1 * fb;
+      acc[i][2] += r2 * r2 * fb;
+      acc[i][3] += r3 * r3 * fb;
+    }
+  }
+  double* o = part + ((size_t)split * g_.n3 + z) * n1 * n2;
+  const int y = 16 * yt + mm_perm<T>(c);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int x = 16 * xt + 4 * i + gq;
+    if (x > n1 / 2 || y > n2 / 2) continue;
+    const bool mx = x != 0 && 2 * x != n1, my = y != 0 && 2 * y != n2;
+    o[(size_t)y * n1 + x] = acc[i][0];
+    if (mx) o[(size_t)y * n1 + n1 - x] = acc[i][1];
+    if (my) o[(size_t)(n2 - y) * n1 + x] = acc[i][2];
+    if (mx && my) o[(size_t)(n2 - y) * n1 + n1 - x] = acc[i][3];
+  }
+}
+
 }  // namespace pw

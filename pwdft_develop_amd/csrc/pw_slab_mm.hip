@@ -207,13 +207,20 @@ bool mm_slab_ready(const pw_ctx* c) {
 }
 
 template <typename T>
-int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
+static MmArgs<T> mm_args(const pw_ctx* c, int nb) {
   typedef typename cx<T>::t C;
   const SlabMm* m = c->mm;
   const int d = sizeof(T) == 8 ? PW_F64 : PW_F32;
   const C* tab = (const C*)m->tab[d];
-  MmArgs<T> a{tab, tab + m->off_hx, tab + m->off_ky, tab + m->off_hy, m->sp[d], (const typename MmV<T>::t*)m->v[d],
-              m->TX, m->TY, m->XS, m->YS, c->n3, c->sp.nstick, nb, m->half, m->shared};
+  return MmArgs<T>{tab, tab + m->off_hx, tab + m->off_ky, tab + m->off_hy, m->sp[d], (const typename MmV<T>::t*)m->v[d],
+                   m->TX, m->TY, m->XS, m->YS, c->n3, c->sp.nstick, nb, m->half, m->shared};
+}
+
+template <typename T>
+int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
+  typedef typename cx<T>::t C;
+  const SlabMm* m = c->mm;
+  const int d = sizeof(T) == 8 ? PW_F64 : PW_F32;
   const auto kern = mm_kernel<T>(m->KS);
   const size_t lds = mm_lds<T>(m->KS, m->TX, m->TY, m->shared);
   PW_TRY(ensure_lds((const void*)kern, lds));
@@ -228,10 +235,44 @@ int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
   const int items = c->n3 * ((nb + kMmWaves - 1) / kMmWaves);
   // (8 at least: every XCD's run of items needs a workgroup)
   hipLaunchKernelGGL(kern, dim3((unsigned)std::max(8, std::min(items, gr.blocks))), dim3(64 * kMmWaves), lds,
-                     c->stream, (const C*)t1, (C*)t2, a);
+                     c->stream, (const C*)t1, (C*)t2, mm_args<T>(c, nb));
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
+
+// Splits of the bands that give the density about four waves per SIMD.
+int mm_density_splits(const pw_ctx* c, int nb) {
+  if (!c->mm) return 0;
+  const long tiles = (long)c->n3 * c->mm->TX * c->mm->TY;
+  return (int)std::max<long>(1, std::min<long>({(long)nb, 16, (4096 + tiles - 1) / tiles}));
+}
+
+template <typename T>
+int mm_density(pw_ctx* c, int nb, const void* t1, const double* f, int nsplit, double* part) {
+  typedef typename cx<T>::t C;
+  const SlabMm* m = c->mm;
+  const long units = (long)c->n3 * m->TX * m->TY * nsplit;
+  const dim3 grid((unsigned)((units + kMmWaves - 1) / kMmWaves)), block(64 * kMmWaves);
+#define PW_MM_DENSITY(K)                                                                                       \
+  case K:                                                                                                      \
+    hipLaunchKernelGGL((k_density_mm<T, K, kMmWaves>), grid, block, 0, c->stream, (const C*)t1, mm_args<T>(c, nb), f, \
+                       1.0 / (double)c->N, nsplit, c->n1, c->n2, part);                                        \
+    break;
+  switch (m->KS) {
+    PW_MM_DENSITY(2)
+    PW_MM_DENSITY(3)
+    PW_MM_DENSITY(4)
+    PW_MM_DENSITY(5)
+    PW_MM_DENSITY(6)
+    PW_MM_DENSITY(8)
+    default: return fail(PW_ERR_STATE, "mm_density: no kernel for %d k-steps", m->KS);
+  }
+#undef PW_MM_DENSITY
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+template int mm_density<double>(pw_ctx*, int, const void*, const double*, int, double*);
+template int mm_density<float>(pw_ctx*, int, const void*, const double*, int, double*);
 template bool mm_slab_ready<double>(const pw_ctx*);
 template bool mm_slab_ready<float>(const pw_ctx*);
 template int mm_slab<double>(pw_ctx*, int, const void*, void*);

@@ -313,6 +313,9 @@ extern "C" int pw_free_workspace(pw_ctx* c) {
   c->eig_ws_bytes = 0;
   if (c->d_geig_ws) (void)hipFree(c->d_geig_ws);
   c->d_geig_ws = nullptr;
+  if (c->d_adj_ws) (void)hipFree(c->d_adj_ws);
+  c->d_adj_ws = nullptr;
+  c->adj_ws_bytes = 0;
   c->geig_ws_bytes = 0;
   // the captured filter graph refers to the workspace: drop it too
   if (c->fg_exec) (void)hipGraphExecDestroy(c->fg_exec);

@@ -158,21 +158,32 @@ class Context:
 
     # ---- inputs that the adjoint differentiates ----
     def set_vtot(self, vtot):
+        """Host array or tensor of N values; a device tensor stays there."""
+        t = self.torch
+        if isinstance(vtot, t.Tensor):
+            if vtot.is_cuda and not vtot.is_complex() and vtot.numel() == int(np.prod(self.prob.grid)):
+                v = vtot.detach().to(device=self.device, dtype=t.float64).contiguous()
+                self._after_current(v)
+                check(_lib.lib().pw_set_vtot_device(self.h, C.c_void_p(v.data_ptr())))
+                return
+            vtot = vtot.detach().cpu().numpy()
         v = np.ascontiguousarray(np.asarray(vtot, dtype=np.float64).reshape(-1))
         check(_lib.lib().pw_set_vtot(self.h, v))
+
+    def _after_current(self, v):
+        """Work of the context's stream on v comes after what made v."""
+        cur = self.torch.cuda.current_stream(self.device)
+        if cur != self.stream:
+            self.stream.wait_stream(cur)
+            v.record_stream(self.stream)
 
     def set_atoms(self, pos):
         """Rebuild the Gaussian projector block at new atom positions (same
         recipe and couplings as the problem) and load it."""
         p = self.prob
         pos = np.ascontiguousarray(np.asarray(pos, dtype=np.float64).reshape(-1, 3))
-        beta = np.zeros(2 * p.npw * p.nbeta)
-        w = np.zeros(p.nbeta)
-        check(_lib.lib().pw_gaussian_projectors(
-            np.asarray(p.grid, np.int32), np.ascontiguousarray(p.supercell, np.float64).reshape(-1), p.npw, p.idx,
-            len(pos), pos.reshape(-1), p.proj_sigma, p.lmax, np.ascontiguousarray(p.wgt_channel.reshape(-1)),
-            beta, w))
-        check(_lib.lib().pw_set_nonlocal(self.h, p.nbeta, beta, w))
+        check(_lib.lib().pw_set_gaussian_projectors(self.h, len(pos), pos.reshape(-1), p.proj_sigma, p.lmax,
+                                                    np.ascontiguousarray(p.wgt_channel.reshape(-1))))
         self.atoms_loaded = pos.copy()
 
     def density(self, x, f, out=None, accumulate=False):
