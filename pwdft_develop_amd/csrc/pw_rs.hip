@@ -8,30 +8,37 @@
 // Per batch of bands (all on the handle's stream), when every grid length
 // factors into 2, 3, 5 and at most one prime 7..31 (the reference's decks:
 // 62 = 2*31, 124 = 4*31, 88 = 8*11, 102 = 2*3*17):
-//   1. coarse R2C of psi: k_rs_x_r2c (rows), k_rs_pencil along y and z
-//   2. fine C2R restricted to the coarse band: k_rs_zinv_c2f (inverse z of
-//      the live columns, gathered from the coarse spectrum by IP_c2f's
-//      rules), k_rs_pencil along y, k_rs_x_c2r (writing psi and V psi)
+//   1. coarse R2C of psi
+//   2. fine C2R restricted to the coarse band, its inverse z transform reading
+//      the live columns from the coarse spectrum by IP_c2f's rules
 //   3. k_rs_weights: w[p, b] = vol/Nf * wgt_p * sum_i val_p[i] psi_b[idx[i]]
 //   4. k_rs_nl_apply once per colour of a colouring of the atoms by shared
-//      points (V psi += projector terms); k_rs_vmul + k_rs_local (V psi and
-//      the projector terms through a point-major index of the entries) when
-//      an atom lists a point twice
-//   5. fine R2C keeping the coarse band: k_rs_x_r2c, k_rs_pencil along y and
-//      z (live rows and planes only)
+//      points (psi <- V psi + projector terms on their points); k_rs_local (V
+//      psi and the projector terms everywhere, through a point-major index of
+//      the entries) when an atom lists a point twice
+//   5. fine R2C of what 4 left, times V off the projectors' points, keeping
+//      the coarse band
 //   6. k_rs_f2c_ekin_p: IP_f2c as a gather on that pruned spectrum plus the
 //      kinetic term
-//   7. coarse C2R: k_rs_pencil along z and y, k_rs_x_c2r straight into a3.
+//   7. coarse C2R straight into a3.
+// The transforms are k_rs_plane_fwd / _inv (x and y together) and
+// k_rs_pencil_mm (z) on matrix cores for coarse lengths up to 62 and fine ones
+// up to 126 (442 bands of 62^3 / 124^3: 30.3 -> 15.7 ms with the potential
+// folded into step 5), and k_rs_x_r2c, k_rs_x_c2r, k_rs_pencil, k_rs_zinv_c2f
+// (butterflies in LDS, one axis a pass) beyond, where the k axis no longer
+// fits two 16-column tiles.
 // Other lengths are refused (PW_ERR_UNSUPPORTED).  FFTWExecute's vol/N and 1/vol factors
 // (src/SCF/fourier.cpp:695-760) cancel pairwise and are folded into the
 // gathers as 1/Nc and 1/Nf.
 
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <mutex>
 
 #include "pw_fft.h"
 #include "pw_internal.h"
+#include "pw_rs_mm.h"
 
 using namespace pw;
 
@@ -45,10 +52,27 @@ struct AtomRec {
 
 constexpr int kRowThreads = 64;
 constexpr int kNlBands = 16;  // bands per k_rs_nl_apply workgroup
+constexpr unsigned kNlFirst = 1u << 31;  // fine-grid indices are below 2^31
+constexpr int kNlSplits = 8;  // most splits of the weights' sums
 
 }  // namespace
 
+// Matrix-core transforms (pw_rs_mm.h) of a handle whose coarse lengths are at
+// most 62 and fine ones at most 126.
+struct RsMm {
+  int KS = 0;                            // k-steps of the planes' axes (x and y together)
+  int KZ = 0;                            // k-steps of the z axis
+  RsAxis cx, cy, fx, fy, cz, fz;
+  const int *c_rp, *c_rm, *f_rp, *f_rm;  // spectrum rows of a coarse and of a fine plane (32 entries)
+  const int *cz_p, *cz_m;                // coarse z entries by +-k
+  const int *lz_p, *lz_m;                // live fine planes by +-k
+  const int *gz_p, *gz_m;                // coarse z entries that feed the fine +-k
+  const int *fz_p, *fz_m;                // fine z by +-h
+  void* buf = nullptr;
+};
+
 struct pw_rs {
+  RsMm* mm = nullptr;
   int nc[3], nf[3];
   int hc0, hf0;             // n0/2 + 1 of the coarse and the fine grid
   long Nc, Nf, Hc, Hf;      // real and half-spectrum sizes per band
@@ -60,10 +84,11 @@ struct pw_rs {
   double* d_teter = nullptr;    // b / (b + 16 a^4), a = 2 ekin (CalculateEkin)
   double* d_vtot = nullptr;
   // projectors
-  int natom = 0, nproj_tot = 0, npmax = 0;
+  int natom = 0, nproj_tot = 0, npmax = 0, ptmax = 0;  // ptmax: points of the largest atom
   AtomRec* d_atab = nullptr;
   int* d_apt_off = nullptr;   // natom + 1 offsets into d_idx
   int* d_idx = nullptr;
+  unsigned* d_pts = nullptr;  // d_idx with kNlFirst on each point's first colour
   double* d_val = nullptr;
   double* d_wgt = nullptr;
   int* d_rowptr = nullptr;    // Nf + 1
@@ -86,7 +111,7 @@ struct pw_rs {
   double2* d_u0 = nullptr;      // [m][l][i]  nz x ny x hc
   double2* d_cv = nullptr;      // coarse [z][y][i] scratch
   double2* d_cw = nullptr;
-  double* d_pv = nullptr;       // V psi on the fine grid (fused local term)
+  double* d_vfwd = nullptr;     // the forward transform's factors of psi (k_rs_vfwd)
   double* d_f = nullptr;        // density weights of a batch, then sums
   double* d_part = nullptr;     // partial sums (kSumBlocks)
   int* d_ymap = nullptr;        // fine y -> live row or -1 (f1)
@@ -101,9 +126,13 @@ struct pw_rs {
 // ---------------------------------------------------------------- kernels
 
 // Step 4: projector weights of one atom for BB bands.  Grid (natom, band
-// groups), 256 threads striding over the atom's points; NPMAX x BB partial
-// sums per thread, reduced across each wavefront with DPP and across the
-// four wavefronts through LDS.  coef[p * nbc + b].
+// groups, splits of the points), 256 threads striding over the atom's points;
+// NPMAX x BB partial sums per thread, reduced across each wavefront with DPP
+// and across the four wavefronts through LDS.  coef[split * ldc + p * nbc +
+// b], the splits added in order by the reader.  A dozen atoms and bands give
+// too few workgroups to hide a chain of 14 dependent gathers each: with the
+// points split to about 2048 workgroups an 8-atom, 16-band call spends 6 us
+// here against 49, and 8 us per colour against 131 in the update.
 template <int NPMAX, int BB>
 __global__ __launch_bounds__(256) void k_rs_weights(const double* __restrict__ pf,
                                                    const AtomRec* __restrict__ atab,
@@ -111,7 +140,7 @@ __global__ __launch_bounds__(256) void k_rs_weights(const double* __restrict__ p
                                                    const int* __restrict__ idx,
                                                    const double* __restrict__ val,
                                                    const double* __restrict__ wgt,
-                                                   double* __restrict__ coef, int nbc, long Nf,
+                                                   double* __restrict__ coef, long ldc, int nbc, long Nf,
                                                    double scale) {
   __shared__ double part[4][NPMAX * BB];
   const int a = blockIdx.x;
@@ -125,7 +154,7 @@ __global__ __launch_bounds__(256) void k_rs_weights(const double* __restrict__ p
   for (int p = 0; p < NPMAX; p++)
 #pragma unroll
     for (int q = 0; q < BB; q++) acc[p][q] = 0.0;
-  for (int i = threadIdx.x; i < rec.npts; i += 256) {
+  for (int i = blockIdx.z * 256 + threadIdx.x; i < rec.npts; i += 256 * gridDim.z) {
     const long r = ia[i];
     double ps[BB];
 #pragma unroll
@@ -152,7 +181,7 @@ __global__ __launch_bounds__(256) void k_rs_weights(const double* __restrict__ p
     const int p = t / BB, q = t % BB;
     if (q < nbb) {
       const double s = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
-      coef[(long)(rec.pg0 + p) * nbc + b0 + q] = s * (scale * wgt[rec.pg0 + p]);
+      coef[blockIdx.z * ldc + (long)(rec.pg0 + p) * nbc + b0 + q] = s * (scale * wgt[rec.pg0 + p]);
     }
   }
 }
@@ -198,43 +227,32 @@ __global__ __launch_bounds__(256) void k_rs_local(double* __restrict__ pf,
   }
 }
 
-// Step 5, split for speed when the atoms colour cleanly: pf <- vtot .* pf
-// over the whole fine grid (two points and eight bands per thread) ...
-__global__ __launch_bounds__(256) void k_rs_vmul(double* __restrict__ pf, const double* __restrict__ vtot,
-                                                int nbc, long Nf) {
-  const long r = 2 * ((long)blockIdx.x * 256 + threadIdx.x);
-  if (r >= Nf) return;
-  const int b0 = blockIdx.y * 8;
-  const int nbb = min(8, nbc - b0);
-  if (r + 1 < Nf) {
-    const double2 v = *reinterpret_cast<const double2*>(vtot + r);
-    double2 x[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (q < nbb) x[q] = *reinterpret_cast<const double2*>(pf + (long)(b0 + q) * Nf + r);
-#pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (q < nbb) {
-        x[q].x *= v.x;
-        x[q].y *= v.y;
-        *reinterpret_cast<double2*>(pf + (long)(b0 + q) * Nf + r) = x[q];
-      }
-  } else {
-    for (int q = 0; q < nbb; q++) pf[(long)(b0 + q) * Nf + r] *= vtot[r];
-  }
+// Step 5, split for speed when the atoms colour cleanly: V psi is formed where
+// the forward transform reads psi, by the factors vfwd = V off the projectors'
+// points and 1 on them, where the first colour's update has already replaced
+// psi by V psi.  No array holds V psi beside psi: the inverse transform of the
+// 62 / 124-point deck writes 15 MB a band instead of 30.
+__global__ __launch_bounds__(256) void k_rs_vfwd(const double* __restrict__ vtot, const int* __restrict__ rowptr,
+                                                double* __restrict__ out, long Nf) {
+  for (long r = (long)blockIdx.x * 256 + threadIdx.x; r < Nf; r += (long)gridDim.x * 256)
+    out[r] = rowptr && rowptr[r + 1] > rowptr[r] ? 1.0 : vtot[r];
 }
 
-// ... then, one launch per colour, each atom's projectors added at its own
-// points: pf[b, idx_i] += sum_p val[i, p] coef[p, b].  Atoms of one colour
+// One launch per colour, each atom's projectors added at its own points:
+// pf[b, r_i] = [V(r_i)] pf[b, r_i] + sum_p val[i, p] coef[p, b], the factor V
+// where this colour is the point's first (kNlFirst in pts).  Atoms of one colour
 // share no point, so the read-modify-writes never meet.  Grid (atoms of the
-// colour, groups of kNlBands bands); the atom's coefficient block sits in LDS.
+// colour, groups of kNlBands bands, splits of the points); the atom's
+// coefficient block, summed over the weights' splits in order, sits in LDS.
 template <int NPMAX>
 __global__ __launch_bounds__(256) void k_rs_nl_apply(double* __restrict__ pf, const int* __restrict__ clist,
                                                     const AtomRec* __restrict__ atab,
                                                     const int* __restrict__ apt_off,
-                                                    const int* __restrict__ idx,
+                                                    const unsigned* __restrict__ pts,
+                                                    const double* __restrict__ vtot,
                                                     const double* __restrict__ val,
-                                                    const double* __restrict__ coef, int nbc, long Nf) {
+                                                    const double* __restrict__ coef, int nsplit, long ldc, int nbc,
+                                                    long Nf) {
   constexpr int BG = kNlBands;
   __shared__ double cl[NPMAX * BG];
   const int a = clist[blockIdx.x];
@@ -243,13 +261,18 @@ __global__ __launch_bounds__(256) void k_rs_nl_apply(double* __restrict__ pf, co
   const int nbb = min(BG, nbc - b0);
   for (int t = threadIdx.x; t < rec.np * BG; t += 256) {
     const int p = t / BG, q = t % BG;
-    cl[t] = (q < nbb) ? coef[(long)(rec.pg0 + p) * nbc + b0 + q] : 0.0;
+    double s = 0.0;
+    if (q < nbb)
+      for (int u = 0; u < nsplit; u++) s += coef[u * ldc + (long)(rec.pg0 + p) * nbc + b0 + q];
+    cl[t] = s;
   }
   __syncthreads();
-  const int* ia = idx + apt_off[a];
+  const unsigned* ia = pts + apt_off[a];
   const double* va = val + rec.vo;
-  for (int i = threadIdx.x; i < rec.npts; i += 256) {
-    const long r = ia[i];
+  for (int i = blockIdx.z * 256 + threadIdx.x; i < rec.npts; i += 256 * gridDim.z) {
+    const unsigned e = ia[i];
+    const long r = e & ~kNlFirst;
+    const double vr = e & kNlFirst ? vtot[r] : 1.0;
     double v[NPMAX];
 #pragma unroll
     for (int p = 0; p < NPMAX; p++) v[p] = (p < rec.np) ? va[(long)p * rec.npts + i] : 0.0;
@@ -266,7 +289,7 @@ __global__ __launch_bounds__(256) void k_rs_nl_apply(double* __restrict__ pf, co
 #pragma unroll
         for (int p = 0; p < NPMAX; p++)
           if (p < rec.np) u = fma(v[p], cl[p * BG + q0 + q], u);
-        x[q] += u;
+        x[q] = vr * x[q] + u;
       }
 #pragma unroll
       for (int q = 0; q < 8; q++)
@@ -495,8 +518,8 @@ __global__ __launch_bounds__(256) void k_rs_zinv_c2f(const double2* __restrict__
         const bool ni = (i == In), nj = (j == Jn), nk = (k == Kn);
         double f;
         if (dj == 0 && dk == 0) f = (ni || nj || nk) ? 0.5 : 1.0;
-        else if (dj == 1 && dk == 0) f = (!ni && !nk) ? 0.5 : 0.0;
-        else if (dj == 0) f = (!ni && !nj) ? 0.5 : 0.0;
+        else if (dj == 1 && dk == 0) f = (!ni && (!nk || f2 == c2)) ? 0.5 : 0.0;
+        else if (dj == 0) f = (!ni && (!nj || ny == c1)) ? 0.5 : 0.0;  // (ny == c1: y not refined)
         else f = !ni ? 0.5 : 0.0;
         if (f != 0.0) {
           const double2 x = xc[b * Hc + ((long)k * c1 + j) * hc + i];
@@ -582,8 +605,7 @@ __global__ __launch_bounds__(256) void k_rs_pencil(PenArgs a, const double* __re
 template <int PR>
 __global__ __launch_bounds__(256) void k_rs_x_c2r(const double2* __restrict__ in, double* __restrict__ out,
                                                  const double2* __restrict__ twg, const double* __restrict__ cs,
-                                                 int n, int hw, int npair, long in_bs, long out_bs, int P,
-                                                 const double* __restrict__ vloc, double* __restrict__ out2) {
+                                                 int n, int hw, int npair, long in_bs, long out_bs, int P) {
   extern __shared__ double2 sm[];
   const int ld = n;
   double2* tw = sm;
@@ -630,24 +652,18 @@ __global__ __launch_bounds__(256) void k_rs_x_c2r(const double2* __restrict__ in
       double2* o = reinterpret_cast<double2*>(out + b * out_bs + off);
       o[0] = make_double2(z0.x, z1.x);
       o[h] = make_double2(z0.y, z1.y);
-      if (vloc) {
-        // V psi beside psi (the local-potential term of the fine grid)
-        const double2 v0 = *reinterpret_cast<const double2*>(vloc + off);
-        const double2 v1 = *reinterpret_cast<const double2*>(vloc + off + n);
-        double2* o2 = reinterpret_cast<double2*>(out2 + b * out_bs + off);
-        o2[0] = make_double2(v0.x * z0.x, v0.y * z1.x);
-        o2[h] = make_double2(v1.x * z0.y, v1.y * z1.y);
-      }
     }
   }
 }
 
-// R2C of real rows along x, two rows per complex transform, keeping the
-// first hw entries of each row's half spectrum.
+// R2C of real rows along x (times the potential vloc where given), two rows
+// per complex transform, keeping the first hw entries of each row's half
+// spectrum.
 template <int PR>
 __global__ __launch_bounds__(256) void k_rs_x_r2c(const double* __restrict__ in, double2* __restrict__ out,
                                                  const double2* __restrict__ twg, const double* __restrict__ cs,
-                                                 int n, int hw, int npair, long in_bs, long out_bs, int P) {
+                                                 int n, int hw, int npair, long in_bs, long out_bs, int P,
+                                                 const double* __restrict__ vloc) {
   extern __shared__ double2 sm[];
   const int ld = n;
   double2* tw = sm;
@@ -664,8 +680,10 @@ __global__ __launch_bounds__(256) void k_rs_x_r2c(const double* __restrict__ in,
     const int e = t % n, p = t / n, g = g0 + p;
     double2 z = make_double2(0.0, 0.0);
     if (t < P * n && g < npair) {
-      const double* r0 = in + b * in_bs + (long)(2 * g) * n;
-      z = make_double2(__builtin_nontemporal_load(r0 + e), __builtin_nontemporal_load(r0 + n + e));
+      const long row = (long)(2 * g) * n + e;
+      const double* r0 = in + b * in_bs + row;
+      z = make_double2(__builtin_nontemporal_load(r0), __builtin_nontemporal_load(r0 + n));
+      if (vloc) z = make_double2(vloc[row] * z.x, vloc[row + n] * z.y);
     }
     vt[it] = z;
   }
@@ -854,12 +872,14 @@ void free_nonlocal(pw_rs* rs) {
   hipFree(rs->d_rowptr);
   hipFree(rs->d_ent);
   hipFree(rs->d_clist);
+  hipFree(rs->d_pts);
   hipFree(rs->d_coef);
   rs->d_atab = nullptr;
   rs->d_apt_off = rs->d_idx = rs->d_rowptr = nullptr;
   rs->d_val = rs->d_wgt = rs->d_coef = nullptr;
   rs->d_ent = nullptr;
   rs->d_clist = nullptr;
+  rs->d_pts = nullptr;
   rs->ncolor = 0;
   rs->color_off.clear();
   rs->natom = rs->nproj_tot = rs->npmax = 0;
@@ -949,12 +969,86 @@ int setup_own_fft(pw_rs* rs) {
   const size_t tz = (size_t)rs->nf[2] * rs->ny * hc, tf = (size_t)rs->nf[2] * rs->nf[1] * hc;
   const size_t u0 = (size_t)rs->nz * rs->ny * hc;
   if (hipMalloc((void**)&rs->d_tz, sizeof(double2) * tz * ch) != hipSuccess ||
-      hipMalloc((void**)&rs->d_tf, sizeof(double2) * tf * ch) != hipSuccess ||
+      (!rs->mm && hipMalloc((void**)&rs->d_tf, sizeof(double2) * tf * ch) != hipSuccess) ||
       hipMalloc((void**)&rs->d_u0, sizeof(double2) * u0 * ch) != hipSuccess ||
       hipMalloc((void**)&rs->d_cv, sizeof(double2) * rs->Hc * ch) != hipSuccess ||
-      hipMalloc((void**)&rs->d_cw, sizeof(double2) * rs->Hc * ch) != hipSuccess ||
-      hipMalloc((void**)&rs->d_pv, sizeof(double) * rs->Nf * ch) != hipSuccess)
+      (!rs->mm && hipMalloc((void**)&rs->d_cw, sizeof(double2) * rs->Hc * ch) != hipSuccess) ||
+      hipMalloc((void**)&rs->d_vfwd, sizeof(double) * rs->Nf) != hipSuccess)
     return fail(PW_ERR_NOMEM, "pw_rs_create: cannot allocate %d-band transform buffers", rs->chunk);
+  return PW_OK;
+}
+
+// Storage index of +k and -k, k <= c / 2, of a c-point axis whose -c/2 entry
+// is its own (f == c) or sits behind the others (f > c).
+void pair_map(int c, int f, std::vector<int>& p, std::vector<int>& m) {
+  const int K = c / 2 + 1;
+  p.assign((size_t)std::max(K, 32), -1);
+  m = p;
+  for (int k = 0; k < K; k++) {
+    p[(size_t)k] = k;
+    m[(size_t)k] = k == 0 ? -1 : 2 * k < c ? c - k : f > c ? c : -1;
+  }
+}
+
+int setup_mm(pw_rs* rs) {
+  const int *nc = rs->nc, *nf = rs->nf;
+  for (int d = 0; d < 3; d++)
+    if (nc[d] > 62 || nf[d] > 126) return PW_OK;
+  auto steps = [](int c) {
+    const int k = (c / 2 + 4) / 4;  // ceil((c / 2 + 1) / 4)
+    return k <= 2 ? 2 : k == 7 ? 8 : k;
+  };
+  RsMm* m = new RsMm();
+  rs->mm = m;
+  m->KS = std::max(steps(nc[0]), steps(nc[1]));
+  m->KZ = steps(nc[2]);
+  std::vector<double2> tab;
+  std::vector<int> ints;
+  auto axis = [&](int n, int kmax, int KS, size_t* kt, size_t* ht) {
+    const int T = (n / 2 + 16) / 16, TK = (KS + 3) / 4;
+    *kt = tab.size();
+    *ht = *kt + 64 * (size_t)KS * T;
+    tab.resize(*ht + 64 * (size_t)4 * TK * T);
+    axis_tables<double>(n, kmax, KS, T, tab.data() + *kt);
+  };
+  size_t at[6][2];
+  const bool sq = nc[0] == nc[1] && nf[0] == nf[1];  // the y axes share the x tables
+  axis(nc[0], nc[0] / 2, m->KS, &at[0][0], &at[0][1]);
+  axis(nf[0], nc[0] / 2, m->KS, &at[2][0], &at[2][1]);
+  for (int d : {0, 2}) { at[d + 1][0] = at[d][0]; at[d + 1][1] = at[d][1]; }
+  if (!sq) {
+    axis(nc[1], nc[1] / 2, m->KS, &at[1][0], &at[1][1]);
+    axis(nf[1], nc[1] / 2, m->KS, &at[3][0], &at[3][1]);
+  }
+  axis(nc[2], nc[2] / 2, m->KZ, &at[4][0], &at[4][1]);
+  axis(nf[2], nc[2] / 2, m->KZ, &at[5][0], &at[5][1]);
+  size_t off[12];
+  auto ints_of = [&](const std::vector<int>& v, size_t* o) {
+    *o = ints.size();
+    ints.insert(ints.end(), v.begin(), v.end());
+  };
+  std::vector<int> p, q;
+  const int spec[6][2] = {{nc[1], nc[1]}, {nc[1], nf[1]}, {nc[2], nc[2]}, {nc[2], nf[2]}, {nc[2], nf[2]}, {nf[2], nf[2]}};
+  for (int i = 0; i < 6; i++) {
+    pair_map(spec[i][0], spec[i][1], p, q);
+    if (i == 4 && nf[2] > nc[2]) q[(size_t)(nc[2] / 2)] = nc[2] / 2;  // the fine -c/2 is fed by the coarse c/2
+    ints_of(p, &off[2 * i]);
+    ints_of(q, &off[2 * i + 1]);
+  }
+  const size_t tb = sizeof(double2) * tab.size(), ib = sizeof(int) * ints.size();
+  std::vector<unsigned char> host(tb + ib);
+  memcpy(host.data(), tab.data(), tb);
+  memcpy(host.data() + tb, ints.data(), ib);
+  PW_HIP(hipMalloc(&m->buf, host.size()));
+  PW_HIP(hipMemcpy(m->buf, host.data(), host.size(), hipMemcpyHostToDevice));
+  const double2* t = (const double2*)m->buf;
+  const int* n = (const int*)((unsigned char*)m->buf + tb);
+  RsAxis* ax[6] = {&m->cx, &m->cy, &m->fx, &m->fy, &m->cz, &m->fz};
+  const int len[6] = {nc[0], nc[1], nf[0], nf[1], nc[2], nf[2]};
+  for (int i = 0; i < 6; i++) *ax[i] = RsAxis{t + at[i][0], t + at[i][1], len[i], len[i] / 2 + 1, (len[i] / 2 + 16) / 16};
+  const int** dst[12] = {&m->c_rp, &m->c_rm, &m->f_rp, &m->f_rm, &m->cz_p, &m->cz_m,
+                         &m->lz_p, &m->lz_m, &m->gz_p, &m->gz_m, &m->fz_p, &m->fz_m};
+  for (int i = 0; i < 12; i++) *dst[i] = n + off[i];
   return PW_OK;
 }
 
@@ -1019,7 +1113,7 @@ extern "C" int pw_rs_create(pw_rs** out, const int grid[3], const int grid_fine[
   if (hipMalloc((void**)&rs->d_xc, sizeof(double2) * rs->Hc * rs->chunk) != hipSuccess ||
       hipMalloc((void**)&rs->d_pf, sizeof(double) * rs->Nf * rs->chunk) != hipSuccess)
     return bail(fail(PW_ERR_NOMEM, "pw_rs_create: cannot allocate %d-band chunk buffers", rs->chunk));
-  if ((rc = setup_own_fft(rs)) != PW_OK) return bail(rc);
+  if ((rc = setup_mm(rs)) != PW_OK || (rc = setup_own_fft(rs)) != PW_OK) return bail(rc);
   *out = rs;
   return PW_OK;
 }
@@ -1040,7 +1134,7 @@ extern "C" int pw_rs_destroy(pw_rs* rs) {
   hipFree(rs->d_u0);
   hipFree(rs->d_cv);
   hipFree(rs->d_cw);
-  hipFree(rs->d_pv);
+  hipFree(rs->d_vfwd);
   hipFree(rs->d_f);
   hipFree(rs->d_part);
   hipFree(rs->d_ymap);
@@ -1049,6 +1143,8 @@ extern "C" int pw_rs_destroy(pw_rs* rs) {
   hipFree(rs->d_mmap);
   hipFree(rs->d_cs);
   for (auto& kv : rs->d_tw) hipFree(kv.second);
+  if (rs->mm) hipFree(rs->mm->buf);
+  delete rs->mm;
   delete rs;
   return PW_OK;
 }
@@ -1069,12 +1165,24 @@ extern "C" int pw_rs_info(const pw_rs* rs, long* ntot, long* ntot_fine, int* chu
   return PW_OK;
 }
 
+namespace {
+// after the potential or the projectors have changed
+int forward_factors(pw_rs* rs) {
+  if (!rs->d_vtot) return PW_OK;
+  const bool nl = rs->natom > 0 && rs->nproj_tot > 0;
+  hipLaunchKernelGGL(k_rs_vfwd, dim3((unsigned)std::min<long>((rs->Nf + 255) / 256, 4096)), dim3(256), 0, rs->stream,
+                     (const double*)rs->d_vtot, (const int*)(nl ? rs->d_rowptr : nullptr), rs->d_vfwd, rs->Nf);
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+}  // namespace
+
 extern "C" int pw_rs_set_vtot(pw_rs* rs, const double* vtot) {
   if (!rs || !vtot) return fail(PW_ERR_ARG, "pw_rs_set_vtot: bad argument");
   PW_HIP(hipStreamSynchronize(rs->stream));
   if (!rs->d_vtot) PW_HIP(hipMalloc((void**)&rs->d_vtot, sizeof(double) * rs->Nf));
   PW_HIP(hipMemcpy(rs->d_vtot, vtot, sizeof(double) * rs->Nf, hipMemcpyHostToDevice));
-  return PW_OK;
+  return forward_factors(rs);
 }
 
 extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const int* nproj,
@@ -1122,6 +1230,7 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
   // than 32 colours, leaves the point-major kernel in charge
   int ncolor = 0;
   std::vector<int> color_of((size_t)natom, 0);
+  std::vector<unsigned> pts((size_t)tot_pts);
   {
     std::vector<uint32_t> mask((size_t)rs->Nf, 0u);
     std::vector<int> stamp((size_t)rs->Nf, -1);
@@ -1141,6 +1250,11 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
       for (int i = 0; i < npts[a]; i++) mask[idx[apt_off[a] + i]] |= 1u << c;
     }
     if (!ok) ncolor = 0;
+    for (int a = 0; a < natom && ok; a++)
+      for (int i = apt_off[a]; i < apt_off[a + 1]; i++) {
+        const bool first = (mask[idx[i]] & ((1u << color_of[a]) - 1u)) == 0;
+        pts[(size_t)i] = (unsigned)idx[i] | (first ? kNlFirst : 0u);
+      }
   }
   std::vector<int> clist, color_off;
   if (ncolor > 0) {
@@ -1161,21 +1275,23 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
       (rc = upload_rs(&rs->d_wgt, wgt, (size_t)tot_proj)) != PW_OK ||
       (rc = upload_rs(&rs->d_rowptr, rowptr.data(), rowptr.size())) != PW_OK ||
       (rc = upload_rs(&rs->d_ent, ent.data(), ent.size())) != PW_OK ||
-      (rc = upload_rs(&rs->d_clist, clist.data(), clist.size())) != PW_OK) {
+      (rc = upload_rs(&rs->d_clist, clist.data(), clist.size())) != PW_OK ||
+      (rc = upload_rs(&rs->d_pts, pts.data(), pts.size())) != PW_OK) {
     free_nonlocal(rs);
     return rc;
   }
   if (tot_proj > 0 &&
-      hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * rs->chunk) != hipSuccess) {
+      hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * rs->chunk * kNlSplits) != hipSuccess) {
     free_nonlocal(rs);
     return fail(PW_ERR_NOMEM, "pw_rs_set_nonlocal: cannot allocate projector weights");
   }
   rs->natom = natom;
   rs->nproj_tot = tot_proj;
   rs->npmax = npmax;
+  rs->ptmax = natom > 0 ? *std::max_element(npts, npts + natom) : 0;
   rs->ncolor = ncolor;
   rs->color_off = color_off;
-  return PW_OK;
+  return forward_factors(rs);
 }
 
 namespace {
@@ -1194,7 +1310,7 @@ int launch_pencil(pw_rs* rs, PenArgs a, int nbc) {
 }
 
 int launch_x(pw_rs* rs, bool c2r, const void* in, void* out, int n, int hw, int nrows, long in_bs, long out_bs,
-             int nbc, const double* vt = nullptr, double* out2 = nullptr) {
+             int nbc, const double* vt = nullptr) {
   const int P = pencils(n);
   const int npair = nrows / 2;
   const dim3 g((npair + P - 1) / P, nbc);
@@ -1203,13 +1319,13 @@ int launch_x(pw_rs* rs, bool c2r, const void* in, void* out, int n, int hw, int 
   if (c2r) {
 #define RS_LAUNCH(PRV)                                                                                    \
   hipLaunchKernelGGL(k_rs_x_c2r<PRV>, g, dim3(256), pencil_lds(n, P), rs->stream, (const double2*)in, \
-                     (double*)out, tw, cs, n, hw, npair, in_bs, out_bs, P, vt, out2)
+                     (double*)out, tw, cs, n, hw, npair, in_bs, out_bs, P)
     RS_PR_SWITCH(big_prime(n), RS_LAUNCH)
 #undef RS_LAUNCH
   } else {
 #define RS_LAUNCH(PRV)                                                                                   \
   hipLaunchKernelGGL(k_rs_x_r2c<PRV>, g, dim3(256), pencil_lds(n, P), rs->stream, (const double*)in, \
-                     (double2*)out, tw, cs, n, hw, npair, in_bs, out_bs, P)
+                     (double2*)out, tw, cs, n, hw, npair, in_bs, out_bs, P, vt)
     RS_PR_SWITCH(big_prime(n), RS_LAUNCH)
 #undef RS_LAUNCH
   }
@@ -1217,11 +1333,100 @@ int launch_x(pw_rs* rs, bool c2r, const void* in, void* out, int n, int hw, int 
   return PW_OK;
 }
 
+#define RS_KS_SWITCH(KSV, CALL)                                                    \
+  switch (KSV) {                                                                   \
+    case 2: CALL(2); break;                                                        \
+    case 3: CALL(3); break;                                                        \
+    case 4: CALL(4); break;                                                        \
+    case 5: CALL(5); break;                                                        \
+    case 6: CALL(6); break;                                                        \
+    case 8: CALL(8); break;                                                        \
+    default: return fail(PW_ERR_STATE, "dual-grid plane: no kernel for %d k-steps", KSV); \
+  }
+
+// real planes, times vloc where given -> spectra (coarse, or fine pruned to
+// the coarse band)
+int mm_plane_fwd(pw_rs* rs, bool fine, const double* in, const double* vloc, double2* out, int nbc) {
+  const RsMm* m = rs->mm;
+  constexpr int NW = 4;
+  const RsPlane g{fine ? m->fx : m->cx, fine ? m->fy : m->cy, fine ? m->f_rp : m->c_rp, fine ? m->f_rm : m->c_rm,
+                  rs->hc0, fine ? rs->ny : rs->nc[1], fine ? rs->nf[2] : rs->nc[2], nbc};
+  const int TK = (m->KS + 3) / 4;
+  const size_t lds = sizeof(double2) * 64 * 4 * TK * (g.y.T + (g.x.ht == g.y.ht ? 0 : g.x.T));
+  const dim3 grid((unsigned)(g.nplane * ((nbc + NW - 1) / NW)));
+#define RS_LAUNCH(K)                                                                          \
+  {                                                                                           \
+    const auto kern = vloc ? &k_rs_plane_fwd<K, NW, true> : &k_rs_plane_fwd<K, NW, false>;    \
+    PW_TRY(ensure_lds((const void*)kern, lds));                                               \
+    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, rs->stream, in, g, vloc, out);         \
+  }
+  RS_KS_SWITCH(m->KS, RS_LAUNCH)
+#undef RS_LAUNCH
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+
+// spectra -> real planes
+int mm_plane_inv(pw_rs* rs, bool fine, const double2* in, double* out, int nbc) {
+  const RsMm* m = rs->mm;
+  const RsPlane g{fine ? m->fx : m->cx, fine ? m->fy : m->cy, fine ? m->f_rp : m->c_rp, fine ? m->f_rm : m->c_rm,
+                  rs->hc0, fine ? rs->ny : rs->nc[1], fine ? rs->nf[2] : rs->nc[2], nbc};
+  const size_t lds = rs_plane_inv_lds(m->KS, g.x.T);
+#define RS_LAUNCH(K)                                                                                   \
+  {                                                                                                    \
+    PW_TRY(ensure_lds((const void*)&k_rs_plane_inv<K>, lds));                                          \
+    hipLaunchKernelGGL(k_rs_plane_inv<K>, dim3((unsigned)(g.nplane * nbc)), dim3(256), lds, rs->stream, in, g, out); \
+  }
+  RS_KS_SWITCH(m->KS, RS_LAUNCH)
+#undef RS_LAUNCH
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+
+int mm_pencil(pw_rs* rs, RsPencil g, int TH, bool c2f, int nbc) {
+  constexpr int NW = 4;
+  const int ngrp = (g.ncol + 15) / 16;
+  const long groups = (long)ngrp * nbc;
+  const size_t lds = sizeof(double2) * 64 * TH * g.KS;
+  const dim3 grid((unsigned)std::min<long>((groups + NW - 1) / NW, 1024));
+#define RS_LAUNCH(TH_, C_)                                                                                         \
+  {                                                                                                                \
+    PW_TRY(ensure_lds((const void*)&k_rs_pencil_mm<TH_, C_, NW>, lds));                                            \
+    hipLaunchKernelGGL((k_rs_pencil_mm<TH_, C_, NW>), grid, dim3(64 * NW), lds, rs->stream, g, ngrp, groups);      \
+  }
+  if (c2f) switch (TH) {
+    case 1: RS_LAUNCH(1, true) break;
+    case 2: RS_LAUNCH(2, true) break;
+    case 3: RS_LAUNCH(3, true) break;
+    default: RS_LAUNCH(4, true) break;
+  } else switch (TH) {
+    case 1: RS_LAUNCH(1, false) break;
+    case 2: RS_LAUNCH(2, false) break;
+    case 3: RS_LAUNCH(3, false) break;
+    default: RS_LAUNCH(4, false) break;
+  }
+#undef RS_LAUNCH
+  PW_HIP(hipGetLastError());
+  return PW_OK;
+}
+
+// forward along z: planes of the axis (hp, hm by +-h) -> entries by +-k
+int mm_z_fwd(pw_rs* rs, const RsAxis& ax, const int* hp, const int* hm, const int* kp, const int* km,
+             const double2* in, double2* out, int ncol, long in_bs, long out_bs, int nbc) {
+  const RsPencil g{in, out, ax.ht, hp, hm, kp, km, 4 * ax.T, (ax.H + 3) / 4, ax.H, rs->nc[2] / 2 + 1, ncol, in_bs,
+                   out_bs, ncol, ncol, -1.0, 1.0, 0, 0, 0, 0, 0, 0};
+  return mm_pencil(rs, g, (rs->mm->KZ + 3) / 4, false, nbc);
+}
+
 // coarse psi -> xc (unscaled coarse spectrum)
 int own_coarse_fwd(pw_rs* rs, const double* psi, int nbc) {
   const int* nc = rs->nc;
   const int hc = rs->hc0;
   const long Hc = rs->Hc;
+  if (const RsMm* m = rs->mm) {
+    PW_TRY(mm_plane_fwd(rs, false, psi, nullptr, rs->d_cv, nbc));
+    return mm_z_fwd(rs, m->cz, m->cz_p, m->cz_m, m->cz_p, m->cz_m, rs->d_cv, rs->d_xc, nc[1] * hc, Hc, Hc, nbc);
+  }
   PW_TRY(launch_x(rs, false, psi, rs->d_cv, nc[0], hc, nc[1] * nc[2], rs->Nc, Hc, nbc));
   PenArgs y{rs->d_cv, Hc, (long)nc[1] * hc, hc, nullptr, rs->d_cw, Hc, (long)nc[1] * hc, hc, nullptr,
             nc[1], nc[2], hc, nc[1], 0, -1.0, nullptr};
@@ -1237,6 +1442,13 @@ int own_coarse_inv(pw_rs* rs, double* a3, int nbc) {
   const int* nc = rs->nc;
   const int hc = rs->hc0;
   const long Hc = rs->Hc;
+  if (const RsMm* m = rs->mm) {
+    const int ncol = nc[1] * hc, K = nc[2] / 2 + 1;
+    const RsPencil g{rs->d_xc, rs->d_cv, m->cz.kt, m->cz_p, m->cz_m, m->cz_p, m->cz_m, m->KZ, (K + 3) / 4, K, m->cz.H,
+                     ncol, Hc, Hc, ncol, ncol, 1.0, 1.0, 0, 0, 0, 0, 0, 0};
+    PW_TRY(mm_pencil(rs, g, m->cz.T, false, nbc));
+    return mm_plane_inv(rs, false, rs->d_cv, a3, nbc);
+  }
   PenArgs z{rs->d_xc, Hc, hc, (long)nc[1] * hc, nullptr, rs->d_cv, Hc, hc, (long)nc[1] * hc, nullptr,
             nc[2], nc[1], hc, nc[2], 0, 1.0, nullptr};
   PW_TRY(launch_pencil(rs, z, nbc));
@@ -1248,13 +1460,21 @@ int own_coarse_inv(pw_rs* rs, double* a3, int nbc) {
 }
 
 // coarse psi -> xc (coarse spectrum) -> pf (psi on the fine grid)
-int own_to_fine(pw_rs* rs, const double* psi, int nbc, bool fuse_v) {
+int own_to_fine(pw_rs* rs, const double* psi, int nbc) {
   const int *nc = rs->nc, *nf = rs->nf;
   const int hc = rs->hc0;
   const long Hc = rs->Hc;
   PW_TRY(own_coarse_fwd(rs, psi, nbc));
   // fine inverse: z (with the coarse-to-fine gather), y, x
   const long Tzb = (long)nf[2] * rs->ny * hc, Tfb = (long)nf[2] * nf[1] * hc;
+  if (const RsMm* m = rs->mm) {
+    const int ncol = rs->ny * hc, K = nc[2] / 2 + 1;
+    const RsPencil g{rs->d_xc, rs->d_tz, m->fz.kt, m->gz_p, m->gz_m, m->fz_p, m->fz_m, m->KZ, (K + 3) / 4, K, m->fz.H,
+                     ncol, Hc, Tzb, (long)nc[1] * hc, ncol, 1.0, 1.0 / (double)rs->Nc, nc[0], nc[1], nc[2], hc,
+                     nf[1] == nc[1], nf[2] == nc[2]};
+    PW_TRY(mm_pencil(rs, g, m->fz.T, true, nbc));
+    return mm_plane_inv(rs, true, rs->d_tz, rs->d_pf, nbc);
+  }
   {
     const int P = pencils(nf[2]);
     const dim3 g((rs->ny * hc + P - 1) / P, nbc);
@@ -1270,25 +1490,29 @@ int own_to_fine(pw_rs* rs, const double* psi, int nbc, bool fuse_v) {
   PenArgs yi{rs->d_tz, Tzb, (long)rs->ny * hc, hc, rs->d_ymap, rs->d_tf, Tfb, (long)nf[1] * hc, hc, nullptr,
              nf[1], nf[2], hc, nf[1], 0, 1.0, nullptr};
   PW_TRY(launch_pencil(rs, yi, nbc));
-  PW_TRY(launch_x(rs, true, rs->d_tf, rs->d_pf, nf[0], hc, nf[1] * nf[2], Tfb, rs->Nf, nbc,
-                  fuse_v ? rs->d_vtot : nullptr, rs->d_pv));
+  PW_TRY(launch_x(rs, true, rs->d_tf, rs->d_pf, nf[0], hc, nf[1] * nf[2], Tfb, rs->Nf, nbc));
   return PW_OK;
 }
 
-// pf (H psi terms on the fine grid) -> restriction + kinetic -> a3
-int own_to_coarse(pw_rs* rs, const double* fine, double* a3, int nbc) {
+// vloc .* fine (vloc null: fine) -> restriction + kinetic -> a3
+int own_to_coarse(pw_rs* rs, const double* fine, const double* vloc, double* a3, int nbc) {
   const int *nc = rs->nc, *nf = rs->nf;
   const int hc = rs->hc0;
   const long Hc = rs->Hc;
   const long Tzb = (long)nf[2] * rs->ny * hc, Tfb = (long)nf[2] * nf[1] * hc;
   const long U0b = (long)rs->nz * rs->ny * hc;
-  PW_TRY(launch_x(rs, false, fine, rs->d_tf, nf[0], hc, nf[1] * nf[2], rs->Nf, Tfb, nbc));
+  if (const RsMm* m = rs->mm) {
+    PW_TRY(mm_plane_fwd(rs, true, fine, vloc, rs->d_tz, nbc));
+    PW_TRY(mm_z_fwd(rs, m->fz, m->fz_p, m->fz_m, m->lz_p, m->lz_m, rs->d_tz, rs->d_u0, rs->ny * hc, Tzb, U0b, nbc));
+  } else {
+  PW_TRY(launch_x(rs, false, fine, rs->d_tf, nf[0], hc, nf[1] * nf[2], rs->Nf, Tfb, nbc, vloc));
   PenArgs yf{rs->d_tf, Tfb, (long)nf[1] * hc, hc, nullptr, rs->d_tz, Tzb, (long)rs->ny * hc, hc, rs->d_lmap,
              rs->ny, nf[2], hc, nf[1], 0, -1.0, nullptr};
   PW_TRY(launch_pencil(rs, yf, nbc));
   PenArgs zf{rs->d_tz, Tzb, hc, (long)rs->ny * hc, nullptr, rs->d_u0, U0b, hc, (long)rs->ny * hc, rs->d_mmap,
              rs->nz, rs->ny, hc, nf[2], 0, -1.0, nullptr};
   PW_TRY(launch_pencil(rs, zf, nbc));
+  }
   hipLaunchKernelGGL(k_rs_f2c_ekin_p, dim3(nc[1] * nc[2], nbc), dim3(kRowThreads), 0, rs->stream, rs->d_xc,
                      rs->d_u0, rs->d_ekin, rs->d_ymap, rs->d_zmap, nc[0], nc[1], nc[2], nf[1], nf[2], hc, rs->ny,
                      Hc, U0b, 1.0 / (double)rs->Nc, 1.0 / (double)rs->Nf);
@@ -1296,49 +1520,49 @@ int own_to_coarse(pw_rs* rs, const double* fine, double* a3, int nbc) {
   return own_coarse_inv(rs, a3, nbc);
 }
 
-// Projector weights (from psi on the fine grid, pf), then V psi and the
-// projector terms.  fused: V psi is already in d_pv (written by the C2R
-// row pass) and the projector terms go there; else in place on pf.
-int local_terms(pw_rs* rs, int nbc, bool fused) {
+// Projector weights (from psi on the fine grid, pf), then the projector terms
+// in place on pf: colour by colour, V psi left to the forward transform's
+// factors (k_rs_vfwd) off their points, or whole by k_rs_local.  *vloc: the
+// factors pf still lacks, or null.
+int local_terms(pw_rs* rs, int nbc, const double** vloc) {
   const bool nl = rs->natom > 0 && rs->nproj_tot > 0;
-  double* u = fused ? rs->d_pv : rs->d_pf;
+  *vloc = !nl || rs->ncolor > 0 ? rs->d_vfwd : nullptr;
+  // splits of an atom's points that bring `blocks` workgroups to about 2048,
+  // each with a point per thread at least
+  const int most = (rs->ptmax + 255) / 256;
+  auto splits = [&](long blocks, int cap) {
+    return (int)std::max<long>(1, std::min<long>({2048 / std::max<long>(blocks, 1), (long)most, (long)cap}));
+  };
+  const long ldc = (long)rs->nproj_tot * nbc;
+  int nsplit = 1;
   if (nl) {
     const double scale = rs->vol / (double)rs->Nf;
-    if (rs->npmax <= 8)
-      hipLaunchKernelGGL((k_rs_weights<8, 8>), dim3(rs->natom, (nbc + 7) / 8), dim3(256), 0, rs->stream,
-                         rs->d_pf, rs->d_atab, rs->d_apt_off, rs->d_idx, rs->d_val, rs->d_wgt, rs->d_coef,
-                         nbc, rs->Nf, scale);
-    else if (rs->npmax <= 16)
-      hipLaunchKernelGGL((k_rs_weights<16, 4>), dim3(rs->natom, (nbc + 3) / 4), dim3(256), 0, rs->stream,
-                         rs->d_pf, rs->d_atab, rs->d_apt_off, rs->d_idx, rs->d_val, rs->d_wgt, rs->d_coef,
-                         nbc, rs->Nf, scale);
-    else
-      hipLaunchKernelGGL((k_rs_weights<32, 2>), dim3(rs->natom, (nbc + 1) / 2), dim3(256), 0, rs->stream,
-                         rs->d_pf, rs->d_atab, rs->d_apt_off, rs->d_idx, rs->d_val, rs->d_wgt, rs->d_coef,
-                         nbc, rs->Nf, scale);
+    const int BB = rs->npmax <= 8 ? 8 : rs->npmax <= 16 ? 4 : 2, groups = (nbc + BB - 1) / BB;
+    // (the point-major kernel reads one split)
+    if (rs->ncolor > 0) nsplit = splits((long)rs->natom * groups, kNlSplits);
+    const dim3 g(rs->natom, groups, nsplit);
+#define RS_LAUNCH(NP, B)                                                                                            \
+  hipLaunchKernelGGL((k_rs_weights<NP, B>), g, dim3(256), 0, rs->stream, rs->d_pf, rs->d_atab, rs->d_apt_off,       \
+                     rs->d_idx, rs->d_val, rs->d_wgt, rs->d_coef, ldc, nbc, rs->Nf, scale)
+    if (BB == 8) RS_LAUNCH(8, 8);
+    else if (BB == 4) RS_LAUNCH(16, 4);
+    else RS_LAUNCH(32, 2);
+#undef RS_LAUNCH
     PW_HIP(hipGetLastError());
   }
   if (!nl || rs->ncolor > 0) {
-    if (!fused) {
-      // Nf is even (even grids), so every band row starts 16-byte aligned
-      const unsigned nblk = (unsigned)((rs->Nf / 2 + 255) / 256);
-      hipLaunchKernelGGL(k_rs_vmul, dim3(nblk, (nbc + 7) / 8), dim3(256), 0, rs->stream, rs->d_pf, rs->d_vtot,
-                         nbc, rs->Nf);
-      PW_HIP(hipGetLastError());
-    }
     for (int c = 0; nl && c < rs->ncolor; c++) {
       const int na = rs->color_off[c + 1] - rs->color_off[c];
       const int* cl = rs->d_clist + rs->color_off[c];
-      const dim3 g(na, (nbc + kNlBands - 1) / kNlBands);
-      if (rs->npmax <= 8)
-        hipLaunchKernelGGL(k_rs_nl_apply<8>, g, dim3(256), 0, rs->stream, u, cl, rs->d_atab, rs->d_apt_off,
-                           rs->d_idx, rs->d_val, rs->d_coef, nbc, rs->Nf);
-      else if (rs->npmax <= 16)
-        hipLaunchKernelGGL(k_rs_nl_apply<16>, g, dim3(256), 0, rs->stream, u, cl, rs->d_atab,
-                           rs->d_apt_off, rs->d_idx, rs->d_val, rs->d_coef, nbc, rs->Nf);
-      else
-        hipLaunchKernelGGL(k_rs_nl_apply<32>, g, dim3(256), 0, rs->stream, u, cl, rs->d_atab,
-                           rs->d_apt_off, rs->d_idx, rs->d_val, rs->d_coef, nbc, rs->Nf);
+      const int groups = (nbc + kNlBands - 1) / kNlBands;
+      const dim3 g(na, groups, splits((long)na * groups, most));
+#define RS_LAUNCH(NP)                                                                                          \
+  hipLaunchKernelGGL(k_rs_nl_apply<NP>, g, dim3(256), 0, rs->stream, rs->d_pf, cl, rs->d_atab, rs->d_apt_off,  \
+                     rs->d_pts, rs->d_vtot, rs->d_val, rs->d_coef, nsplit, ldc, nbc, rs->Nf)
+      if (rs->npmax <= 8) RS_LAUNCH(8);
+      else if (rs->npmax <= 16) RS_LAUNCH(16);
+      else RS_LAUNCH(32);
+#undef RS_LAUNCH
       PW_HIP(hipGetLastError());
     }
   } else {
@@ -1357,15 +1581,12 @@ extern "C" int pw_rs_mult_spinor(pw_rs* rs, int nb, const double* psi, double* a
   int dev;
   PW_HIP(hipGetDevice(&dev));
   if (dev != rs->device) return fail(PW_ERR_STATE, "pw_rs_mult_spinor: handle belongs to device %d", rs->device);
-  const int* nc = rs->nc;
-  const int* nf = rs->nf;
   for (int b0 = 0; b0 < nb; b0 += rs->chunk) {
     const int nbc = std::min(rs->chunk, nb - b0);
-    const bool nl = rs->natom > 0 && rs->nproj_tot > 0;
-    const bool fuse_v = !nl || rs->ncolor > 0;
-    PW_TRY(own_to_fine(rs, psi + (long)b0 * rs->Nc, nbc, fuse_v));
-    PW_TRY(local_terms(rs, nbc, fuse_v));
-    PW_TRY(own_to_coarse(rs, fuse_v ? rs->d_pv : rs->d_pf, a3 + (long)b0 * rs->Nc, nbc));
+    const double* vloc = nullptr;
+    PW_TRY(own_to_fine(rs, psi + (long)b0 * rs->Nc, nbc));
+    PW_TRY(local_terms(rs, nbc, &vloc));
+    PW_TRY(own_to_coarse(rs, rs->d_pf, vloc, a3 + (long)b0 * rs->Nc, nbc));
   }
   return PW_OK;
 }
@@ -1402,7 +1623,7 @@ extern "C" int pw_rs_calculate_density(pw_rs* rs, int nb, const double* psi, con
   for (int b0 = 0; b0 < nb; b0 += rs->chunk) {
     const int nbc = std::min(rs->chunk, nb - b0);
     const double* xb = psi + (long)b0 * rs->Nc;
-    PW_TRY(own_to_fine(rs, xb, nbc, false));
+    PW_TRY(own_to_fine(rs, xb, nbc));
     for (int b = 0; b < nbc; b++) f[(size_t)b] = num_spin * occ[b0 + b];
     // the previous batch's accumulation reads d_f: copy in stream order
     PW_HIP(hipMemcpyAsync(rs->d_f, f.data(), sizeof(double) * nbc, hipMemcpyHostToDevice, rs->stream));

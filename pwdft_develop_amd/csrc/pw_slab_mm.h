@@ -33,7 +33,9 @@
 // Bound by the matrix pipes.  Constants (tables of {cos, sin}) come from LDS,
 // one read per four products; V from a copy in operand order.
 #pragma once
+#include <cmath>
 #include <type_traits>
+#include <vector>
 
 #include "pw_fft.h"
 #include "pw_internal.h"
@@ -55,6 +57,38 @@ __device__ __forceinline__ MmV<float>::t mm16(float a, float b, MmV<float>::t c)
 template <typename T>
 __host__ __device__ __forceinline__ int mm_perm(int c) {
   return sizeof(T) == 8 ? c : 4 * (c & 3) + (c >> 2);
+}
+
+// {cos, sin} of 2 pi m / n, m = 0 .. n - 1, the quadrant taken exactly
+inline std::vector<double2> roots_of(int n) {
+  std::vector<double2> w(n);
+  for (long m = 0; m < n; m++) {
+    const long q = 4 * m / n, rem = 4 * m - q * n;
+    const long double a = (long double)rem / (long double)n * 1.57079632679489661923132169163975144L;
+    const double c = (double)cosl(a), s = (double)sinl(a);
+    w[m] = q == 0 ? double2{c, s} : q == 1 ? double2{-s, c} : q == 2 ? double2{-c, -s} : double2{s, -c};
+  }
+  return w;
+}
+
+// The two tables of one axis: kt [T][KS][64] = {cos, sin}(2 pi h k / n) at
+// k = 4 s + lane / 16, h = 16 tile + perm(lane % 16); ht [TK][4 T][64] at h =
+// 4 u + lane / 16, k = 16 tile + perm(lane % 16); zero beyond kmax and n / 2.
+template <typename T>
+inline typename cx<T>::t* axis_tables(int n, int kmax, int KS, int tiles, typename cx<T>::t* out) {
+  const int TK = (KS + 3) / 4, H = n / 2 + 1;
+  const std::vector<double2> w = roots_of(n);
+  auto put = [&](int k, int h) {
+    const double2 e = k <= kmax && h < H ? w[(long)k * h % n] : double2{0, 0};
+    *out++ = typename cx<T>::t{(T)e.x, (T)e.y};
+  };
+  for (int a = 0; a < tiles; a++)
+    for (int s = 0; s < KS; s++)
+      for (int l = 0; l < 64; l++) put(4 * s + l / 16, 16 * a + mm_perm<T>(l % 16));
+  for (int a = 0; a < TK; a++)
+    for (int u = 0; u < 4 * tiles; u++)
+      for (int l = 0; l < 64; l++) put(16 * a + mm_perm<T>(l % 16), 4 * u + l / 16);
+  return out;
 }
 
 // Stick entry of (kx, ky >= 0): x = stick of +ky, y = stick of -ky; kMmNone
