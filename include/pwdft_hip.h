@@ -334,7 +334,7 @@ int pw_set_timing(pw_ctx* ctx, int enable);
 int pw_get_timing(pw_ctx* ctx, double* ms4, int* ncalls);
 
 /* ------------------------------------------------------------------ */
-/* Many independent cells in one persistent launch.  No single counterpart
+/* Many independent cells in one call.  No single counterpart
  * in the reference, which runs one cell per MPI job and applies H band by
  * band (Spinor::AddMultSpinorFineR2C, src/SCF/spinor.cpp:562-677, with
  * EigenSolver::NonlocalMultX, src/EigenSolver/eigensolver.cpp:471-515): a
@@ -347,15 +347,9 @@ int pw_get_timing(pw_ctx* ctx, double* ms4, int* ncalls);
  * The band blocks of all cells live in one device buffer of complex floats
  * (FP32, the PW_F32 layout per cell): cell c's npw[c] x nb[c] block starts
  * at complex offset xoff[c] = sum_{c' < c} npw[c'] nb[c'].
- * One launch of a persistent grid (as many workgroups as the device holds
- * at once) runs every filter step as four stages over queues that mix all
- * cells' items -- z-inverse sticks of one band and 16 x 16 projection tiles;
- * one z plane of one band; z-forward sticks of one band; 64 rows x 16 bands
- * of the projector apply fused with the recurrence -- with a device-wide
- * barrier between stages.  The reset of the barrier and the launch are
- * captured into a hipGraph on the second call of a shape and replayed
- * afterwards.  Calls return after the launch has finished (the barrier's
- * error word is read back: PW_ERR_HIP if a barrier ever timed out). */
+ * The cells run on lanes (streams) whose kernels overlap; every step of every
+ * cell is captured into a hipGraph on the second call of a degree and replayed
+ * afterwards.  Calls return after the work has finished. */
 typedef struct pw_batch pw_batch;
 int pw_batch_create(pw_batch** batch, int ncell, const int* grid, const double* supercell,
                     const int* npw, const int* idx, const int* npad, const int* pad_src,
@@ -364,33 +358,31 @@ int pw_batch_create(pw_batch** batch, int ncell, const int* grid, const double* 
                     const double* wgt, const int* nb, void* stream);
 int pw_batch_destroy(pw_batch* batch);
 int pw_batch_set_stream(pw_batch* batch, void* stream);
-/* Total complex elements of the block buffer, jobs per filter step,
- * workgroups of the persistent grid, LDS bytes per workgroup. */
+/* Total complex elements of the block buffer, jobs (bands of all cells) per
+ * filter step, lanes, and 0 (no LDS is shared by the cells' kernels). */
 int pw_batch_info(const pw_batch* batch, long* xtotal, int* njobs, int* nwg, int* lds);
-/* Re-plan: x row pairs per slab job, 16-stick chunks per z job, workgroups
- * (0 = the default of each; the grid never exceeds what the device holds at
- * once).  The autotuner's knobs. */
+/* Re-plan: nwg lanes (0 = the default; at most 16 and the cell count).  rp
+ * and zc are accepted and have no effect on the plan.  The autotuner's knob. */
 int pw_batch_tune(pw_batch* batch, int rp, int zc, int nwg);
 int pw_batch_set_graphs(pw_batch* batch, int enable);
 
-/* Stage timing of the batched launch (as pw_set_timing / pw_get_timing for a
- * context; no counterpart in the reference): when enabled, the launch stamps
- * the device wall clock after each of its stage barriers, and
- * pw_batch_timing returns the last launch's time per stage (ms, 4 values:
- * z-inverse + projections, xy slabs, z-forward, projector apply +
- * recurrence), summed over its steps.  Enabling or disabling drops a
- * captured graph. */
+/* Stage timing of the batched calls (as pw_set_timing / pw_get_timing for a
+ * context; no counterpart in the reference): when enabled, calls run eagerly
+ * and stamp the device wall clock around the stages of every cell's step, and
+ * pw_batch_timing returns the last call's time per stage (ms, 4 values:
+ * z-inverse, xy slabs, z-forward, projector products + recurrence), summed
+ * over steps and cells (lanes overlap, so the sum exceeds the call's time). */
 int pw_batch_set_timing(pw_batch* batch, int enable);
 int pw_batch_timing(pw_batch* batch, double* stage_ms);
-/* The batch's autotuner (as pw_autotune): times work-per-item, row-pair
- * and z-chunk splits on pw_batch_apply_h over every cell, applies the
- * fastest and records it in cache_path (NULL: no file). */
+/* The batch's autotuner (as pw_autotune): times numbers of lanes on
+ * pw_batch_apply_h over every cell, applies the fastest and records it in
+ * cache_path (NULL: no file). */
 int pw_batch_autotune(pw_batch* batch, const char* cache_path, char* summary, int len);
-/* HX = H X (FP32, local + kinetic + nonlocal) for every cell in one launch;
+/* HX = H X (FP32, local + kinetic + nonlocal) for every cell;
  * X and HX: device, xtotal complex floats each, not aliased. */
 int pw_batch_apply_h(pw_batch* batch, const void* X, void* HX);
 /* Scaled Chebyshev filter of degree m (as pw_cheb_filter, FP32) applied in
- * place to every cell's block in one launch; bounds: host, (a, b, aL) per
+ * place to every cell's block; bounds: host, (a, b, aL) per
  * cell. */
 int pw_batch_cheb_filter(pw_batch* batch, int m, const double* bounds, void* X);
 /* The same filter cell by cell through pw_cheb_filter on each cell's own

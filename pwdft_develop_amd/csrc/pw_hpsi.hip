@@ -818,8 +818,15 @@ extern "C" int pw_get_timing(pw_ctx* c, double* ms, int* ncalls) {
 namespace pw {
 
 // Event k of the current timed call (k = 0..4); no-op when timing is off or
-// the pool is full (the caller then sees fewer timed calls).
+// the pool is full (the caller then sees fewer timed calls).  Under a batch's
+// stage timing a device clock stamp instead.
+__global__ void k_stamp(unsigned long long* p) { *p = wall_clock64(); }
 static int mark(pw_ctx* c, int k) {
+  if (c->stamps) {
+    hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, c->stream, c->stamps + 5 * c->stamp_calls + k);
+    if (k == 4) c->stamp_calls++;
+    return PW_OK;
+  }
   if (!c->timing || c->ev_calls >= pw_ctx::kTimedCalls) return PW_OK;
   PW_HIP(hipEventRecord(c->ev_pool[5 * c->ev_calls + k], c->stream));
   if (k == 4) c->ev_calls++;
@@ -1109,6 +1116,12 @@ int pw::cheb_step_apply(pw_ctx* c, int dtype, int nb, const void* Y, void* HY, c
   PW_TRY(check_call(c, dtype, nb, Y, HY));
   if (dtype == PW_F64) return cheb_step<double>(c, nb, Y, HY, Yp, Ynew, c->d_coef, step);
   return cheb_step<float>(c, nb, Y, HY, Yp, Ynew, c->d_coef_f, step);
+}
+
+int pw::cheb_step_coef(pw_ctx* c, int nb, const void* Y, void* HY, const void* Yp, void* Ynew, const float* coef,
+                       int step) {
+  PW_TRY(check_call(c, PW_F32, nb, Y, HY));
+  return cheb_step<float>(c, nb, Y, HY, Yp, Ynew, coef, step);
 }
 
 extern "C" int pw_mult_spinor(pw_ctx* c, int dtype, int nb, const void* psi, void* a3) {

@@ -241,6 +241,8 @@ int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2);
 int mm_density_splits(const pw_ctx* c, int nb);
 template <typename T>
 int mm_density(pw_ctx* c, int nb, const void* t1, const double* f, int nsplit, double* part);
+// The FP32 step with its coefficients at coef on the device.
+int cheb_step_coef(pw_ctx* c, int nb, const void* Y, void* HY, const void* Yp, void* Ynew, const float* coef, int step);
 // Exact exchange (pw_exx.hip): a3 += V_x psi when the context holds an
 // exchange operator; state freed with the context.
 struct ExxState;
@@ -353,6 +355,8 @@ struct pw_ctx {
   static constexpr int kTimedCalls = 1024;
   bool timing = false;
   std::vector<hipEvent_t> ev_pool;  // 5 events per timed call
+  unsigned long long* stamps = nullptr;  // a batch's stage timing: 5 device clock stamps per call
+  int stamp_calls = 0;
   int ev_calls = 0, ev_total = 0;
   double stage_ms[4] = {0, 0, 0, 0};
 };

@@ -1,7 +1,6 @@
 // The xy slab transform with every 1D FFT in one thread's registers, as
 // workgroup-level device code: slab_xy_reg_body (one z plane of SB bands;
-// the body of pw_hpsi.hip's k_slab_xy_reg, also run by the batched
-// persistent kernel), built from the phases of SlabReg.
+// the body of pw_hpsi.hip's k_slab_xy_reg), built from the phases of SlabReg.
 //
 // For compile-time N1 = N2: one z plane of SB bands per call (bands b0 ..).
 // V's plane is staged once in LDS as (row 2q, row 2q + 1) pairs, one 64-bit
