@@ -625,6 +625,7 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
     for (auto& pl : c->plan) {
       pl.reg = !(sl && std::string(sl).compare(0, 3, "lds") == 0);
       pl.mm = pl.reg;
+      pl.mm_only = sl && std::string(sl) == "mm";  // wherever the context has the plan
       // "reg[:<ly>...]": the transforms held in registers (on matrix cores or
       // as register FFTs with ly lanes per y column), as by default
       if (sl && std::string(sl).compare(0, 4, "reg:") == 0) pl.ly = std::max(1, atoi(sl + 4));
@@ -851,7 +852,7 @@ static size_t slab_lds(const pw_ctx* c, int esz, int rp, int cg) {
 //        40: 40 -> 42                        103 -> 69
 //        48: 58 -> 49 / 22 -> 13 / 20 -> 10  141 -> 82 / 29 -> 20 / 22 -> 12
 //        60: 94 -> 71 / 26 -> 17 / 24 -> 11  348 -> 124 / 54 -> 26 / 28 -> 14
-//        64: 201 -> 121                      438 -> 224
+//        64: 201 -> 117                      438 -> 209
 //        72: 309 -> 250 / 72 -> 51 / 39 -> 22   655 -> 675 / 117 -> 125 / 41 -> 46
 // The quarter plane is padded to 16-row tiles: 32..40 points (17..21 rows)
 // pay most for it, which only FP32 with the whole chip busy loses, and at 72

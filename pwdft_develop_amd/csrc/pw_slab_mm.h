@@ -33,6 +33,7 @@
 // Bound by the matrix pipes.  Constants (tables of {cos, sin}) come from LDS,
 // one read per four products; V from a copy in operand order.
 #pragma once
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -319,6 +320,165 @@ k_slab_mm(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restric
       if (e[s].y >= 0 && !(e[s].y & kMmConj)) dst[e[s].y] = C{a + b, q - p};
     }
   }
+  }
+}
+
+// The same transform for spheres of more than 16 columns, where one wavefront
+// would need the whole register file for its tiles: a workgroup takes NB bands
+// of a plane, wavefront (band, y tile) runs products 1 to 3 for its tile with
+// the class matrices in LDS, and the third products' results go through LDS
+// (two classes at a time, in the class matrices' place) to the fourth, whose
+// (ky, kx) tiles the band's wavefronts share out.  The x tables stay in LDS
+// for all items of a workgroup.
+//
+// Bound by the matrix pipes: a 180 x 180 plane of 45 columns is 5076 products
+// in FP32, 69 ns of the chip; it takes 113 ns, against 173 ns of butterflies in
+// LDS (k_slab_xy), 120 x 120 planes of 30 columns 40 ns against 329.
+template <typename T>
+inline size_t mm_wg_band(int KS, int TY) {  // LDS bytes of one band
+  const int TK = (KS + 3) / 4;
+  return 64 * sizeof(T) * (size_t)TK * std::max(4 * KS, 8 * TY);
+}
+template <typename T>
+inline size_t mm_wg_tables(int KS, int TX) {
+  return 64 * sizeof(typename cx<T>::t) * (size_t)TX * (KS + 4 * ((KS + 3) / 4));
+}
+template <typename T, int TK, int MAXT>
+__global__ void __launch_bounds__(MAXT)
+k_slab_mm_wg(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __restrict__ t2, const MmArgs<T> g_, int KS,
+             int NB) {
+  typedef typename cx<T>::t C;
+  typedef typename MmV<T>::t V;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  C* kxt = reinterpret_cast<C*>(smem_raw);
+  C* hxt = kxt + 64 * KS * g_.TX;
+  const C* kyt = g_.shared ? kxt : g_.ky_t;
+  const C* hyt = g_.shared ? hxt : g_.hy_t;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, c = lane & 15, TY = g_.TY;
+  const int bl = w / TY, yt = w - bl * TY;
+  T* buf = reinterpret_cast<T*>(hxt + 64 * 4 * TK * g_.TX) + (size_t)bl * 64 * TK * max(4 * KS, 8 * TY);
+  for (int e = t; e < 64 * KS * g_.TX; e += blockDim.x) kxt[e] = g_.kx_t[e];
+  for (int e = t; e < 64 * 4 * TK * g_.TX; e += blockDim.x) hxt[e] = g_.hx_t[e];
+  const int ngrp = (g_.nb + NB - 1) / NB, items = g_.n3 * ngrp;
+  const int xcd = blockIdx.x & 7, step = (gridDim.x + 7 - xcd) >> 3;
+  const int q8 = items >> 3, r8 = items & 7;
+  const int last = (xcd + 1) * q8 + min(xcd + 1, r8);
+  const V zero = {0, 0, 0, 0};
+  for (int item = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3); item < last; item += step) {
+    const int z = item / ngrp, band = (item - z * ngrp) * NB + bl;
+    const bool live = band < g_.nb;
+    const size_t base = ((size_t)(live ? band : 0) * g_.n3 + z) * g_.nstick;
+    const C* src = t1 + base;
+    // class matrices [kx tile][k-step][class][64]
+    for (int e = yt * 64 + lane; e < 64 * TK * KS; e += 64 * TY) {
+      const int kx = 16 * ((e >> 6) / KS) + mm_perm<T>(c);
+      const T wt = (kx == 0 || kx == g_.half) ? (T)1 : (T)2;
+      const int2 se = g_.sp[e];
+      C p = src[se.x == kMmNone ? 0 : (se.x & ~kMmConj)], m = src[se.y == kMmNone ? 0 : (se.y & ~kMmConj)];
+      if (se.x & kMmConj) p.y = -p.y;
+      if (se.y & kMmConj) m.y = -m.y;
+      if (se.x == kMmNone) p = C{0, 0};
+      if (se.y == kMmNone) m = C{0, 0};
+      T* o = buf + (size_t)(e >> 6) * 256 + lane;
+      o[0] = wt * (p.x + m.x);
+      o[64] = -wt * (p.y + m.y);
+      o[128] = -wt * (p.y - m.y);
+      o[192] = -wt * (p.x - m.x);
+    }
+    __syncthreads();
+    V dee[TK], doe[TK], deo[TK], doo[TK];
+#pragma unroll
+    for (int k = 0; k < TK; k++) dee[k] = doe[k] = deo[k] = doo[k] = zero;
+#pragma unroll 2
+    for (int s = 0; s < KS; s++) {
+      const C q = kyt[(yt * KS + s) * 64 + lane];
+#pragma unroll
+      for (int k = 0; k < TK; k++) {
+        const T* a = buf + (size_t)(k * KS + s) * 256 + lane;
+        dee[k] = mm16(a[0], q.x, dee[k]);
+        doe[k] = mm16(a[64], q.x, doe[k]);
+        deo[k] = mm16(a[128], q.y, deo[k]);
+        doo[k] = mm16(a[192], q.y, doo[k]);
+      }
+    }
+    V fee[TK], foe[TK], feo[TK], foo[TK];
+#pragma unroll
+    for (int k = 0; k < TK; k++) fee[k] = foe[k] = feo[k] = foo[k] = zero;
+    const V* vp = g_.v + ((size_t)(z * TY + yt) * g_.TX * 4) * 64 + lane;
+    for (int xt = 0; xt < g_.TX; xt++) {
+      V v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = vp[(xt * 4 + i) * 64];
+      V ree = zero, roe = zero, reo = zero, roo = zero;
+#pragma unroll
+      for (int k = 0; k < TK; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (k + 1 < TK || 4 * k + i < KS) {
+            const C q = kxt[(xt * KS + 4 * k + i) * 64 + lane];
+            ree = mm16(q.x, dee[k][i], ree);
+            roe = mm16(q.y, doe[k][i], roe);
+            reo = mm16(q.x, deo[k][i], reo);
+            roo = mm16(q.y, doo[k][i], roo);
+          }
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const T e0 = ree[i], e1 = roe[i], e2 = reo[i], e3 = roo[i];
+        const T w0 = v[i][0], w1 = v[i][1], w2 = v[i][2], w3 = v[i][3];
+        ree[i] = w0 * e0 + w1 * e1 + w2 * e2 + w3 * e3;
+        roe[i] = w1 * e0 + w0 * e1 + w3 * e2 + w2 * e3;
+        reo[i] = w2 * e0 + w3 * e1 + w0 * e2 + w1 * e3;
+        roo[i] = w3 * e0 + w2 * e1 + w1 * e2 + w0 * e3;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i == 0 || 4 * xt + i < g_.XS) {
+#pragma unroll
+          for (int k = 0; k < TK; k++) {
+            const C q = hxt[(k * 4 * g_.TX + 4 * xt + i) * 64 + lane];
+            fee[k] = mm16(ree[i], q.x, fee[k]);
+            foe[k] = mm16(roe[i], q.y, foe[k]);
+            feo[k] = mm16(reo[i], q.x, feo[k]);
+            foo[k] = mm16(roo[i], q.y, foo[k]);
+          }
+        }
+    }
+    // Re (ee, oo), then Im (oe, eo): [class of the pair][kx tile][4 TY][64]
+    T* pa = buf;
+    T* pb = buf + (size_t)TK * 4 * TY * 64;
+#pragma unroll
+    for (int im = 0; im < 2; im++) {
+      __syncthreads();  // the class matrices, then the first pair, have been read
+#pragma unroll
+      for (int k = 0; k < TK; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int at = (k * 4 * TY + 4 * yt + i) * 64 + lane;
+          pa[at] = im ? foe[k][i] : fee[k][i];
+          pb[at] = im ? feo[k][i] : foo[k][i];
+        }
+      __syncthreads();
+      for (int u = yt; u < TK * TK; u += TY) {
+        const int ky = u / TK, kx = u - ky * TK;
+        V za = zero, zb = zero;
+#pragma unroll 4
+        for (int s = 0; s < g_.YS; s++) {
+          const C q = hyt[(ky * 4 * TY + s) * 64 + lane];
+          za = mm16(q.x, pa[(kx * 4 * TY + s) * 64 + lane], za);
+          zb = mm16(q.y, pb[(kx * 4 * TY + s) * 64 + lane], zb);
+        }
+        if (!live) continue;
+        T* dst = reinterpret_cast<T*>(t2 + base) + im;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (4 * ky + i < KS) {
+            const int2 e = g_.sp[(kx * KS + 4 * ky + i) * 64 + lane];
+            if (e.x >= 0 && !(e.x & kMmConj)) dst[2 * e.x] = im ? -(za[i] + zb[i]) : za[i] - zb[i];
+            if (e.y >= 0 && !(e.y & kMmConj)) dst[2 * e.y] = im ? zb[i] - za[i] : za[i] + zb[i];
+          }
+      }
+    }
+    __syncthreads();  // before the next item's class matrices
   }
 }
 

@@ -13,7 +13,7 @@ namespace pw {
 
 struct SlabMm {
   int KS = 0, TX = 0, TY = 0, XS = 0, YS = 0, half = -1, shared = 0;
-  struct Grid { int blocks = 0; } grid[2];  // resident workgroups, asked for once
+  struct Grid { int blocks = 0; } grid[2], wgrid[2][2];  // resident workgroups, asked for once
   size_t off_hx = 0, off_ky = 0, off_hy = 0;
   void* buf = nullptr;                // tables and stick entries of both precisions
   const void* tab[2];                 // [PW_F64], [PW_F32]: x and y tables
@@ -78,14 +78,14 @@ static void fill_plan(const pw_ctx* c, SlabMm* m, int kymax, const std::vector<i
   m->sp[d] = (const int2*)(dev + tab_bytes);
 }
 
-// The plan of a context, where the transform covers its sphere: at most 32
-// kx and 32 ky, and one stick of each conjugate pair of the kx = 0 column.
+// The plan of a context, where the transform covers its sphere: at most 64
+// kx and 64 ky, and one stick of each conjugate pair of the kx = 0 column.
 int mm_plan(pw_ctx* c) {
   const StickPlan& st = c->sp;
   int kymax = 0;
   for (int s = 0; s < st.nstick; s++) kymax = std::max(kymax, std::abs(kgrid(st.ky[s], c->n2)));
   const int K = std::max(st.kxmax, kymax) + 1, KS = (K + 3) / 4;
-  if (KS > 8) return PW_OK;
+  if (KS > 16) return PW_OK;
   SlabMm* m = new SlabMm();
   m->KS = KS <= 2 ? 2 : (KS == 7 ? 8 : KS);
   m->TX = (c->n1 / 2 + 16) / 16;
@@ -167,11 +167,72 @@ static mm_fn<T> mm_kernel(int KS) {
   }
 }
 
+// The workgroup kernel beyond four k-steps: threads at most (12 wavefronts
+// where 168 registers hold the tiles, else 8), bands per workgroup (the fewest
+// that reach the most resident wavefronts), LDS.  nb = 0: it does not fit.
+struct WgShape {
+  int maxt = 0, nb = 0;
+  size_t lds = 0;
+};
+template <typename T>
+static WgShape wg_shape(const SlabMm* m) {
+  WgShape w;
+  const int TK = (m->KS + 3) / 4;
+  if (sizeof(T) == 8 && TK > 2) return w;  // 384 registers of tiles a wavefront
+  w.maxt = sizeof(T) == 4 && TK <= 3 ? 768 : 512;
+  int best = 0;
+  for (int nb = 1; nb * m->TY * 64 <= w.maxt; nb++) {
+    const size_t lds = mm_wg_tables<T>(m->KS, m->TX) + nb * mm_wg_band<T>(m->KS, m->TY);
+    if (lds > 160 * 1024) break;
+    const int waves = std::min<int>((160 * 1024) / lds * nb * m->TY, w.maxt / 64 / (nb * m->TY) * nb * m->TY);
+    if (waves > best) {
+      best = waves;
+      w.nb = nb;
+      w.lds = lds;
+    }
+  }
+  return w;
+}
+template <typename T>
+using wg_fn = decltype(&k_slab_mm_wg<T, 2, 512>);
+template <typename T>
+static wg_fn<T> wg_kernel(int KS) {
+  if constexpr (sizeof(T) == 4) {
+    switch ((KS + 3) / 4) {
+      case 2: return &k_slab_mm_wg<T, 2, 768>;
+      case 3: return &k_slab_mm_wg<T, 3, 768>;
+      default: return &k_slab_mm_wg<T, 4, 512>;
+    }
+  } else {
+    return &k_slab_mm_wg<T, 2, 512>;
+  }
+}
+
+// The workgroup kernel rather than one wavefront per plane: always beyond eight
+// k-steps (the tiles of 33 columns no longer fit a wavefront), never up to four.
+// Between, us of wavefront / workgroup kernel:
+//   FP32, 128 bands: 72^3 128 / 259, 96 x 96 x 24 81 / 99, 120 x 120 x 24 106 /
+//   122; 8 bands 22 / 26, 31 / 18, 39 / 20: the workgroup where the planes are
+//   too few to fill the chip and a plane has four y tiles to split;
+//   FP64, 128 bands: 72^3 350 / 392, 96 x 54 x 24 119 / 103, 96 x 96 x 24 192 /
+//   163, 120 x 120 x 24 289 / 211; 8 bands 46 / 44, 38 / 35, 60 / 31, 86 / 38:
+//   the workgroup from four tiles on (the wavefront spills at one per SIMD).
+template <typename T>
+static bool use_wg(const pw_ctx* c, int nb) {
+  const SlabMm* m = c->mm;
+  if (m->KS <= 4) return false;
+  if (wg_shape<T>(m).nb == 0) return false;
+  if (m->KS > 8 || mm_lds<T>(m->KS, m->TX, m->TY, m->shared) > 160 * 1024) return true;
+  if (sizeof(T) == 8) return std::max(m->TX, m->TY) >= 4;
+  return m->TY >= 4 && (long)nb * c->n3 < 1024;
+}
+
 template <typename T>
 bool mm_slab_ready(const pw_ctx* c) {
   if (!c->mm) return false;
   const SlabMm* m = c->mm;
-  return mm_lds<T>(m->KS, m->TX, m->TY, m->shared) <= 160 * 1024;
+  return (m->KS <= 8 && mm_lds<T>(m->KS, m->TX, m->TY, m->shared) <= 160 * 1024) ||
+         (m->KS > 4 && wg_shape<T>(m).nb > 0);
 }
 
 template <typename T>
@@ -189,6 +250,29 @@ int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
   typedef typename cx<T>::t C;
   const SlabMm* m = c->mm;
   const int d = sizeof(T) == 8 ? PW_F64 : PW_F32;
+  if (use_wg<T>(c, nb)) {
+    const auto kwg = wg_kernel<T>(m->KS);
+    WgShape w = wg_shape<T>(m);
+    const bool few = (long)c->n3 * ((nb + w.nb - 1) / w.nb) < 256;  // one band each: more workgroups
+    if (few) {
+      w.lds -= (w.nb - 1) * mm_wg_band<T>(m->KS, m->TY);
+      w.nb = 1;
+    }
+    const int threads = 64 * w.nb * m->TY;
+    PW_TRY(ensure_lds((const void*)kwg, w.lds));
+    SlabMm::Grid& gw = c->mm->wgrid[d][few];
+    if (gw.blocks == 0) {
+      int per_cu = 0, ncu = 0;
+      PW_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kwg, threads, w.lds));
+      PW_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+      gw.blocks = std::max(1, per_cu) * std::max(8, ncu);
+    }
+    const int nitem = c->n3 * ((nb + w.nb - 1) / w.nb);
+    hipLaunchKernelGGL(kwg, dim3((unsigned)std::max(8, std::min(nitem, gw.blocks))), dim3(threads), w.lds, c->stream,
+                       (const C*)t1, (C*)t2, mm_args<T>(c, nb), m->KS, w.nb);
+    PW_HIP(hipGetLastError());
+    return PW_OK;
+  }
   const auto kern = mm_kernel<T>(m->KS);
   const size_t lds = mm_lds<T>(m->KS, m->TX, m->TY, m->shared);
   PW_TRY(ensure_lds((const void*)kern, lds));
@@ -210,7 +294,7 @@ int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
 
 // Splits of the bands that give the density about four waves per SIMD.
 int mm_density_splits(const pw_ctx* c, int nb) {
-  if (!c->mm) return 0;
+  if (!c->mm || c->mm->KS > 8) return 0;
   const long tiles = (long)c->n3 * c->mm->TX * c->mm->TY;
   return (int)std::max<long>(1, std::min<long>({(long)nb, 16, (4096 + tiles - 1) / tiles}));
 }

@@ -1,12 +1,13 @@
 """The xy slab transform on matrix cores, at the edges of its 16-row tiles:
-quarter planes of 13, 16, 17, 23..28, 31, 33, 37 and 49 rows, 2 to 8 k-steps
-per axis (one and two tiles of columns), odd lengths, unequal axes, one band
-and ragged band groups, against the oracle; and a sphere that stores the other
-half of its kx = 0 column.
+quarter planes of 13, 16, 17, 23..28, 31, 33, 37, 49 and up to 113 rows, 2 to
+15 k-steps per axis (one to four tiles of columns), odd lengths, unequal axes,
+one band and ragged band groups, one wavefront and one workgroup per plane,
+against the oracle; and a sphere that stores the other half of its kx = 0
+column.
 
 Tolerance: every output passes four chained sums whose inner lengths add up to
-at most 2 (32 + n / 2) <= 160 terms, in each of which a rounding is at most
-one unit of the largest partial sum: 160 eps, taken as 256 eps of max |H psi|.
+at most 2 (64 + n / 2) <= 360 terms, in each of which a rounding is at most
+one unit of the largest partial sum: 360 eps of max |H psi|.
 """
 import numpy as np
 import pytest
@@ -31,7 +32,9 @@ def _rel(a, ref):
 
 @pytest.mark.parametrize("grid,nb", [((24, 24, 24), 1), ((30, 30, 27), 5), ((32, 32, 32), 6), ((45, 50, 25), 3),
                                      ((60, 24, 32), 4), ((25, 60, 30), 7), ((60, 60, 24), 2), ((64, 64, 24), 5),
-                                     ((72, 54, 24), 3), ((72, 72, 25), 9), ((96, 96, 24), 2), ((108, 30, 24), 2)])
+                                     ((72, 54, 24), 3), ((72, 72, 25), 9), ((96, 96, 24), 2), ((108, 30, 24), 2),
+                                     ((96, 96, 12), 90), ((30, 108, 12), 3), ((135, 144, 12), 5),
+                                     ((150, 32, 10), 30), ((180, 180, 10), 2), ((225, 160, 10), 1)])
 def test_matrix_core_slab_against_oracle(grid, nb):
     import torch
     from pwdft_develop_amd.ops import Context
@@ -41,9 +44,9 @@ def test_matrix_core_slab_against_oracle(grid, nb):
     ctx = Context(prob)
     for dt, eps in ((torch.complex128, 2.0 ** -53), (torch.complex64, 2.0 ** -24)):
         got = ctx.mult_spinor(ctx.to_device(prob.psi, dt)).cpu().numpy()
-        assert _rel(got, ref) < 256 * eps
+        assert _rel(got, ref) < 360 * eps
         one = ctx.mult_spinor(ctx.to_device(prob.psi[nb - 1:], dt)).cpu().numpy()
-        assert _rel(one[0], got[nb - 1]) < 256 * eps  # (another kernel where a band alone takes one)
+        assert _rel(one[0], got[nb - 1]) < 360 * eps  # (another kernel where a band alone takes one)
     ctx.close()
 
 
