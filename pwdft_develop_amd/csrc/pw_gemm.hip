@@ -3,16 +3,16 @@
 //   TN:  C(n1 x n2) = A^T B, A: K x n1, B: K x n2, K = 2 npw long
 //        (Gram blocks Re(X^H Y), projections Re(beta^H X); blas.cpp:997-1029,
 //        eigensolver.cpp:471-515, lobpcg.cpp:227-419).  Split-K: each
-//        workgroup reduces one K chunk of one 64x64 tile into a partial
-//        buffer; a second kernel sums the partials in a fixed order, so the
-//        result is deterministic.
+//        workgroup reduces one K chunk of one tile into a partial buffer; a
+//        second kernel sums the partials in a fixed order, so the result is
+//        deterministic.
 //   NN:  Y(m x n) = alpha A(m x k) B(k x n) + beta Y  (subspace rotations,
-//        beta * W; blas.cpp:1031-1067, lobpcg.cpp:445-526), 64 x 64 tiles;
+//        beta * W; blas.cpp:1031-1067, lobpcg.cpp:445-526);
 //        the projector apply inside H Y takes an epilogue that adds H's
 //        other terms or forms a Chebyshev step.
 //
-// Both use 64x64 workgroup tiles, 4 waves of 32x32, and the 16x16x4 MFMA
-// (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).  Lane layout of the
+// Both use the 16x16x4 MFMA (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32)
+// on operands in registers, or split-BF16 products on tiles in LDS.  Lane layout of the
 // 16x16x4 MFMA: A operand lane l = (row l%16, k l/16), B operand lane l =
 // (k l/16, col l%16).  Accumulator lane l register i holds column l%16 and
 // row 4(l/16)+i for the FP32 MFMA but row 4i + l/16 for the FP64 one
@@ -50,8 +50,8 @@ constexpr int BM = 64, BN = 64, BK = 32;
 struct TnBlock {
   int i, j, split;
 };
-__device__ __forceinline__ TnBlock tn_block(int n1, int n2, int K, int kc, int tb) {
-  const int ti = (n1 + tb - 1) / tb, tj = (n2 + tb - 1) / tb, tiles = ti * tj;
+__device__ __forceinline__ TnBlock tn_block(int n1, int n2, int K, int kc, int t1, int t2) {
+  const int ti = (n1 + t1 - 1) / t1, tj = (n2 + t2 - 1) / t2, tiles = ti * tj;
   const int n = tiles * ((K + kc - 1) / kc), b = blockIdx.x;
   const int q = n >> 3, r = n & 7, x = b & 7;
   const int L = x * q + min(x, r) + (b >> 3);
@@ -59,109 +59,116 @@ __device__ __forceinline__ TnBlock tn_block(int n1, int n2, int K, int kc, int t
   return TnBlock{tile % ti, tile / ti, L / tiles};
 }
 
+// Four consecutive values of a matrix, at any element's alignment (global
+// loads and stores of 16 bytes need 4-byte alignment only).
+template <typename T> struct run4;
+template <> struct run4<double> { typedef double t __attribute__((ext_vector_type(4), aligned(8))); };
+template <> struct run4<float> { typedef float t __attribute__((ext_vector_type(4), aligned(4))); };
+
+// Both native products keep a wavefront's operands in registers, straight
+// from global memory: a 64 x 64 tile takes 64 MFMAs per 16 k (4096 cycles in
+// FP64, 2048 in FP32) for 8 loads of four values a lane, 8 KiB (4 KiB), so
+// the next 16 k arrive during the current ones from L2 with no LDS, no
+// barrier and one address step.  The k of an MFMA are any four as long as A
+// and B agree: lane group g = lane / 16 takes k = 16 q + 4 g + i for MFMA i,
+// four consecutive values where k is the contiguous dimension.  The tiles are
+// mfma(b, a) = (A B)^T: accumulator register r holds row lane % 16 (of the
+// MFMA's 16) and column acc_col.
 template <typename T>
-__device__ __forceinline__ int acc_row(int lane, int r) {
+__device__ __forceinline__ int acc_col(int lane, int r) {
   return sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r;
 }
 
-// NN products accumulate FP64 tiles transposed (mfma(b, a) = (A B)^T): the
-// 16x16x4f64 accumulator then holds, in register r, 16 consecutive rows of
-// column 4 r + lane / 16 in lanes 16 j .. 16 j + 15, so the epilogue reads
-// and writes 128-byte runs; FP32 tiles keep A B (four consecutive rows of
-// column lane % 16 per lane).  (row, column) of accumulator register r:
-__device__ __forceinline__ d4v mfma_nn(double a, double b, d4v c) { return mfma16(b, a, c); }
-__device__ __forceinline__ f4v mfma_nn(float a, float b, f4v c) { return mfma16(a, b, c); }
-template <typename T>
-__device__ __forceinline__ int nn_row(int lane, int r) {
-  return sizeof(T) == 8 ? (lane & 15) : 4 * (lane >> 4) + r;
-}
-template <typename T>
-__device__ __forceinline__ int nn_col(int lane, int r) {
-  return sizeof(T) == 8 ? 4 * r + (lane >> 4) : (lane & 15);
-}
-
-// Partial C tile of A^T B over K rows [kb, ke): P[split](n1 x n2, ld n1).
-// TM = 1: 64 x 64 tile, each wave 32 x 32; TM = 2: 128 x 128 tile, each wave
-// 64 x 64 (twice the flops per loaded byte, for large outputs).
-// Software-pipelined: the next K chunk is loaded into registers while the
-// MFMAs run on the current one in LDS (dynamic LDS: 2 x 64 TM x (BK + 1)).
-// Chunk loads are column runs: load q of wave w reads column 16 TM w + 2 q +
-// lane/32, rows lane%32 (one 32-row segment per half wave), for A and for B.
-template <typename T, int TM>
-__global__ void __launch_bounds__(256)
+// Partial C tile of A^T B over K rows [kb, ke): P[split](n1 x n2, ld n1), a
+// 16 NI x 16 NJ tile per workgroup whose four wavefronts take a quarter of
+// the rows each and meet in LDS (4 NI NJ KiB a wavefront in FP64, half in
+// FP32), summed in the order of the rows: a quarter of the partials that
+// tiles split over the wavefronts write.
+template <typename T, int NI, int NJ>
+__global__ void __launch_bounds__(256, (int)sizeof(T) * NI * NJ > 96 ? 1 : 2)
 k_gemm_tn_partial(const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, int K, int n1, int n2,
                   int kc, T* __restrict__ P, const T* const* __restrict__ Ab, const T* const* __restrict__ Bb,
                   long sP) {
   typedef typename acc4<T>::t V;
+  typedef typename run4<T>::t R;
   if (Ab) {  // product blockIdx.y of a batch: operands from the pointer tables
     A = Ab[blockIdx.y];
     B = Bb[blockIdx.y];
     P += blockIdx.y * sP;
   }
-  constexpr int TB = BM * TM, NQ = 8 * TM, NA = 2 * TM;
   extern __shared__ __align__(16) unsigned char gemm_smem[];
-  T (*As)[BK + 1] = reinterpret_cast<T (*)[BK + 1]>(gemm_smem);
-  T (*Bs)[BK + 1] = As + TB;
-  const TnBlock tb = tn_block(n1, n2, K, kc, TB);
-  const int i0 = tb.i * TB, j0 = tb.j * TB, split = tb.split;
-  const int kb = split * kc, ke = min(K, kb + kc);
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = (w & 1) * 32 * TM, wj = (w >> 1) * 32 * TM;
-  V acc[NA][NA];
+  V* const red = (V*)gemm_smem;  // [4][NI * NJ][64]
+  const TnBlock tb = tn_block(n1, n2, K, kc, 16 * NI, 16 * NJ);
+  const int i0 = tb.i * 16 * NI, j0 = tb.j * 16 * NJ, split = tb.split;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int kw = kc >> 2, kb = min(K, split * kc + w * kw), ke = min(K, kb + kw);
+  V acc[NI][NJ];
 #pragma unroll
-  for (int a = 0; a < NA; a++)
+  for (int a = 0; a < NI; a++)
 #pragma unroll
-    for (int b = 0; b < NA; b++) acc[a][b] = V{0, 0, 0, 0};
-  const int lr = lane & 31, lcol = 16 * TM * w + (lane >> 5);  // column of load q: lcol + 2 q
-  T ra[NQ], rb[NQ];
-  // unconditional loads at clamped indices, the zero fill outside the
-  // operands at the LDS store (a select on a loaded value makes the
-  // compiler wait for the load where it is issued)
-  auto load = [&](int k0) {
-    const int r = min(k0 + lr, ke - 1);
+    for (int b = 0; b < NJ; b++) acc[a][b] = V{0, 0, 0, 0};
+  const T *pa[NI], *pb[NJ];  // columns beyond the matrix repeat its last one
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const int ci = min(i0 + lcol + 2 * q, n1 - 1), cj = min(j0 + lcol + 2 * q, n2 - 1);
-      ra[q] = A[(size_t)ci * lda + r];
-      rb[q] = B[(size_t)cj * ldb + r];
-    }
+  for (int a = 0; a < NI; a++) pa[a] = A + (size_t)min(i0 + 16 * a + c, n1 - 1) * lda;
+#pragma unroll
+  for (int b = 0; b < NJ; b++) pb[b] = B + (size_t)min(j0 + 16 * b + c, n2 - 1) * ldb;
+  auto mm = [&](const R (&ra)[NI], const R (&rb)[NJ]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int a = 0; a < NI; a++)
+#pragma unroll
+        for (int b = 0; b < NJ; b++) acc[a][b] = mfma16(rb[b][i], ra[a][i], acc[a][b]);
   };
-  load(kb);
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    const bool okr = k0 + lr < ke;
+  const int nq = (ke - kb) >> 4;  // full chunks of 16 rows
+  if (nq > 0) {
+    auto load = [&](R (&ra)[NI], R (&rb)[NJ], int q) {
+      const int k = kb + 16 * min(q, nq - 1) + 4 * g;  // (the chunk past the end: read and dropped)
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      As[lcol + 2 * q][lr] = (okr && i0 + lcol + 2 * q < n1) ? ra[q] : (T)0;
-      Bs[lcol + 2 * q][lr] = (okr && j0 + lcol + 2 * q < n2) ? rb[q] : (T)0;
+      for (int a = 0; a < NI; a++) ra[a] = *(const R*)(pa[a] + k);
+#pragma unroll
+      for (int b = 0; b < NJ; b++) rb[b] = *(const R*)(pb[b] + k);
+    };
+    R a0[NI], b0[NJ], a1[NI], b1[NJ];
+    load(a0, b0, 0);
+    int q = 0;
+    for (; q + 2 <= nq; q += 2) {
+      load(a1, b1, q + 1);
+      mm(a0, b0);
+      load(a0, b0, q + 2);
+      mm(a1, b1);
     }
-    lds_barrier();
-    if (k0 + BK < ke) load(k0 + BK);  // in flight during the MFMAs below and the barrier after them
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T av[NA], bv[NA];
-#pragma unroll
-      for (int a = 0; a < NA; a++) av[a] = As[wi + a * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int b = 0; b < NA; b++) bv[b] = Bs[wj + b * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int a = 0; a < NA; a++)
-#pragma unroll
-        for (int b = 0; b < NA; b++) acc[a][b] = mfma16(av[a], bv[b], acc[a][b]);
-    }
-    lds_barrier();
+    if (q < nq) mm(a0, b0);
   }
-  T* Ps = P + (size_t)split * n1 * n2;
+  if (kb + 16 * nq < ke) {  // the last, incomplete chunk
+    R ra[NI], rb[NJ];
 #pragma unroll
-  for (int a = 0; a < NA; a++)
+    for (int i = 0; i < 4; i++) {
+      const int k = kb + 16 * nq + 4 * g + i, kk = min(k, ke - 1);
 #pragma unroll
-    for (int b = 0; b < NA; b++) {
-      const int col = j0 + wj + b * 16 + (lane & 15);
+      for (int a = 0; a < NI; a++) ra[a][i] = k < ke ? pa[a][kk] : (T)0;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = i0 + wi + a * 16 + acc_row<T>(lane, r);
-        if (row < n1 && col < n2) Ps[row + (size_t)n1 * col] = acc[a][b][r];
-      }
+      for (int b = 0; b < NJ; b++) rb[b][i] = k < ke ? pb[b][kk] : (T)0;
     }
+    mm(ra, rb);
+  }
+#pragma unroll
+  for (int a = 0; a < NI; a++)
+#pragma unroll
+    for (int b = 0; b < NJ; b++) red[((w * NI + a) * NJ + b) * 64 + lane] = acc[a][b];
+  __syncthreads();
+  T* Ps = P + (size_t)split * n1 * n2;
+  for (int e = w; e < NI * NJ; e += 4) {
+    V s = red[e * 64 + lane];
+#pragma unroll
+    for (int v = 1; v < 4; v++) s += red[(v * NI * NJ + e) * 64 + lane];
+    const int row = i0 + 16 * (e / NJ) + c;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int col = j0 + 16 * (e % NJ) + acc_col<T>(lane, r);
+      if (row < n1 && col < n2) Ps[row + (size_t)n1 * col] = s[r];
+    }
+  }
 }
 
 // ---- split BF16 products (FP32 data, FP32 accumulation) ----
@@ -235,9 +242,12 @@ constexpr int BKP = 40;  // LDS row stride of the bf16 tiles (80 bytes: 16-byte 
 __device__ constexpr int kSplitPairA[6] = {2, 0, 1, 1, 0, 0};
 __device__ constexpr int kSplitPairB[6] = {0, 2, 1, 0, 1, 0};
 
-// k_gemm_tn_partial with FP32 inputs split into NS BF16 terms: the same
-// tiles, loads and split-K partials; each 32-row K chunk is one 16x16x32
-// product per kept pairing of terms instead of eight 16x16x4 FP32 products.
+// A^T B partials with FP32 inputs split into NS BF16 terms.  TM = 1: 64 x 64
+// tile, each wave 32 x 32; TM = 2: 128 x 128 tile, each wave 64 x 64 (twice
+// the flops per loaded byte, for large outputs).  The next 32-row K chunk is
+// loaded into registers while the MFMAs run on the current one in LDS; a
+// chunk is one 16x16x32 product per kept pairing of terms instead of eight
+// 16x16x4 FP32 products.
 template <int TM, int NS>
 __global__ void __launch_bounds__(256)
 k_gemm_tn_partial_bf(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, int K, int n1,
@@ -246,7 +256,7 @@ k_gemm_tn_partial_bf(const float* __restrict__ A, int lda, const float* __restri
   extern __shared__ __align__(16) unsigned char gemm_smem[];
   unsigned short* As = reinterpret_cast<unsigned short*>(gemm_smem);  // NS term tiles of A, then of B
   unsigned short* Bs = As + NS * TB * BKP;
-  const TnBlock tb = tn_block(n1, n2, K, kc, TB);
+  const TnBlock tb = tn_block(n1, n2, K, kc, TB, TB);
   const int i0 = tb.i * TB, j0 = tb.j * TB, split = tb.split;
   const int kb = split * kc, ke = min(K, kb + kc);
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -338,14 +348,14 @@ k_gemm_tn_partial_bf(const float* __restrict__ A, int lda, const float* __restri
       const int col = j0 + wj + b * 16 + (lane & 15);
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int row = i0 + wi + a * 16 + acc_row<float>(lane, r);
+        const int row = i0 + wi + a * 16 + acc_col<float>(lane, r);
         if (row < n1 && col < n2) Ps[row + (size_t)n1 * col] = acc[a][b][r];
       }
     }
 }
 
 // C[i + ldc j] = rowscale[i] * sum_s P[s][i + n1 j] (+ beta C), rowscale may
-// be null.  The partials are summed in split order (deterministic), eight
+// be null.  The partials are summed in split order (deterministic), 16
 // loads in flight at a time.
 template <typename T>
 __global__ void k_gemm_tn_reduce(const T* __restrict__ P, int nsplit, int n1, int n2, T* __restrict__ C, int ldc,
@@ -358,12 +368,12 @@ __global__ void k_gemm_tn_reduce(const T* __restrict__ P, int nsplit, int n1, in
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
     const int i = (int)(e % n1), j = (int)(e / n1);
     T s = 0;
-    for (int q0 = 0; q0 < nsplit; q0 += 8) {
-      T v[8];
+    for (int q0 = 0; q0 < nsplit; q0 += 16) {
+      T v[16];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = (q0 + u < nsplit) ? P[(size_t)(q0 + u) * total + e] : (T)0;
+      for (int u = 0; u < 16; u++) v[u] = (q0 + u < nsplit) ? P[(size_t)(q0 + u) * total + e] : (T)0;
 #pragma unroll
-      for (int u = 0; u < 8; u++) s += v[u];
+      for (int u = 0; u < 16; u++) s += v[u];
     }
     if (rowscale) s *= rowscale[i];
     T* c = C + i + (size_t)ldc * j;
@@ -380,78 +390,6 @@ __device__ __forceinline__ void nn_tile_origin(int m, int n, int& i0, int& j0) {
   const int item = xcd_item(blockIdx.x, ti * tj), i = item / tj;
   i0 = i * BM;
   j0 = (item - i * tj) * BN;
-}
-
-// Y = alpha A B + beta Y; A m x k (lda), B k x n (ldb), Y m x n (ldy).
-// Pipelined like k_gemm_tn_partial.  A chunk (64 rows x 32 k): load q of
-// wave w reads k = 8 w + q, rows lane (one 64-row run per wave); B chunk
-// (32 k x 64 columns): column 16 w + 2 q + lane/32, k lane%32.
-template <typename T>
-__global__ void __launch_bounds__(256)
-k_gemm_nn(const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, T* __restrict__ Y, int ldy, int m,
-          int n, int k, T alpha, T beta) {
-  typedef typename acc4<T>::t V;
-  __shared__ T As[BK][BM + 1];
-  __shared__ T Bs[BN][BK + 1];
-  int i0, j0;
-  nn_tile_origin(m, n, i0, j0);
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = (w & 1) * 32, wj = (w >> 1) * 32;
-  V acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++) acc[a][b] = V{0, 0, 0, 0};
-  const int bk = lane & 31, bcol = 16 * w + (lane >> 5);
-  const int ar = i0 + lane;
-  T ra[8], rb[8];
-  // unconditional loads at clamped indices, the zero fill at the LDS store
-  auto load = [&](int k0) {
-    const int arc = min(ar, m - 1);
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int kk = min(k0 + 8 * w + q, k - 1);
-      ra[q] = A[(size_t)kk * lda + arc];
-      const int cj = min(j0 + bcol + 2 * q, n - 1), kq = min(k0 + bk, k - 1);
-      rb[q] = B[(size_t)cj * ldb + kq];
-    }
-  };
-  load(0);
-  for (int k0 = 0; k0 < k; k0 += BK) {
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      As[8 * w + q][lane] = (ar < m && k0 + 8 * w + q < k) ? ra[q] : (T)0;
-      Bs[bcol + 2 * q][bk] = (j0 + bcol + 2 * q < n && k0 + bk < k) ? rb[q] : (T)0;
-    }
-    lds_barrier();
-    if (k0 + BK < k) load(k0 + BK);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; a++) av[a] = As[kk + (lane >> 4)][wi + a * 16 + (lane & 15)];
-#pragma unroll
-      for (int b = 0; b < 2; b++) bv[b] = Bs[wj + b * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = mfma_nn(av[a], bv[b], acc[a][b]);
-    }
-    lds_barrier();
-  }
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = i0 + wi + a * 16 + nn_row<T>(lane, r), col = j0 + wj + b * 16 + nn_col<T>(lane, r);
-        if (row < m && col < n) {
-          T* y = Y + row + (size_t)ldy * col;
-          const T v = alpha * acc[a][b][r];
-          *y = (beta == (T)0) ? v : v + beta * *y;
-        }
-      }
 }
 
 // Epilogue of the projector apply inside H Y (acc = (beta w) W for one
@@ -486,6 +424,23 @@ __device__ __forceinline__ void nn_epilogue(const NnEpilogue<T>& ep, size_t e, T
   } else {
     const T v = ep.alpha * acc;
     ep.out[e] = ep.beta == (T)0 ? v : v + ep.beta * ep.H[e];
+  }
+}
+
+// The same for four consecutive rows.
+template <typename T, bool kCheb>
+__device__ __forceinline__ void nn_epilogue4(const NnEpilogue<T>& ep, size_t e, typename run4<T>::t acc) {
+  typedef typename run4<T>::t R;
+  if constexpr (kCheb) {
+    const R h = *(const R*)(ep.H + e) + acc;
+    const T c = ep.coef[3 * ep.step], s1 = ep.coef[3 * ep.step + 1], s2 = ep.coef[3 * ep.step + 2];
+    R v = (h - c * *(const R*)(ep.Yc + e)) * s1;
+    if (ep.Yp) v -= s2 * *(const R*)(ep.Yp + e);
+    *(R*)(ep.out + e) = v;
+  } else {
+    R v = ep.alpha * acc;
+    if (ep.beta != (T)0) v += ep.beta * *(const R*)(ep.H + e);
+    *(R*)(ep.out + e) = v;
   }
 }
 
@@ -565,7 +520,7 @@ k_gemm_nn_bf(const float* __restrict__ A, int lda, const float* __restrict__ B, 
     for (int b = 0; b < 2; b++)
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        Ct[(wj + b * 16 + (lane & 15)) * 65 + wi + a * 16 + acc_row<float>(lane, i)] = acc[a][b][i];
+        Ct[(wj + b * 16 + (lane & 15)) * 65 + wi + a * 16 + acc_col<float>(lane, i)] = acc[a][b][i];
   __syncthreads();
   const int col = j0 + (t >> 2), r0 = 16 * (t & 3);
   if (col < n) {
@@ -728,70 +683,87 @@ k_gemm_nn_pre(const unsigned short* __restrict__ Ab, const unsigned short* __res
   }
 }
 
-// The same product on v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32
-// (pipelined like k_gemm_nn), with the same epilogue.
-template <typename T, bool kCheb>
-__global__ void __launch_bounds__(256)
+// The same product in the operands' own precision: a wavefront takes 64 rows
+// x 16 NJ columns, the four of a workgroup consecutive (row, column) tiles,
+// so that where n > 16 NJ they read the same rows of A.  MFMA row c of row
+// tile t is row 4 c + t: one load of four consecutive rows per lane and k
+// feeds four MFMAs, and a lane's results are four consecutive rows too.  The
+// last rows' lanes start early enough to stay inside the matrix and write
+// only what no other lane does.
+template <typename T, int NJ, bool kCheb>
+__global__ void __launch_bounds__(256, 2)
 k_gemm_nn_ep(const T* __restrict__ A, int lda, const T* __restrict__ B, int ldb, int m, int n, int k,
              NnEpilogue<T> ep) {
   typedef typename acc4<T>::t V;
-  __shared__ T As[BK][BM + 1];
-  __shared__ T Bs[BN][BK + 1];
-  int i0, j0;
-  nn_tile_origin(m, n, i0, j0);
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = (w & 1) * 32, wj = (w >> 1) * 32;
-  V acc[2][2];
+  typedef typename run4<T>::t R;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int ti = (m + 63) / 64, tj = (n + 16 * NJ - 1) / (16 * NJ);
+  const int item = 4 * xcd_item(blockIdx.x, gridDim.x) + w;
+  if (item >= ti * tj) return;
+  const int i = item / tj, j0 = 16 * NJ * (item - i * tj);
+  const int r0 = 64 * i + 4 * c, rb0 = max(0, min(r0, m - 4));
+  V acc[4][NJ];
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int t = 0; t < 4; t++)
 #pragma unroll
-    for (int b = 0; b < 2; b++) acc[a][b] = V{0, 0, 0, 0};
-  const int bk = lane & 31, bcol = 16 * w + (lane >> 5);
-  const int ar = i0 + lane;
-  T ra[8], rb[8];
-  // unconditional loads at clamped indices, the zero fill at the LDS store
-  auto load = [&](int k0) {
-    const int arc = min(ar, m - 1);
+    for (int b = 0; b < NJ; b++) acc[t][b] = V{0, 0, 0, 0};
+  const T *pa = A + rb0, *pb[NJ];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int kk = min(k0 + 8 * w + q, k - 1);
-      ra[q] = A[(size_t)kk * lda + arc];
-      const int cj = min(j0 + bcol + 2 * q, n - 1), kq = min(k0 + bk, k - 1);
-      rb[q] = B[(size_t)cj * ldb + kq];
-    }
+  for (int b = 0; b < NJ; b++) pb[b] = B + (size_t)min(j0 + 16 * b + c, n - 1) * ldb;
+  auto mm = [&](const R (&ra)[4], const R (&rb)[NJ]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int b = 0; b < NJ; b++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc[t][b] = mfma16(rb[b][q], ra[q][t], acc[t][b]);
   };
-  load(0);
-  for (int k0 = 0; k0 < k; k0 += BK) {
+  const int nq = m >= 4 ? k >> 4 : 0;
+  if (nq > 0) {
+    auto load = [&](R (&ra)[4], R (&rb)[NJ], int q) {
+      const int k0 = 16 * min(q, nq - 1) + 4 * g;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      As[8 * w + q][lane] = (ar < m && k0 + 8 * w + q < k) ? ra[q] : (T)0;
-      Bs[bcol + 2 * q][bk] = (j0 + bcol + 2 * q < n && k0 + bk < k) ? rb[q] : (T)0;
+      for (int u = 0; u < 4; u++) ra[u] = *(const R*)(pa + (size_t)(k0 + u) * lda);
+#pragma unroll
+      for (int b = 0; b < NJ; b++) rb[b] = *(const R*)(pb[b] + k0);
+    };
+    R a0[4], b0[NJ], a1[4], b1[NJ];
+    load(a0, b0, 0);
+    int q = 0;
+    for (; q + 2 <= nq; q += 2) {
+      load(a1, b1, q + 1);
+      mm(a0, b0);
+      load(a0, b0, q + 2);
+      mm(a1, b1);
     }
-    lds_barrier();
-    if (k0 + BK < k) load(k0 + BK);
+    if (q < nq) mm(a0, b0);
+  }
+  for (int k1 = 16 * nq; k1 < k; k1 += 16) {  // the last, incomplete chunk (all of them where m < 4)
+    R ra[4], rb[NJ];
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T av[2], bv[2];
+    for (int u = 0; u < 4; u++) {
+      const int kq = k1 + 4 * g + u, kk = min(kq, k - 1);
 #pragma unroll
-      for (int a = 0; a < 2; a++) av[a] = As[kk + (lane >> 4)][wi + a * 16 + (lane & 15)];
+      for (int t = 0; t < 4; t++) ra[u][t] = kq < k ? A[(size_t)kk * lda + min(rb0 + t, m - 1)] : (T)0;
 #pragma unroll
-      for (int b = 0; b < 2; b++) bv[b] = Bs[wj + b * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-      for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = mfma_nn(av[a], bv[b], acc[a][b]);
+      for (int b = 0; b < NJ; b++) rb[b][u] = kq < k ? pb[b][kk] : (T)0;
     }
-    lds_barrier();
+    mm(ra, rb);
   }
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int b = 0; b < NJ; b++)
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int r = 0; r < 4; r++) {
+      const int col = j0 + 16 * b + acc_col<T>(lane, r);
+      if (col >= n || r0 >= m) continue;
+      const size_t e = (size_t)col * ep.ld + rb0;
+      if (rb0 == r0 && m >= 4)
+        nn_epilogue4<T, kCheb>(ep, e, R{acc[0][b][r], acc[1][b][r], acc[2][b][r], acc[3][b][r]});
+      else
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = i0 + wi + a * 16 + nn_row<T>(lane, r), col = j0 + wj + b * 16 + nn_col<T>(lane, r);
-        if (row < m && col < n) nn_epilogue<T, kCheb>(ep, (size_t)col * ep.ld + row, acc[a][b][r]);
-      }
+        for (int t = 0; t < 4; t++)
+          if (rb0 + t >= r0 && rb0 + t < m) nn_epilogue<T, kCheb>(ep, e + t, acc[t][b][r]);
+    }
 }
 
 // Elementwise form of the epilogue (no projectors: acc = 0).
@@ -898,6 +870,57 @@ static int grow_gemm_ws(pw_ctx* c, size_t need) {
   return PW_OK;
 }
 
+// 16-wide tiles of a workgroup along a dimension of n: as few workgroups of
+// up to most tiles as cover it, evenly filled (77 columns are two of 48, not
+// of 64).
+static int tiles16(int n, int most) {
+  const int t = (n + 15) / 16, nb = (t + most - 1) / most;
+  return std::max(2, (t + nb - 1) / nb);
+}
+
+template <typename T>
+using TnKernel = void (*)(const T*, int, const T*, int, int, int, int, int, T*, const T* const*, const T* const*, long);
+
+template <typename T>
+static TnKernel<T> tn_kernel(int ni, int nj) {
+  static const TnKernel<T> k[3][3] = {
+      {k_gemm_tn_partial<T, 2, 2>, k_gemm_tn_partial<T, 2, 3>, k_gemm_tn_partial<T, 2, 4>},
+      {k_gemm_tn_partial<T, 3, 2>, k_gemm_tn_partial<T, 3, 3>, k_gemm_tn_partial<T, 3, 4>},
+      {k_gemm_tn_partial<T, 4, 2>, k_gemm_tn_partial<T, 4, 3>, k_gemm_tn_partial<T, 4, 4>}};
+  return k[ni - 2][nj - 2];
+}
+
+// Tiles, splits and rows per split of nbatch products K x n1 x n2: as many
+// workgroups as the CUs hold (cap: aimed at instead), so that all of them run
+// at once; at least 128 rows a split, and at most 64 splits, whose partials
+// the reduction reads one after the other.  Tiles of up to 64 x 64, or 32 x 32
+// where those leave most CUs without work.  us, FP64: 26268 x 256 x 256 with
+// 64 x 64 tiles 43.3 (256 workgroups; 512: 53.4), 32 x 64 46.5, 48 x 48 55.5,
+// 32 x 32 57.0 (through LDS, 64 x 64 split over the wavefronts: 58.9); 15100 x
+// 76 x 77 7.9, 8.8 with 32 x 48 tiles; 5700 x 48 x 64 8.2, 5.0 with 32 x 32.
+// FP32, 152400 x 256 x 256: 195 with two 64 x 64 workgroups a CU, 235 with one,
+// 217 with 32 x 64, 274 with 32 x 32 (through LDS: 240).
+struct TnShape {
+  int ni, nj, tiles, nsplit, kc;
+  size_t lds;
+};
+template <typename T>
+static TnShape tn_shape(int K, int n1, int n2, int nbatch, int cap, int max_split) {
+  TnShape s;
+  const int rows = std::min(64, (K + 127) / 128);
+  const int most = (long)((n1 + 63) / 64) * ((n2 + 63) / 64) * nbatch * rows >= 192 ? 4 : 2;
+  s.ni = tiles16(n1, most);
+  s.nj = tiles16(n2, most);
+  s.lds = 4 * sizeof(T) * 256 * (size_t)s.ni * s.nj;
+  s.tiles = ((n1 + 16 * s.ni - 1) / (16 * s.ni)) * ((n2 + 16 * s.nj - 1) / (16 * s.nj));
+  if (cap <= 0) cap = sizeof(T) * s.ni * s.nj > 96 ? 256 : 512;
+  const long all = (long)s.tiles * nbatch;
+  s.nsplit = (int)std::max(1L, std::min({cap / all, (long)(K + 127) / 128, 64L, (long)max_split}));
+  s.kc = ((K + s.nsplit - 1) / s.nsplit + 63) / 64 * 64;
+  s.nsplit = std::max(1, (K + s.kc - 1) / s.kc);
+  return s;
+}
+
 // ws == null: the partials go to the context's buffer (grown on demand);
 // else to ws (ws_bytes long), with fewer K splits when the usual count does
 // not fit and PW_ERR_UNSUPPORTED when not even one split does.
@@ -920,68 +943,50 @@ int gemm_tn_ws(pw_ctx* c, int K, int n1, int n2, const T* A, int lda, const T* B
     PW_HIP(hipGetLastError());
     return PW_OK;
   }
-  // outputs of 256 or more 64 x 64 tiles (1024 x 1024 and up) take
-  // 128 x 128 tiles
   const pw_ctx::Plan& pl = c->plan[sizeof(T) == 8 ? PW_F64 : PW_F32];
-  const int tm = pl.tn_tm > 0 ? pl.tn_tm : (((n1 + BM - 1) / BM) * ((n2 + BN - 1) / BN) >= 256 ? 2 : 1);
-  const int ti = (n1 + BM * tm - 1) / (BM * tm), tj = (n2 + BN * tm - 1) / (BN * tm);
-  const int tiles = ti * tj;
-  // about 1024 partial workgroups, but at most 256 K-splits for one or two
-  // output tiles (the sb x sb Gram blocks of PPCG over a long K): the
-  // reduction then reads 256 partials per entry, not ~1000
-  const int cap = pl.tn_cap > 0 ? pl.tn_cap : (tiles <= 2 ? 256 : 1024);
-  int nsplit = std::max(1, std::min((cap + tiles - 1) / tiles, (K + 255) / 256));
   const size_t per_split = sizeof(T) * (size_t)n1 * n2;
-  if (ws) {
-    if (per_split > ws_bytes)
-      return fail(PW_ERR_UNSUPPORTED, "a %d x %d projection exceeds the %zu-byte scratch", n1, n2, ws_bytes);
-    nsplit = (int)std::min<size_t>(nsplit, ws_bytes / per_split);
-  }
-  int kc = (K + nsplit - 1) / nsplit;
-  kc = (kc + BK - 1) / BK * BK;
-  nsplit = (K + kc - 1) / kc;
-  const size_t need = per_split * nsplit;
-  if (!ws) PW_TRY(grow_gemm_ws(c, need));
-  T* P = (T*)(ws ? ws : c->d_gemm_ws);
+  if (ws && per_split > ws_bytes)
+    return fail(PW_ERR_UNSUPPORTED, "a %d x %d projection exceeds the %zu-byte scratch", n1, n2, ws_bytes);
+  const int max_split = ws ? (int)std::min<size_t>(ws_bytes / per_split, 1 << 20) : 1 << 20;
+  const long total = (long)n1 * n2;
+  const int g = (int)std::min<long>((total + 255) / 256, 4096);
+  T* P = nullptr;
+  int nsplit = 0;
+  bool done = false;
   if constexpr (sizeof(T) == 4) {
     // the split kernels load float pairs: K, lda and ldb even
     if ((split == 2 || split == 3) && !(K & 1) && !(lda & 1) && !(ldb & 1)) {
+      // outputs of 256 or more 64 x 64 tiles (1024 x 1024 and up) take
+      // 128 x 128 tiles
+      const int tm = pl.tn_tm > 0 ? pl.tn_tm : (((n1 + BM - 1) / BM) * ((n2 + BN - 1) / BN) >= 256 ? 2 : 1);
+      const int tiles = ((n1 + BM * tm - 1) / (BM * tm)) * ((n2 + BN * tm - 1) / (BN * tm));
+      // about 1024 partial workgroups, but at most 256 K-splits for one or two
+      // output tiles: the reduction then reads 256 partials per entry, not
+      // ~1000
+      const int cap = pl.tn_cap > 0 ? pl.tn_cap : (tiles <= 2 ? 256 : 1024);
+      nsplit = std::max(1, std::min({(cap + tiles - 1) / tiles, (K + 255) / 256, max_split}));
+      const int kc = ((K + nsplit - 1) / nsplit + BK - 1) / BK * BK;
+      nsplit = (K + kc - 1) / kc;
+      if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
+      P = (T*)(ws ? ws : c->d_gemm_ws);
       const size_t ldsb = sizeof(unsigned short) * 2 * split * (size_t)(BM * tm) * BKP;
-      const dim3 gp(ti * tj * nsplit);
-      if (split == 3 && tm == 2) {
-        PW_TRY(ensure_lds((const void*)k_gemm_tn_partial_bf<2, 3>, ldsb));
-        hipLaunchKernelGGL((k_gemm_tn_partial_bf<2, 3>), gp, dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2,
-                           kc, P);
-      } else if (split == 3) {
-        hipLaunchKernelGGL((k_gemm_tn_partial_bf<1, 3>), gp, dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2,
-                           kc, P);
-      } else if (tm == 2) {
-        PW_TRY(ensure_lds((const void*)k_gemm_tn_partial_bf<2, 2>, ldsb));
-        hipLaunchKernelGGL((k_gemm_tn_partial_bf<2, 2>), gp, dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2,
-                           kc, P);
-      } else {
-        hipLaunchKernelGGL((k_gemm_tn_partial_bf<1, 2>), gp, dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2,
-                           kc, P);
-      }
-      const long total = (long)n1 * n2;
-      const int g = (int)std::min<long>((total + 255) / 256, 4096);
-      hipLaunchKernelGGL(k_gemm_tn_reduce<T>, dim3(g), dim3(256), 0, c->stream, (const T*)P, nsplit, n1, n2, C, ldc,
-                         rowscale, beta, (T* const*)nullptr, 0L);
-      PW_HIP(hipGetLastError());
-      return PW_OK;
+      const auto kern = split == 3 ? (tm == 2 ? k_gemm_tn_partial_bf<2, 3> : k_gemm_tn_partial_bf<1, 3>)
+                                   : (tm == 2 ? k_gemm_tn_partial_bf<2, 2> : k_gemm_tn_partial_bf<1, 2>);
+      PW_TRY(ensure_lds((const void*)kern, ldsb));
+      hipLaunchKernelGGL(kern, dim3(tiles * nsplit), dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2, kc, P);
+      done = true;
     }
   }
-  const size_t lds = sizeof(T) * 2 * (size_t)(BM * tm) * (BK + 1);
-  if (tm == 2) {
-    PW_TRY(ensure_lds((const void*)k_gemm_tn_partial<T, 2>, lds));
-    hipLaunchKernelGGL((k_gemm_tn_partial<T, 2>), dim3(ti * tj * nsplit), dim3(256), lds, c->stream, A, lda, B, ldb,
-                       K, n1, n2, kc, P, (const T* const*)nullptr, (const T* const*)nullptr, 0L);
-  } else {
-    hipLaunchKernelGGL((k_gemm_tn_partial<T, 1>), dim3(ti * tj * nsplit), dim3(256), lds, c->stream, A, lda, B, ldb,
-                       K, n1, n2, kc, P, (const T* const*)nullptr, (const T* const*)nullptr, 0L);
+  if (!done) {
+    const TnShape s = tn_shape<T>(K, n1, n2, 1, pl.tn_cap, max_split);
+    nsplit = s.nsplit;
+    if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
+    P = (T*)(ws ? ws : c->d_gemm_ws);
+    const auto kern = tn_kernel<T>(s.ni, s.nj);
+    PW_TRY(ensure_lds((const void*)kern, s.lds));
+    hipLaunchKernelGGL(kern, dim3(s.tiles * nsplit), dim3(256), s.lds, c->stream, A, lda, B, ldb, K, n1, n2, s.kc, P,
+                       (const T* const*)nullptr, (const T* const*)nullptr, 0L);
   }
-  const long total = (long)n1 * n2;
-  const int g = (int)std::min<long>((total + 255) / 256, 4096);
   hipLaunchKernelGGL(k_gemm_tn_reduce<T>, dim3(g), dim3(256), 0, c->stream, (const T*)P, nsplit, n1, n2, C, ldc,
                      rowscale, beta, (T* const*)nullptr, 0L);
   PW_HIP(hipGetLastError());
@@ -994,6 +999,21 @@ int gemm_tn(pw_ctx* c, int K, int n1, int n2, const T* A, int lda, const T* B, i
   return gemm_tn_ws<T>(c, K, n1, n2, A, lda, B, ldb, C, ldc, rowscale, beta, split, nullptr, 0);
 }
 
+// 16 columns a wavefront where that takes fewer rounds of the chip's 1024 SIMDs
+// than 32 (few rows, or the ragged end of n), else 32.  us with 16 / 32 / 48 /
+// 64 columns: FP64 26268 x 256 x 256 50.6 / 47.2 / 77.2 / 55.2 (through LDS:
+// 65.8), 7550 x 77 x 76 12.5 / 21.6 / 29.1 / 36.9; FP32 152400 x 256 x 256
+// 269 / 235 / 235 / 239 (through LDS: 302).
+template <typename T, bool kCheb>
+static void launch_nn(pw_ctx* c, const T* A, int lda, const T* B, int ldb, int m, int n, int k,
+                      const NnEpilogue<T>& ep) {
+  const int ti = (m + 63) / 64, it1 = ti * ((n + 15) / 16), it2 = ti * ((n + 31) / 32);
+  const bool one = (it1 + 1023) / 1024 < 2 * ((it2 + 1023) / 1024);
+  const int items = one ? it1 : it2;
+  const auto kern = one ? k_gemm_nn_ep<T, 1, kCheb> : k_gemm_nn_ep<T, 2, kCheb>;
+  hipLaunchKernelGGL(kern, dim3((items + 3) / 4), dim3(256), 0, c->stream, A, lda, B, ldb, m, n, k, ep);
+}
+
 template <typename T>
 int gemm_nn(pw_ctx* c, int m, int n, int k, T alpha, const T* A, int lda, const T* B, int ldb, T beta, T* Y,
             int ldy) {
@@ -1003,8 +1023,7 @@ int gemm_nn(pw_ctx* c, int m, int n, int k, T alpha, const T* A, int lda, const 
     PW_HIP(hipGetLastError());
     return PW_OK;
   }
-  hipLaunchKernelGGL(k_gemm_nn<T>, dim3(((m + BM - 1) / BM) * ((n + BN - 1) / BN)), dim3(256), 0, c->stream, A, lda, B,
-                     ldb, Y, ldy, m, n, k, alpha, beta);
+  launch_nn<T, false>(c, A, lda, B, ldb, m, n, k, NnEpilogue<T>{Y, nullptr, nullptr, Y, ldy, nullptr, 0, alpha, beta});
   PW_HIP(hipGetLastError());
   return PW_OK;
 }
@@ -1047,9 +1066,9 @@ int gemm_nn_ep(pw_ctx* c, int m, int n, int k, const T* A, int lda, const T* B, 
   }
   if (!done) {
     if (cheb)
-      hipLaunchKernelGGL((k_gemm_nn_ep<T, true>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, m, n, k, ep);
+      launch_nn<T, true>(c, A, lda, B, ldb, m, n, k, ep);
     else
-      hipLaunchKernelGGL((k_gemm_nn_ep<T, false>), grid, dim3(256), 0, c->stream, A, lda, B, ldb, m, n, k, ep);
+      launch_nn<T, false>(c, A, lda, B, ldb, m, n, k, ep);
   }
   PW_HIP(hipGetLastError());
   return PW_OK;
@@ -1115,25 +1134,22 @@ template int gemm_nn_ep<float>(pw_ctx*, int, int, int, const float*, int, const 
 // nbatch products C_b = A_b^T B_b (n1 x n2, K rows; A_b, B_b, C_b from
 // device pointer tables dA, dB, dC, one leading dimension each): one
 // launch of split-K partial tiles for all products and one fixed-order
-// reduction, each about 2048 workgroups in all.
+// reduction.
 template <typename T>
 int gemm_tn_batched(pw_ctx* c, int K, int n1, int n2, const T* const* dA, int lda, const T* const* dB, int ldb,
                     T* const* dC, int ldc, int nbatch) {
   if (n1 <= 0 || n2 <= 0 || nbatch <= 0) return PW_OK;
-  const int ti = (n1 + BM - 1) / BM, tj = (n2 + BN - 1) / BN, tiles = ti * tj;
-  int nsplit = std::max(1, std::min((2048 + tiles * nbatch - 1) / (tiles * nbatch), (K + 255) / 256));
-  int kc = (K + nsplit - 1) / nsplit;
-  kc = (kc + BK - 1) / BK * BK;
-  nsplit = (K + kc - 1) / kc;
-  const long per = (long)n1 * n2 * nsplit;  // partials of one product
+  const TnShape s = tn_shape<T>(K, n1, n2, nbatch, 0, 1 << 20);
+  const long per = (long)n1 * n2 * s.nsplit;  // partials of one product
   PW_TRY(grow_gemm_ws(c, sizeof(T) * (size_t)per * nbatch));
   T* P = (T*)c->d_gemm_ws;
-  const size_t lds = sizeof(T) * 2 * (size_t)BM * (BK + 1);
-  hipLaunchKernelGGL((k_gemm_tn_partial<T, 1>), dim3(tiles * nsplit, nbatch), dim3(256), lds, c->stream,
-                     (const T*)nullptr, lda, (const T*)nullptr, ldb, K, n1, n2, kc, P, dA, dB, per);
+  const auto kern = tn_kernel<T>(s.ni, s.nj);
+  PW_TRY(ensure_lds((const void*)kern, s.lds));
+  hipLaunchKernelGGL(kern, dim3(s.tiles * s.nsplit, nbatch), dim3(256), s.lds, c->stream, (const T*)nullptr, lda,
+                     (const T*)nullptr, ldb, K, n1, n2, s.kc, P, dA, dB, per);
   const long total = (long)n1 * n2;
   const int g = (int)std::max<long>(1, std::min<long>((total + 255) / 256, 4096));
-  hipLaunchKernelGGL(k_gemm_tn_reduce<T>, dim3(g, nbatch), dim3(256), 0, c->stream, (const T*)P, nsplit, n1, n2,
+  hipLaunchKernelGGL(k_gemm_tn_reduce<T>, dim3(g, nbatch), dim3(256), 0, c->stream, (const T*)P, s.nsplit, n1, n2,
                      (T*)nullptr, ldc, (const T*)nullptr, (T)0, dC, per);
   PW_HIP(hipGetLastError());
   return PW_OK;

@@ -334,8 +334,8 @@ struct pw_ctx {
   //   compiled (PW_SLAB=lds: the LDS kernel); cg / rp / threads: the LDS kernel's y column groups (0 = two
   //   y buffers), x row pairs per step, threads per workgroup (0 = the
   //   built-in rule; PW_SLAB=lds:<cg>:<rp>:<threads>); tn_tm / tn_cap: the
-  //   split-K TN product's tile (1: 64 x 64, 2: 128 x 128) and the number of
-  //   partial workgroups aimed at (0 = the built-in rule)
+  //   split-BF16 split-K TN product's tile (1: 64 x 64, 2: 128 x 128) and the
+  //   number of partial workgroups a TN product aims at (0 = the built-in rule)
   struct Plan {
     bool reg = true;
     bool mm = true;        // the matrix-core slab kernel where it wins

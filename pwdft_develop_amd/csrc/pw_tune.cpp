@@ -146,7 +146,7 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
   const std::string base = device_tag(c->device) + "|" + std::to_string(c->n1) + "x" + std::to_string(c->n2) + "x" +
                            std::to_string(c->n3) + "|npw" + std::to_string(c->npw) + "|nb" + std::to_string(nb) +
                            (dtype == PW_F64 ? "|f64" : "|f32");
-  const std::string kslab = base + "|slab", ktn = base + "|tn" + std::to_string(c->nbeta);
+  const std::string kslab = base + "|slab", ktn = base + "|tn-reg" + std::to_string(c->nbeta);
   auto cache = read_cache(cache_path);
   std::string out;
   // blocks to time on (deterministic content)
@@ -220,7 +220,7 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
   if (c->nbeta > 0) {
     int tm = 0, cap = 0;
     auto jt = cache.find(ktn);
-    if (jt != cache.end() && sscanf(jt->second.c_str(), "%d %d", &tm, &cap) == 2 && (tm == 1 || tm == 2) && cap > 0) {
+    if (jt != cache.end() && sscanf(jt->second.c_str(), "%d %d", &tm, &cap) == 2 && tm >= 0 && tm <= 2 && cap > 0) {
       pl.tn_tm = tm;
       pl.tn_cap = cap;
       out += "; tn " + std::to_string(tm) + " " + std::to_string(cap) + " (cached)";
@@ -229,34 +229,32 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
         return done(fail(PW_ERR_NOMEM, "pw_autotune: cannot allocate the projection block"));
       const int K = 2 * c->npw;
       double tbest = 1e30;
-      int btm = 1, bcap = 1024;
-      for (int t : {1, 2})
-        for (int cp : {256, 512, 1024, 2048}) {
-          pl.tn_tm = t;
-          pl.tn_cap = cp;
-          double ms = 0;
-          int rc;
-          if (dtype == PW_F64)
-            rc = time_min(c->stream, 3, [&] {
-              return gemm_tn<double>(c, K, c->nbeta, nb, c->d_beta, K, (const double*)X, K, (double*)W, c->nbeta,
-                                     nullptr, 0.0);
-            }, &ms);
-          else
-            rc = time_min(c->stream, 3, [&] {
-              return gemm_tn<float>(c, K, c->nbeta, nb, c->d_beta_f, K, (const float*)X, K, (float*)W, c->nbeta,
-                                    nullptr, 0.f);
-            }, &ms);
-          if (rc == PW_OK && ms < tbest) {
-            tbest = ms;
-            btm = t;
-            bcap = cp;
-          }
+      int bcap = 256;
+      for (int cp : {128, 256, 512, 1024}) {
+        pl.tn_tm = 0;
+        pl.tn_cap = cp;
+        double ms = 0;
+        int rc;
+        if (dtype == PW_F64)
+          rc = time_min(c->stream, 3, [&] {
+            return gemm_tn<double>(c, K, c->nbeta, nb, c->d_beta, K, (const double*)X, K, (double*)W, c->nbeta,
+                                   nullptr, 0.0);
+          }, &ms);
+        else
+          rc = time_min(c->stream, 3, [&] {
+            return gemm_tn<float>(c, K, c->nbeta, nb, c->d_beta_f, K, (const float*)X, K, (float*)W, c->nbeta,
+                                  nullptr, 0.f);
+          }, &ms);
+        if (rc == PW_OK && ms < tbest) {
+          tbest = ms;
+          bcap = cp;
         }
-      pl.tn_tm = btm;
+      }
+      pl.tn_tm = 0;
       pl.tn_cap = bcap;
-      append_cache(cache_path, ktn, std::to_string(btm) + " " + std::to_string(bcap));
+      append_cache(cache_path, ktn, "0 " + std::to_string(bcap));
       char b[96];
-      snprintf(b, sizeof(b), "; tn %d %d (%.4f ms)", btm, bcap, tbest);
+      snprintf(b, sizeof(b), "; tn 0 %d (%.4f ms)", bcap, tbest);
       out += b;
     }
   }
