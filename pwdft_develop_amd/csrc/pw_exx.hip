@@ -294,14 +294,20 @@ k_exx_pair_acc(const typename cx<T>::t* __restrict__ fst, const T* __restrict__ 
 // 4 where 4 divides N, else 2), so that each thread holds N / L values and
 // the passes need no LDS round trips or barriers of their own.  LDS holds
 // one y-space (kxmax + 1 <= N / 2 + 1 columns of N), which the pair
-// densities' row pairs share before the x transform; ExxReg<T, N> carries
-// the shape.  One workgroup per (z plane, pair) as in the LDS kernels;
+// densities' row pairs share before the x transform, padded so that the lanes
+// of neighbouring columns use different banks; ExxReg<T, N> carries the shape.
+// Bound by LDS and its latency at two to four workgroups a CU: 96 x 96 x 40
+// FP32, 3072 pairs: forward 3002 -> 2082 us (17 ns a plane; its sticks take 6
+// to write), accumulation 3453 -> 2738 (22 ns).  One workgroup per (z plane, pair) as in the LDS kernels;
 // the row-pair and column phases run on N / 2 L and (kxmax + 1) L threads.
 template <typename T, int N>
 struct ExxReg {
   static constexpr int L = N % 4 == 0 ? 4 : 2, M = N / L, NP = N / 2;
   static constexpr int NT = ((NP * L + 63) / 64) * 64;  // threads per workgroup
-  static constexpr int LDS = (NP + 1) * N * (int)sizeof(typename cx<T>::t);
+  // stride of a row pair and of a kx column: an odd multiple of L, so that the
+  // L lanes of neighbouring columns, L values each, fall on different banks
+  static constexpr int S = (N / L) % 2 ? N : N + L;
+  static constexpr int LDS = (NP + 1) * S * (int)sizeof(typename cx<T>::t);
   static constexpr int UMAX = (NP * (NP + 1) + NT - 1) / NT;  // unpack outputs per thread
 };
 
@@ -312,34 +318,31 @@ k_exx_pair_fwd_reg(const T* __restrict__ psir, const T* __restrict__ phir, int n
                    typename cx<T>::t* __restrict__ fst, const int* __restrict__ pos, int n3, int nstick, int kxmax) {
   typedef typename cx<T>::t C;
   typedef ExxReg<T, N> R;
-  constexpr int L = R::L, NP = R::NP, NT = R::NT;
+  struct __align__(16) C2 { C a, b; };
+  constexpr int L = R::L, NP = R::NP, NT = R::NT, S = R::S;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* Z = reinterpret_cast<C*>(smem_raw);  // row pairs Z[q][x], then y-space Y[k][y]
-  T* Zr = reinterpret_cast<T*>(smem_raw);
   const int t = threadIdx.x, z = blockIdx.x, p = blockIdx.y;
   const int k = p % nb, j = j0 + p / nb;
   const size_t plane = (size_t)N * N;
   const T* a = psir + ((size_t)k * n3 + z) * plane;
   const T* b = phir + ((size_t)j * n3 + z) * plane;
   // products, rows 2q and 2q + 1 as the real and imaginary parts of Z[q]
-  for (int e0 = 0; e0 < N * N; e0 += 4 * NT) {
-    T u[4];
+  for (int e0 = 0; e0 < NP * N; e0 += 4 * NT) {
+    C u[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int e = e0 + t + NT * i;
-      u[i] = e < N * N ? a[e] * b[e] : (T)0;
+      const int e = min(e0 + t + NT * i, NP * N - 1), q = e / N, r = q * N + e;
+      u[i] = C{a[r] * b[r], a[r + N] * b[r + N]};
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int e = e0 + t + NT * i;
-      if (e < N * N) {
-        const int y = e / N, x = e - y * N;
-        Zr[2 * ((y >> 1) * N + x) + (y & 1)] = u[i];
-      }
+      const int e = e0 + t + NT * i, q = e / N;
+      if (e < NP * N) Z[q * (S - N) + e] = u[i];
     }
   }
   __syncthreads();
-  if (t < NP * L) col_fft_lanes<T, N, -1, L>(Z + (t / L) * N, t % L);
+  if (t < NP * L) col_fft_lanes<T, N, -1, L>(Z + (t / L) * S, t % L);
   __syncthreads();
   // unpack the two rows' spectra for kx <= kxmax (reads, barrier, writes:
   // the y-space overlays the row pairs)
@@ -348,9 +351,9 @@ k_exx_pair_fwd_reg(const T* __restrict__ psir, const T* __restrict__ phir, int n
 #pragma unroll
   for (int u = 0; u < R::UMAX; u++) {
     const int e = t + NT * u;
-    if (e < NP * nk) {
-      const int q = e / nk, kk = e - q * nk;
-      const C w = Z[q * N + kk], wc = Z[q * N + (kk == 0 ? 0 : N - kk)];
+    const int q = e / (NP + 1), kk = e - q * (NP + 1);
+    if (q < NP && kk < nk) {
+      const C w = Z[q * S + kk], wc = Z[q * S + (kk == 0 ? 0 : N - kk)];
       o1[u] = C{(T)0.5 * (w.x + wc.x), (T)0.5 * (w.y - wc.y)};
       o2[u] = C{(T)0.5 * (w.y + wc.y), (T)0.5 * (wc.x - w.x)};
     }
@@ -359,14 +362,13 @@ k_exx_pair_fwd_reg(const T* __restrict__ psir, const T* __restrict__ phir, int n
 #pragma unroll
   for (int u = 0; u < R::UMAX; u++) {
     const int e = t + NT * u;
-    if (e < NP * nk) {
-      const int q = e / nk, kk = e - q * nk;
-      Z[kk * N + 2 * q] = o1[u];
-      Z[kk * N + 2 * q + 1] = o2[u];
+    const int q = e / (NP + 1), kk = e - q * (NP + 1);
+    if (q < NP && kk < nk) {
+      *(C2*)(Z + kk * S + 2 * q) = C2{o1[u], o2[u]};
     }
   }
   __syncthreads();
-  for (int c = t / L; c < nk; c += NT / L) col_fft_lanes<T, N, -1, L>(Z + c * N, t % L);
+  for (int c = t / L; c < nk; c += NT / L) col_fft_lanes<T, N, -1, L>(Z + c * S, t % L);
   __syncthreads();
   C* dst = fst + ((size_t)p * n3 + z) * nstick;
   for (int s0 = 0; s0 < nstick; s0 += 4 * NT) {
@@ -374,7 +376,7 @@ k_exx_pair_fwd_reg(const T* __restrict__ psir, const T* __restrict__ phir, int n
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int s1 = s0 + t + NT * i;
-      g[i] = s1 < nstick ? Z[pos[s1]] : C{0, 0};
+      g[i] = s1 < nstick ? Z[pos[s1] + (S - N) * (pos[s1] / N)] : C{0, 0};
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -394,9 +396,11 @@ k_exx_pair_acc_reg(const typename cx<T>::t* __restrict__ fst, const T* __restric
                    const int* __restrict__ pos, int n3, int nstick, int kxmax) {
   typedef typename cx<T>::t C;
   typedef ExxReg<T, N> R;
-  constexpr int L = R::L, M = R::M, NP = R::NP, NT = R::NT;
+  struct __align__(16) C2 { C a, b; };
+  constexpr int L = R::L, M = R::M, NP = R::NP, NT = R::NT, S = R::S;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* Y = reinterpret_cast<C*>(smem_raw);
+  constexpr int U = 10;  // sticks a thread has in flight
   const int t = threadIdx.x, z = blockIdx.x, k = blockIdx.y;
   const int nk = kxmax + 1;
   const size_t plane = (size_t)N * N;
@@ -415,24 +419,24 @@ k_exx_pair_acc_reg(const typename cx<T>::t* __restrict__ fst, const T* __restric
     const int j = j0 + jl;
     const T fj = fac[j];
     const int p = k + nb * jl;
-    for (int e = t; e < nk * N; e += NT) Y[e] = C{0, 0};
+    for (int e = t; e < nk * S / 2; e += NT) ((C2*)Y)[e] = C2{C{0, 0}, C{0, 0}};
     __syncthreads();
     const C* src = fst + ((size_t)p * n3 + z) * nstick;
-    for (int s0 = 0; s0 < nstick; s0 += 4 * NT) {
-      C g[4];
+    for (int s0 = 0; s0 < nstick; s0 += U * NT) {
+      C g[U];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < U; i++) {
         const int s1 = s0 + t + NT * i;
         g[i] = s1 < nstick ? src[s1] : C{0, 0};
       }
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < U; i++) {
         const int s1 = s0 + t + NT * i;
-        if (s1 < nstick) Y[pos[s1]] = g[i];
+        if (s1 < nstick) Y[pos[s1] + (S - N) * (pos[s1] / N)] = g[i];
       }
     }
     __syncthreads();
-    for (int c = t / L; c < nk; c += NT / L) col_fft_lanes<T, N, 1, L>(Y + c * N, t % L);
+    for (int c = t / L; c < nk; c += NT / L) col_fft_lanes<T, N, 1, L>(Y + c * S, t % L);
     __syncthreads();
     if (rowt) {
       // Hermitian-extended spectra of rows y1, y2 at x frequencies m L + h,
@@ -446,8 +450,9 @@ k_exx_pair_acc_reg(const typename cx<T>::t* __restrict__ fst, const T* __restric
         if (kf > N / 2) { kk = N - kf; cj = true; }
         C a1 = C{0, 0}, a2 = C{0, 0};
         if (kk <= kxmax) {
-          a1 = Y[kk * N + y1];
-          a2 = Y[kk * N + y2];
+          const C2 y12 = *(const C2*)(Y + kk * S + y1);
+          a1 = y12.a;
+          a2 = y12.b;
           if (cj) { a1.y = -a1.y; a2.y = -a2.y; }
           if (kf == 0 || 2 * kf == N) { a1.y = 0; a2.y = 0; }
         }
@@ -663,15 +668,14 @@ struct ExxRegKernels {
 template <typename T>
 static ExxRegKernels<T> exx_reg_kernels(int n1, int n2) {
   ExxRegKernels<T> k;
-  // FP32 takes the register kernels, FP64 the LDS ones (config-4 exchange,
-  // 1024 x 432 pairs on 96 x 96 x 40: FP32 1.14 s register against 1.89 s
-  // LDS; FP64 3.34 against 3.32 s, the FP64 register kernels at one wave
-  // per SIMD).  PW_EXX_PAIR (for comparisons): "lds" both LDS kernels,
-  // "reg" both register kernels in either precision, "fwd" the register
-  // forward kernel only.
+  // The register kernels wherever the plane has one; us for 32 x 32 pairs, LDS
+  // / register kernels: 96 x 96 x 40 FP32 4732 / 2465, FP64 7938 / 6655; 48^3
+  // 1115 / 634, 2305 / 1387; 30^3 330 / 236, 451 / 395; 24^3 246 / 149, 309 /
+  // 207.  PW_EXX_PAIR (for comparisons): "lds" both LDS kernels, "fwd" the
+  // register forward kernel only.
   const char* f = getenv("PW_EXX_PAIR");
   const std::string mode = f ? f : "";
-  if (n1 != n2 || mode == "lds" || (sizeof(T) == 8 && mode != "reg")) return k;
+  if (n1 != n2 || mode == "lds") return k;
   switch (n1) {
 #define PW_CASE(n)                              \
   case n:                                       \
