@@ -32,18 +32,29 @@
 namespace pw {
 
 // ---------------------------------------------------------------- kernel 1
+// Sixteen sticks a workgroup, transformed in LDS.  FP32 columns are padded to
+// an odd length, so that the sixteen sticks of a z, side by side in t1 and t2,
+// are in different banks (72 points, 256 bands of 180 x 180 columns: inverse
+// 213 -> 204 us, forward 238 -> 229; FP64 columns gain nothing: 60 points 33.5
+// against 35.4 us padded).
+template <typename T>
+__host__ __device__ constexpr int z_ld(int n3) {
+  return sizeof(T) == 4 ? n3 | 1 : n3;
+}
+
 template <typename T, int N3>
 __global__ void __launch_bounds__(256)
 k_sticks_inverse_z(const typename cx<T>::t* __restrict__ psi, int ldpsi,
-                   typename cx<T>::t* __restrict__ t1, int n3_, int nstick, int sc, int nchunk,
+                   typename cx<T>::t* __restrict__ t1, int n3_, int nstick, int nchunk,
                    const int* __restrict__ chunk_off, const int* __restrict__ pt_idx,
                    const int* __restrict__ pt_sz, const typename cx<T>::t* __restrict__ tw3g) {
   typedef typename cx<T>::t C;
-  const int n3 = N3 > 0 ? N3 : n3_;
+  constexpr int sc = kStickChunk;
+  const int n3 = N3 > 0 ? N3 : n3_, ld = z_ld<T>(n3);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* tw = reinterpret_cast<C*>(smem_raw);
   C* A = tw + n3;
-  C* B = A + sc * n3;
+  C* B = A + sc * ld;
   // one row of nchunk x nb blocks; the chunks of a band in order on one XCD
   // (neighbouring chunks share the cache lines at their ends)
   const int item = xcd_item(blockIdx.x, gridDim.x);
@@ -51,7 +62,7 @@ k_sticks_inverse_z(const typename cx<T>::t* __restrict__ psi, int ldpsi,
   const int s0 = c * sc;
   const C* ps = psi + (size_t)band * ldpsi;
   for (int t = threadIdx.x; t < n3; t += blockDim.x) tw[t] = tw3g[t];
-  for (int t = threadIdx.x; t < sc * n3; t += blockDim.x) A[t] = C{0, 0};
+  for (int t = threadIdx.x; t < sc * ld; t += blockDim.x) A[t] = C{0, 0};
   __syncthreads();
   const T is2 = (T)0.70710678118654752440084436210485;
   const int e = chunk_off[c + 1];
@@ -66,14 +77,14 @@ k_sticks_inverse_z(const typename cx<T>::t* __restrict__ psi, int ldpsi,
       C u = ps[-i - 1];
       v = C{u.x * is2, -u.y * is2};
     }
-    A[(sz & 0xffff) * n3 + (sz >> 16)] = v;
+    A[(sz & 0xffff) * ld + (sz >> 16)] = v;
   }
   __syncthreads();
-  C* R = lds_fft_n<T, N3>(A, B, n3, sc, n3, tw, (T)1);
+  C* R = lds_fft_n<T, N3>(A, B, n3, sc, ld, tw, (T)1);
   const int nsl = min(sc, nstick - s0);
-  for (int t = threadIdx.x; t < n3 * nsl; t += blockDim.x) {
-    const int z = t / nsl, sl = t - z * nsl;
-    t1[((size_t)band * n3 + z) * nstick + s0 + sl] = R[sl * n3 + z];
+  for (int t = threadIdx.x; t < n3 * sc; t += blockDim.x) {
+    const int z = t / sc, sl = t - z * sc;
+    if (sl < nsl) t1[((size_t)band * n3 + z) * nstick + s0 + sl] = R[sl * ld + z];
   }
 }
 
@@ -194,16 +205,17 @@ k_slab_xy_reg(const typename cx<T>::t* __restrict__ t1, typename cx<T>::t* __res
 template <typename T, int N3>
 __global__ void __launch_bounds__(256)
 k_sticks_forward_z(const typename cx<T>::t* __restrict__ t2, const typename cx<T>::t* __restrict__ psi,
-                   typename cx<T>::t* __restrict__ out, int ld, int n3_, int nstick, int sc, int nchunk,
+                   typename cx<T>::t* __restrict__ out, int ldo, int n3_, int nstick, int nchunk,
                    const int* __restrict__ gchunk_off, const int* __restrict__ gpt_idx,
                    const int* __restrict__ gpt_sz, const T* __restrict__ ekin,
                    const typename cx<T>::t* __restrict__ tw3g) {
   typedef typename cx<T>::t C;
-  const int n3 = N3 > 0 ? N3 : n3_;
+  constexpr int sc = kStickChunk;
+  const int n3 = N3 > 0 ? N3 : n3_, ld = z_ld<T>(n3);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* tw = reinterpret_cast<C*>(smem_raw);
   C* A = tw + n3;
-  C* B = A + sc * n3;
+  C* B = A + sc * ld;
   const int item = xcd_item(blockIdx.x, gridDim.x);  // as in k_sticks_inverse_z
   const int band = item / nchunk, c = item - band * nchunk;
   const int s0 = c * sc;
@@ -211,18 +223,18 @@ k_sticks_forward_z(const typename cx<T>::t* __restrict__ t2, const typename cx<T
   for (int t = threadIdx.x; t < n3; t += blockDim.x) tw[t] = tw3g[t];
   for (int t = threadIdx.x; t < n3 * sc; t += blockDim.x) {
     const int z = t / sc, sl = t - z * sc;
-    A[sl * n3 + z] = (sl < nsl) ? t2[((size_t)band * n3 + z) * nstick + s0 + sl] : C{0, 0};
+    A[sl * ld + z] = (sl < nsl) ? t2[((size_t)band * n3 + z) * nstick + s0 + sl] : C{0, 0};
   }
   __syncthreads();
-  C* R = lds_fft_n<T, N3>(A, B, n3, sc, n3, tw, (T)-1);
-  const C* ps = psi + (size_t)band * ld;
-  C* o = out + (size_t)band * ld;
+  C* R = lds_fft_n<T, N3>(A, B, n3, sc, ld, tw, (T)-1);
+  const C* ps = psi + (size_t)band * ldo;
+  C* o = out + (size_t)band * ldo;
   const T s2 = (T)1.4142135623730950488016887242097;
   const int e = gchunk_off[c + 1];
   for (int t = gchunk_off[c] + threadIdx.x; t < e; t += blockDim.x) {
     const int i = gpt_idx[t];
     const int sz = gpt_sz[t];
-    C y = R[(sz & 0xffff) * n3 + (sz >> 16)];
+    C y = R[(sz & 0xffff) * ld + (sz >> 16)];
     if (i != 0) y = cscale(y, s2);
     if (ekin) {
       const C cc = ps[i];
@@ -383,13 +395,17 @@ static size_t slab_reg_lds(const pw_ctx* c, size_t csz, int sb) {
          sizeof(int) * 2 * (size_t)c->sp.nstick;
 }
 
+// ... and z lengths: every 2/3/5-smooth one from 24 to 72 besides (54 points,
+// 77 bands of 45 x 50 columns, FP64: 13.4 us at run-time length, 10.1 here)
+#define PW_Z_SIZES(X) PW_FFT_SIZES(X) X(25) X(27) X(45) X(50) X(54) X(64)
+
 template <typename T>
 auto inv_z_kernel(int n3) -> decltype(&k_sticks_inverse_z<T, 0>) {
   switch (n3) {
 #define PW_CASE(n) \
   case n:          \
     return &k_sticks_inverse_z<T, n>;
-    PW_FFT_SIZES(PW_CASE)
+    PW_Z_SIZES(PW_CASE)
 #undef PW_CASE
     default:
       return &k_sticks_inverse_z<T, 0>;
@@ -437,7 +453,7 @@ auto fwd_z_kernel(int n3) -> decltype(&k_sticks_forward_z<T, 0>) {
 #define PW_CASE(n) \
   case n:          \
     return &k_sticks_forward_z<T, n>;
-    PW_FFT_SIZES(PW_CASE)
+    PW_Z_SIZES(PW_CASE)
 #undef PW_CASE
     default:
       return &k_sticks_forward_z<T, 0>;
@@ -540,7 +556,7 @@ static void build_stick_plan(pw_ctx* c, const int* idx) {
         if (kx > sp.kxmax) sp.kxmax = kx;
       }
   sp.nstick = (int)sp.kx.size();
-  sp.nchunk = (sp.nstick + sp.sc - 1) / sp.sc;
+  sp.nchunk = (sp.nstick + kStickChunk - 1) / kStickChunk;
   sp.pos.resize(sp.nstick);
   sp.mpos.resize(sp.nstick);
   for (int s = 0; s < sp.nstick; s++) {
@@ -554,7 +570,7 @@ static void build_stick_plan(pw_ctx* c, const int* idx) {
     const int g = idx[i];
     const int col = g % (h1 * n2), kz = g / (h1 * n2);
     const int s = sid[col];
-    const int ch = s / sp.sc, sl = s % sp.sc;
+    const int ch = s / kStickChunk, sl = s % kStickChunk;
     fw[ch].push_back({kz, sl, i});
     inv[ch].push_back({kz, sl, i});
     // the (0,0) column holds kz >= 0 only; its conj mirror fills -kz
@@ -836,6 +852,10 @@ static int mark(pw_ctx* c, int k) {
 
 // LDS bytes of k_slab_xy: twiddles, y-space (two copies when cg == 0, one
 // plus a cg-column scratch shared with the x rows otherwise), x rows.
+template <typename T>
+static size_t z_lds(const pw_ctx* c) {
+  return sizeof(typename cx<T>::t) * (c->n3 + 2 * (size_t)kStickChunk * z_ld<T>(c->n3));
+}
 static size_t slab_lds(const pw_ctx* c, int esz, int rp, int cg) {
   const size_t nk = c->sp.kxmax + 1, n1 = c->n1, n2 = c->n2;
   if (cg == 0) return esz * (n1 + n2 + 2 * nk * n2 + 2 * (size_t)rp * n1);
@@ -874,7 +894,6 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
   const C* tw3 = tw2 + c->n2;
   const T* vt = (const T*)(sizeof(T) == 8 ? (const void*)c->d_vtot : (const void*)c->d_vtot_f);
   const T* ek = (const T*)(sizeof(T) == 8 ? (const void*)c->d_ekin : (const void*)c->d_ekin_f);
-  const int sc = c->sp.sc;
   C* t1 = (C*)c->d_t1;
   C* t2 = (C*)c->d_t2;
   // x-pass row-pair chunk: as many pairs as fit next to the y buffers in 64 KiB
@@ -931,7 +950,6 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
   const slab_reg_fn<T> kreg = pl.reg && !few ? slab_reg_kernel<T>(c->n1, c->n2, pl.ly) : nullptr;
   if (lds2 > 160 * 1024)
     return fail(PW_ERR_UNSUPPORTED, "H*psi slab needs %zu bytes of LDS (> 160 KiB)", lds2);
-  const size_t lds1 = (size_t)esz * (c->n3 + 2 * (size_t)sc * c->n3);
   PW_TRY(mark(c, 0));
   PW_TRY(launch_inv_z<T>(c, nb, (const C*)psi, t1, tw3));
   PW_TRY(mark(c, 1));
@@ -986,9 +1004,9 @@ int launch_inv_z(pw_ctx* c, int nb, const typename cx<T>::t* psi, typename cx<T>
     hipLaunchKernelGGL(kr, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, c->stream, psi, c->npw, t1,
                        c->sp.nstick, nwork, c->d_zs);
   } else {
-    const size_t lds1 = sizeof(C) * (c->n3 + 2 * (size_t)c->sp.sc * c->n3);
+    const size_t lds1 = z_lds<T>(c);
     hipLaunchKernelGGL(inv_z_kernel<T>(c->n3), dim3(c->sp.nchunk * nb), dim3(256), lds1, c->stream, psi, c->npw,
-                       t1, c->n3, c->sp.nstick, c->sp.sc, c->sp.nchunk, c->d_chunk_off, c->d_pt_idx, c->d_pt_sz,
+                       t1, c->n3, c->sp.nstick, c->sp.nchunk, c->d_chunk_off, c->d_pt_idx, c->d_pt_sz,
                        tw3);
   }
   PW_HIP(hipGetLastError());
@@ -1007,9 +1025,9 @@ int launch_fwd_z(pw_ctx* c, int nb, const typename cx<T>::t* t2, const typename 
     hipLaunchKernelGGL(kr, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, c->stream, t2, psi, out, c->npw,
                        c->sp.nstick, nwork, c->d_zs, ek);
   } else {
-    const size_t lds1 = sizeof(C) * (c->n3 + 2 * (size_t)c->sp.sc * c->n3);
+    const size_t lds1 = z_lds<T>(c);
     hipLaunchKernelGGL(fwd_z_kernel<T>(c->n3), dim3(c->sp.nchunk * nb), dim3(256), lds1, c->stream, t2, psi, out,
-                       c->npw, c->n3, c->sp.nstick, c->sp.sc, c->sp.nchunk, c->d_gchunk_off, c->d_gpt_idx,
+                       c->npw, c->n3, c->sp.nstick, c->sp.nchunk, c->d_gchunk_off, c->d_gpt_idx,
                        c->d_gpt_sz, ek, tw3);
   }
   PW_HIP(hipGetLastError());
@@ -1021,7 +1039,6 @@ template <typename T>
 int sphere_to_sticks(pw_ctx* c, int nb, const void* psi, void* t1) {
   typedef typename cx<T>::t C;
   const C* tw3 = (const C*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32) + c->n1 + c->n2;
-  const size_t lds1 = sizeof(C) * (c->n3 + 2 * (size_t)c->sp.sc * c->n3);
   return launch_inv_z<T>(c, nb, (const C*)psi, (C*)t1, tw3);
 }
 
@@ -1030,7 +1047,6 @@ template <typename T>
 int sticks_to_sphere_add(pw_ctx* c, int nb, const void* t2, void* out) {
   typedef typename cx<T>::t C;
   const C* tw3 = (const C*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32) + c->n1 + c->n2;
-  const size_t lds1 = sizeof(C) * (c->n3 + 2 * (size_t)c->sp.sc * c->n3);
   return launch_fwd_z<T>(c, nb, (const C*)t2, (const C*)nullptr, (C*)out, (const T*)nullptr, tw3);
 }
 

@@ -106,11 +106,12 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+constexpr int kStickChunk = 16;  // sticks a workgroup of the z kernels takes
+
 // Stick decomposition of the half sphere: the distinct (kx, ky) columns of
 // the sphere; each column is transformed along z, each z slab along y and x.
 struct StickPlan {
   int nstick = 0, kxmax = 0;
-  int sc = 16;        // sticks per chunk in the z kernels
   int nchunk = 0;
   std::vector<int> kx, ky;        // per stick (ky = storage index 0..n2-1)
   // per chunk point list, (z, stick) ordered: packed = sphere_idx, and
