@@ -894,10 +894,10 @@ static TnKernel<T> tn_kernel(int ni, int nj) {
 // workgroups as the CUs hold (cap: aimed at instead), so that all of them run
 // at once; at least 128 rows a split, and at most 64 splits, whose partials
 // the reduction reads one after the other.  Tiles of up to 64 x 64, or 32 x 32
-// where those leave most CUs without work.  us, FP64: 26268 x 256 x 256 with
+// where those leave most CUs without work.  us, FP64: 13134 x 256 x 256 with
 // 64 x 64 tiles 43.3 (256 workgroups; 512: 53.4), 32 x 64 46.5, 48 x 48 55.5,
-// 32 x 32 57.0 (through LDS, 64 x 64 split over the wavefronts: 58.9); 15100 x
-// 76 x 77 7.9, 8.8 with 32 x 48 tiles; 5700 x 48 x 64 8.2, 5.0 with 32 x 32.
+// 32 x 32 57.0 (through LDS, 64 x 64 split over the wavefronts: 58.9); 7550 x
+// 76 x 77 7.9, 8.7 with 32 x 48 tiles; 2944 x 48 x 64 8.2, 4.5 with 32 x 32.
 // FP32, 152400 x 256 x 256: 195 with two 64 x 64 workgroups a CU, 235 with one,
 // 217 with 32 x 64, 274 with 32 x 32 (through LDS: 240).
 struct TnShape {
@@ -1001,7 +1001,7 @@ int gemm_tn(pw_ctx* c, int K, int n1, int n2, const T* A, int lda, const T* B, i
 
 // 16 columns a wavefront where that takes fewer rounds of the chip's 1024 SIMDs
 // than 32 (few rows, or the ragged end of n), else 32.  us with 16 / 32 / 48 /
-// 64 columns: FP64 26268 x 256 x 256 50.6 / 47.2 / 77.2 / 55.2 (through LDS:
+// 64 columns: FP64 13134 x 256 x 256 50.6 / 47.2 / 77.2 / 55.2 (through LDS:
 // 65.8), 7550 x 77 x 76 12.5 / 21.6 / 29.1 / 36.9; FP32 152400 x 256 x 256
 // 269 / 235 / 235 / 239 (through LDS: 302).
 template <typename T, bool kCheb>
