@@ -79,6 +79,33 @@ __device__ __forceinline__ int acc_col(int lane, int r) {
   return sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r;
 }
 
+// The four wavefronts' tiles of one workgroup, added in LDS in the order of
+// their rows, into P (n1 x n2).
+template <typename T, int NI, int NJ>
+__device__ __forceinline__ void tn_store(const typename acc4<T>::t (&acc)[NI][NJ], int i0, int j0, int n1, int n2,
+                                         T* __restrict__ P) {
+  typedef typename acc4<T>::t V;
+  extern __shared__ __align__(16) unsigned char gemm_smem[];
+  V* const red = (V*)gemm_smem;  // [4][NI * NJ][64]
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int a = 0; a < NI; a++)
+#pragma unroll
+    for (int b = 0; b < NJ; b++) red[((w * NI + a) * NJ + b) * 64 + lane] = acc[a][b];
+  __syncthreads();
+  for (int e = w; e < NI * NJ; e += 4) {
+    V s = red[e * 64 + lane];
+#pragma unroll
+    for (int v = 1; v < 4; v++) s += red[(v * NI * NJ + e) * 64 + lane];
+    const int row = i0 + 16 * (e / NJ) + (lane & 15);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int col = j0 + 16 * (e % NJ) + acc_col<T>(lane, r);
+      if (row < n1 && col < n2) P[row + (size_t)n1 * col] = s[r];
+    }
+  }
+}
+
 // Partial C tile of A^T B over K rows [kb, ke): P[split](n1 x n2, ld n1), a
 // 16 NI x 16 NJ tile per workgroup whose four wavefronts take a quarter of
 // the rows each and meet in LDS (4 NI NJ KiB a wavefront in FP64, half in
@@ -96,8 +123,6 @@ k_gemm_tn_partial(const T* __restrict__ A, int lda, const T* __restrict__ B, int
     B = Bb[blockIdx.y];
     P += blockIdx.y * sP;
   }
-  extern __shared__ __align__(16) unsigned char gemm_smem[];
-  V* const red = (V*)gemm_smem;  // [4][NI * NJ][64]
   const TnBlock tb = tn_block(n1, n2, K, kc, 16 * NI, 16 * NJ);
   const int i0 = tb.i * 16 * NI, j0 = tb.j * 16 * NJ, split = tb.split;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
@@ -152,23 +177,7 @@ k_gemm_tn_partial(const T* __restrict__ A, int lda, const T* __restrict__ B, int
     }
     mm(ra, rb);
   }
-#pragma unroll
-  for (int a = 0; a < NI; a++)
-#pragma unroll
-    for (int b = 0; b < NJ; b++) red[((w * NI + a) * NJ + b) * 64 + lane] = acc[a][b];
-  __syncthreads();
-  T* Ps = P + (size_t)split * n1 * n2;
-  for (int e = w; e < NI * NJ; e += 4) {
-    V s = red[e * 64 + lane];
-#pragma unroll
-    for (int v = 1; v < 4; v++) s += red[(v * NI * NJ + e) * 64 + lane];
-    const int row = i0 + 16 * (e / NJ) + c;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int col = j0 + 16 * (e % NJ) + acc_col<T>(lane, r);
-      if (row < n1 && col < n2) Ps[row + (size_t)n1 * col] = s[r];
-    }
-  }
+  tn_store<T, NI, NJ>(acc, i0, j0, n1, n2, P + (size_t)split * n1 * n2);
 }
 
 // ---- split BF16 products (FP32 data, FP32 accumulation) ----
@@ -242,116 +251,96 @@ constexpr int BKP = 40;  // LDS row stride of the bf16 tiles (80 bytes: 16-byte 
 __device__ constexpr int kSplitPairA[6] = {2, 0, 1, 1, 0, 0};
 __device__ constexpr int kSplitPairB[6] = {0, 2, 1, 0, 1, 0};
 
-// A^T B partials with FP32 inputs split into NS BF16 terms.  TM = 1: 64 x 64
-// tile, each wave 32 x 32; TM = 2: 128 x 128 tile, each wave 64 x 64 (twice
-// the flops per loaded byte, for large outputs).  The next 32-row K chunk is
-// loaded into registers while the MFMAs run on the current one in LDS; a
-// chunk is one 16x16x32 product per kept pairing of terms instead of eight
-// 16x16x4 FP32 products.
-template <int TM, int NS>
-__global__ void __launch_bounds__(256)
+// k_gemm_tn_partial with FP32 inputs split into NS BF16 terms: a lane loads
+// eight consecutive rows of a column per 32-row chunk (its operand of one
+// 16x16x32 product per kept pairing of terms, in place of eight 16x16x4 FP32
+// products) and splits them in registers.  The splitting (about 50 VALU
+// operations an operand tile) costs as much as the products; the two
+// wavefronts of a SIMD overlap one's with the other's.  13134 x 256 x 256:
+// 21.5 us (28.1 through LDS tiles of 64 x 64 split over the wavefronts).
+template <int NS>
+__device__ __forceinline__ void split8(const f4v& lo, const f4v& hi, bf16x8 (&t)[NS]) {
+  uint2 u[NS], v[NS];
+  bf16_split4<NS>(float2{lo[0], lo[1]}, float2{lo[2], lo[3]}, u);
+  bf16_split4<NS>(float2{hi[0], hi[1]}, float2{hi[2], hi[3]}, v);
+#pragma unroll
+  for (int i = 0; i < NS; i++) t[i] = __builtin_bit_cast(bf16x8, uint4{u[i].x, u[i].y, v[i].x, v[i].y});
+}
+template <int NI, int NJ, int NS>
+__global__ void __launch_bounds__(256, 2)
 k_gemm_tn_partial_bf(const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, int K, int n1,
                      int n2, int kc, float* __restrict__ P) {
-  constexpr int TB = BM * TM, NQ = 8 * TM, NA = 2 * TM;
-  extern __shared__ __align__(16) unsigned char gemm_smem[];
-  unsigned short* As = reinterpret_cast<unsigned short*>(gemm_smem);  // NS term tiles of A, then of B
-  unsigned short* Bs = As + NS * TB * BKP;
-  const TnBlock tb = tn_block(n1, n2, K, kc, TB, TB);
-  const int i0 = tb.i * TB, j0 = tb.j * TB, split = tb.split;
-  const int kb = split * kc, ke = min(K, kb + kc);
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = (w & 1) * 32 * TM, wj = (w >> 1) * 32 * TM;
-  f4v acc[NA][NA];
+  typedef run4<float>::t R;
+  const TnBlock tb = tn_block(n1, n2, K, kc, 16 * NI, 16 * NJ);
+  const int i0 = tb.i * 16 * NI, j0 = tb.j * 16 * NJ, split = tb.split;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int kw = kc >> 2, kb = min(K, split * kc + w * kw), ke = min(K, kb + kw);
+  f4v acc[NI][NJ];
 #pragma unroll
-  for (int a = 0; a < NA; a++)
+  for (int a = 0; a < NI; a++)
 #pragma unroll
-    for (int b = 0; b < NA; b++) acc[a][b] = f4v{0, 0, 0, 0};
-  // thread t loads rows 4 (t % 8) .. + 3 of the chunk (two float pairs) of
-  // columns t / 8 + 32 q: unconditional loads at clamped indices (K, kb and
-  // kc are even, so a pair is wholly inside or outside [kb, ke)), zeroed
-  // outside the operands
-  constexpr int NC = 2 * TM;  // columns per thread and operand
-  const int k4 = 4 * (t & 7), lc = t >> 3;
-  float2 ra[NC][2], rb[NC][2];  // the next chunk in flight during the current one's products
-  auto load = [&](int k0, float2 (&ra)[NC][2], float2 (&rb)[NC][2]) {
+    for (int b = 0; b < NJ; b++) acc[a][b] = f4v{0, 0, 0, 0};
+  const float *pa[NI], *pb[NJ];  // columns beyond the matrix repeat its last one
 #pragma unroll
-    for (int q = 0; q < NC; q++) {
-      const int ci = i0 + lc + 32 * q, cj = j0 + lc + 32 * q;
-      const float* pa = A + (size_t)min(ci, n1 - 1) * lda;
-      const float* pb = B + (size_t)min(cj, n2 - 1) * ldb;
+  for (int a = 0; a < NI; a++) pa[a] = A + (size_t)min(i0 + 16 * a + c, n1 - 1) * lda;
+#pragma unroll
+  for (int b = 0; b < NJ; b++) pb[b] = B + (size_t)min(j0 + 16 * b + c, n2 - 1) * ldb;
+  auto mm = [&](const f4v (&ra)[NI][2], const f4v (&rb)[NJ][2]) {
+    bf16x8 fa[NI][NS];
+#pragma unroll
+    for (int a = 0; a < NI; a++) split8<NS>(ra[a][0], ra[a][1], fa[a]);
+#pragma unroll
+    for (int b = 0; b < NJ; b++) {
+      bf16x8 fb[NS];
+      split8<NS>(rb[b][0], rb[b][1], fb);
+      // term pair outer, tiles inner: mfma_split's order per tile
+#pragma unroll
+      for (int p = 6 - (NS == 3 ? 6 : 3); p < 6; p++)
+#pragma unroll
+        for (int a = 0; a < NI; a++)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kSplitPairB[p]], fa[a][kSplitPairA[p]], acc[a][b],
+                                                               0, 0, 0);
+    }
+  };
+  f4v ra[NI][2], rb[NJ][2];
+  const int nq = (ke - kb) >> 5;  // full chunks of 32 rows
+  if (nq > 0) {
+    auto load = [&](f4v (&xa)[NI][2], f4v (&xb)[NJ][2], int q) {
+      const int k = kb + 32 * min(q, nq - 1) + 8 * g;  // (the chunk past the end: read and dropped)
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        const int rc = min(k0 + k4 + 2 * h, ke - 2);
-        ra[q][h] = *reinterpret_cast<const float2*>(pa + rc);
-        rb[q][h] = *reinterpret_cast<const float2*>(pb + rc);
-      }
-    }
-  };
-  // the zero fill outside the operands at use, not at load (a select on a
-  // loaded value makes the compiler wait for the load where it is issued)
-  auto mask = [&](int k0, float2 (&ra)[NC][2], float2 (&rb)[NC][2]) {
 #pragma unroll
-    for (int q = 0; q < NC; q++) {
-      const int ci = i0 + lc + 32 * q, cj = j0 + lc + 32 * q;
+        for (int a = 0; a < NI; a++) xa[a][h] = *(const R*)(pa[a] + k + 4 * h);
+#pragma unroll
+        for (int b = 0; b < NJ; b++) xb[b][h] = *(const R*)(pb[b] + k + 4 * h);
+      }
+    };
+    load(ra, rb, 0);
+    for (int q = 0; q < nq; q++) {
+      f4v xa[NI][2], xb[NJ][2];
+      load(xa, xb, q + 1);
+      mm(ra, rb);
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        const int r = k0 + k4 + 2 * h;
-        if (!(ci < n1 && r < ke)) ra[q][h] = float2{0.f, 0.f};
-        if (!(cj < n2 && r < ke)) rb[q][h] = float2{0.f, 0.f};
+#pragma unroll
+        for (int a = 0; a < NI; a++) ra[a][h] = xa[a][h];
+#pragma unroll
+        for (int b = 0; b < NJ; b++) rb[b][h] = xb[b][h];
       }
     }
-  };
-  load(kb, ra, rb);
-  const int fr = lane & 15, fk = 8 * (lane >> 4);
-  // one chunk: its operands split into LDS, the next chunk's loads into the
-  // same registers, the products
-  auto chunk = [&](int k0, float2 (&ra)[NC][2], float2 (&rb)[NC][2]) {
-    mask(k0, ra, rb);
+  }
+  if (kb + 32 * nq < ke) {  // the last, incomplete chunk
 #pragma unroll
-    for (int q = 0; q < NC; q++) {
-      uint2 ta[NS], tb[NS];
-      bf16_split4<NS>(ra[q][0], ra[q][1], ta);
-      bf16_split4<NS>(rb[q][0], rb[q][1], tb);
+    for (int i = 0; i < 8; i++) {
+      const int k = kb + 32 * nq + 8 * g + i, kk = min(k, ke - 1);
 #pragma unroll
-      for (int i = 0; i < NS; i++) {
-        *reinterpret_cast<uint2*>(As + i * TB * BKP + (lc + 32 * q) * BKP + k4) = ta[i];
-        *reinterpret_cast<uint2*>(Bs + i * TB * BKP + (lc + 32 * q) * BKP + k4) = tb[i];
-      }
+      for (int a = 0; a < NI; a++) ra[a][i >> 2][i & 3] = k < ke ? pa[a][kk] : 0.f;
+#pragma unroll
+      for (int b = 0; b < NJ; b++) rb[b][i >> 2][i & 3] = k < ke ? pb[b][kk] : 0.f;
     }
-    lds_barrier();
-    if (k0 + BK < ke) load(k0 + BK, ra, rb);
-    bf16x8 fa[NA][NS], fb[NA][NS];
-#pragma unroll
-    for (int a = 0; a < NA; a++)
-#pragma unroll
-      for (int i = 0; i < NS; i++) {
-        fa[a][i] = *reinterpret_cast<const bf16x8*>(As + i * TB * BKP + (wi + a * 16 + fr) * BKP + fk);
-        fb[a][i] = *reinterpret_cast<const bf16x8*>(Bs + i * TB * BKP + (wj + a * 16 + fr) * BKP + fk);
-      }
-    // term pair outer, tiles inner: mfma_split's order per tile
-#pragma unroll
-    for (int p = 6 - (NS == 3 ? 6 : 3); p < 6; p++)
-#pragma unroll
-      for (int a = 0; a < NA; a++)
-#pragma unroll
-        for (int b = 0; b < NA; b++)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a][kSplitPairA[p]], fb[b][kSplitPairB[p]],
-                                                               acc[a][b], 0, 0, 0);
-    lds_barrier();
-  };
-  for (int k0 = kb; k0 < ke; k0 += BK) chunk(k0, ra, rb);
-  float* Ps = P + (size_t)split * n1 * n2;
-#pragma unroll
-  for (int a = 0; a < NA; a++)
-#pragma unroll
-    for (int b = 0; b < NA; b++) {
-      const int col = j0 + wj + b * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = i0 + wi + a * 16 + acc_col<float>(lane, r);
-        if (row < n1 && col < n2) Ps[row + (size_t)n1 * col] = acc[a][b][r];
-      }
-    }
+    mm(ra, rb);
+  }
+  tn_store<float, NI, NJ>(acc, i0, j0, n1, n2, P + (size_t)split * n1 * n2);
 }
 
 // C[i + ldc j] = rowscale[i] * sum_s P[s][i + n1 j] (+ beta C), rowscale may
@@ -890,6 +879,17 @@ static TnKernel<T> tn_kernel(int ni, int nj) {
   return k[ni - 2][nj - 2];
 }
 
+using TnKernelBf = void (*)(const float*, int, const float*, int, int, int, int, int, float*);
+
+template <int NS>
+static TnKernelBf tn_kernel_bf(int ni, int nj) {
+  static const TnKernelBf k[3][3] = {
+      {k_gemm_tn_partial_bf<2, 2, NS>, k_gemm_tn_partial_bf<2, 3, NS>, k_gemm_tn_partial_bf<2, 4, NS>},
+      {k_gemm_tn_partial_bf<3, 2, NS>, k_gemm_tn_partial_bf<3, 3, NS>, k_gemm_tn_partial_bf<3, 4, NS>},
+      {k_gemm_tn_partial_bf<4, 2, NS>, k_gemm_tn_partial_bf<4, 3, NS>, k_gemm_tn_partial_bf<4, 4, NS>}};
+  return k[ni - 2][nj - 2];
+}
+
 // Tiles, splits and rows per split of nbatch products K x n1 x n2: as many
 // workgroups as the CUs hold (cap: aimed at instead), so that all of them run
 // at once; at least 128 rows a split, and at most 64 splits, whose partials
@@ -905,7 +905,7 @@ struct TnShape {
   size_t lds;
 };
 template <typename T>
-static TnShape tn_shape(int K, int n1, int n2, int nbatch, int cap, int max_split) {
+static TnShape tn_shape(int K, int n1, int n2, int nbatch, int cap, int max_split, int rows4 = 64) {
   TnShape s;
   const int rows = std::min(64, (K + 127) / 128);
   const int most = (long)((n1 + 63) / 64) * ((n2 + 63) / 64) * nbatch * rows >= 192 ? 4 : 2;
@@ -916,7 +916,7 @@ static TnShape tn_shape(int K, int n1, int n2, int nbatch, int cap, int max_spli
   if (cap <= 0) cap = sizeof(T) * s.ni * s.nj > 96 ? 256 : 512;
   const long all = (long)s.tiles * nbatch;
   s.nsplit = (int)std::max(1L, std::min({cap / all, (long)(K + 127) / 128, 64L, (long)max_split}));
-  s.kc = ((K + s.nsplit - 1) / s.nsplit + 63) / 64 * 64;
+  s.kc = ((K + s.nsplit - 1) / s.nsplit + rows4 - 1) / rows4 * rows4;  // whole chunks a wavefront
   s.nsplit = std::max(1, (K + s.kc - 1) / s.kc);
   return s;
 }
@@ -952,36 +952,21 @@ int gemm_tn_ws(pw_ctx* c, int K, int n1, int n2, const T* A, int lda, const T* B
   const int g = (int)std::min<long>((total + 255) / 256, 4096);
   T* P = nullptr;
   int nsplit = 0;
+  const TnShape s = tn_shape<T>(K, n1, n2, 1, pl.tn_cap, max_split, sizeof(T) == 4 && split >= 2 ? 128 : 64);
+  nsplit = s.nsplit;
+  if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
+  P = (T*)(ws ? ws : c->d_gemm_ws);
   bool done = false;
   if constexpr (sizeof(T) == 4) {
-    // the split kernels load float pairs: K, lda and ldb even
-    if ((split == 2 || split == 3) && !(K & 1) && !(lda & 1) && !(ldb & 1)) {
-      // outputs of 256 or more 64 x 64 tiles (1024 x 1024 and up) take
-      // 128 x 128 tiles
-      const int tm = pl.tn_tm > 0 ? pl.tn_tm : (((n1 + BM - 1) / BM) * ((n2 + BN - 1) / BN) >= 256 ? 2 : 1);
-      const int tiles = ((n1 + BM * tm - 1) / (BM * tm)) * ((n2 + BN * tm - 1) / (BN * tm));
-      // about 1024 partial workgroups, but at most 256 K-splits for one or two
-      // output tiles: the reduction then reads 256 partials per entry, not
-      // ~1000
-      const int cap = pl.tn_cap > 0 ? pl.tn_cap : (tiles <= 2 ? 256 : 1024);
-      nsplit = std::max(1, std::min({(cap + tiles - 1) / tiles, (K + 255) / 256, max_split}));
-      const int kc = ((K + nsplit - 1) / nsplit + BK - 1) / BK * BK;
-      nsplit = (K + kc - 1) / kc;
-      if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
-      P = (T*)(ws ? ws : c->d_gemm_ws);
-      const size_t ldsb = sizeof(unsigned short) * 2 * split * (size_t)(BM * tm) * BKP;
-      const auto kern = split == 3 ? (tm == 2 ? k_gemm_tn_partial_bf<2, 3> : k_gemm_tn_partial_bf<1, 3>)
-                                   : (tm == 2 ? k_gemm_tn_partial_bf<2, 2> : k_gemm_tn_partial_bf<1, 2>);
-      PW_TRY(ensure_lds((const void*)kern, ldsb));
-      hipLaunchKernelGGL(kern, dim3(tiles * nsplit), dim3(256), ldsb, c->stream, A, lda, B, ldb, K, n1, n2, kc, P);
+    if (split == 2 || split == 3) {
+      const auto kern = split == 3 ? tn_kernel_bf<3>(s.ni, s.nj) : tn_kernel_bf<2>(s.ni, s.nj);
+      PW_TRY(ensure_lds((const void*)kern, s.lds));
+      hipLaunchKernelGGL(kern, dim3(s.tiles * nsplit), dim3(256), s.lds, c->stream, A, lda, B, ldb, K, n1, n2, s.kc,
+                         P);
       done = true;
     }
   }
   if (!done) {
-    const TnShape s = tn_shape<T>(K, n1, n2, 1, pl.tn_cap, max_split);
-    nsplit = s.nsplit;
-    if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
-    P = (T*)(ws ? ws : c->d_gemm_ws);
     const auto kern = tn_kernel<T>(s.ni, s.nj);
     PW_TRY(ensure_lds((const void*)kern, s.lds));
     hipLaunchKernelGGL(kern, dim3(s.tiles * nsplit), dim3(256), s.lds, c->stream, A, lda, B, ldb, K, n1, n2, s.kc, P,

@@ -334,8 +334,7 @@ struct pw_ctx {
   //   mm, reg: the matrix-core slab kernel, else the register-FFT one where
   //   compiled (PW_SLAB=lds: the LDS kernel); cg / rp / threads: the LDS kernel's y column groups (0 = two
   //   y buffers), x row pairs per step, threads per workgroup (0 = the
-  //   built-in rule; PW_SLAB=lds:<cg>:<rp>:<threads>); tn_tm / tn_cap: the
-  //   split-BF16 split-K TN product's tile (1: 64 x 64, 2: 128 x 128) and the
+  //   built-in rule; PW_SLAB=lds:<cg>:<rp>:<threads>); tn_cap: the
   //   number of partial workgroups a TN product aims at (0 = the built-in rule)
   struct Plan {
     bool reg = true;
@@ -343,7 +342,7 @@ struct pw_ctx {
     bool mm_only = false;  // ... and wherever the context has its plan (the autotuner's choice)
     int ly = 0;  // register kernel: lanes per y column transform (0: one)
     int cg = 0, rp = 0, threads = 0;
-    int tn_tm = 0, tn_cap = 0;
+    int tn_cap = 0;
   } plan[2];
   hipStream_t gstream = nullptr;
   hipEvent_t gev[2] = {nullptr, nullptr};

@@ -6,7 +6,7 @@
 // its plans with FFTW_MEASURE (src/SCF/fourier.cpp:62, 112-184), i.e. it
 // times candidate algorithms for each transform shape once and keeps the
 // fastest.  pw_autotune plays that part for this library's transforms and
-// products; pw_batch_autotune does it for the batched persistent launch's
+// products; pw_batch_autotune does it for the batched call's
 // work split.
 //
 // Cache file: one line per tuned shape, "<key> <choice...>", keys made of the
@@ -146,7 +146,7 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
   const std::string base = device_tag(c->device) + "|" + std::to_string(c->n1) + "x" + std::to_string(c->n2) + "x" +
                            std::to_string(c->n3) + "|npw" + std::to_string(c->npw) + "|nb" + std::to_string(nb) +
                            (dtype == PW_F64 ? "|f64" : "|f32");
-  const std::string kslab = base + "|slab", ktn = base + "|tn-reg" + std::to_string(c->nbeta);
+  const std::string kslab = base + "|slab", ktn = base + "|tn-cap" + std::to_string(c->nbeta);
   auto cache = read_cache(cache_path);
   std::string out;
   // blocks to time on (deterministic content)
@@ -218,12 +218,11 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
   }
   // ---- projector product W = beta^T X: split-K tiling ----
   if (c->nbeta > 0) {
-    int tm = 0, cap = 0;
+    int cap = 0;
     auto jt = cache.find(ktn);
-    if (jt != cache.end() && sscanf(jt->second.c_str(), "%d %d", &tm, &cap) == 2 && tm >= 0 && tm <= 2 && cap > 0) {
-      pl.tn_tm = tm;
+    if (jt != cache.end() && sscanf(jt->second.c_str(), "%d", &cap) == 1 && cap > 0) {
       pl.tn_cap = cap;
-      out += "; tn " + std::to_string(tm) + " " + std::to_string(cap) + " (cached)";
+      out += "; tn " + std::to_string(cap) + " (cached)";
     } else {
       if (hipMalloc(&W, es * (size_t)c->nbeta * nb) != hipSuccess)
         return done(fail(PW_ERR_NOMEM, "pw_autotune: cannot allocate the projection block"));
@@ -231,7 +230,6 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
       double tbest = 1e30;
       int bcap = 256;
       for (int cp : {128, 256, 512, 1024}) {
-        pl.tn_tm = 0;
         pl.tn_cap = cp;
         double ms = 0;
         int rc;
@@ -250,11 +248,10 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
           bcap = cp;
         }
       }
-      pl.tn_tm = 0;
       pl.tn_cap = bcap;
-      append_cache(cache_path, ktn, "0 " + std::to_string(bcap));
+      append_cache(cache_path, ktn, std::to_string(bcap));
       char b[96];
-      snprintf(b, sizeof(b), "; tn 0 %d (%.4f ms)", bcap, tbest);
+      snprintf(b, sizeof(b), "; tn %d (%.4f ms)", bcap, tbest);
       out += b;
     }
   }
