@@ -68,6 +68,7 @@ struct pw_batch {
   hipEvent_t gev[2] = {nullptr, nullptr};
   hipGraphExec_t gexec = nullptr;
   long gkey = -1, gwarm = -1;
+  long gepoch = 0;  // epochs() at the capture
   unsigned long long* d_stamps = nullptr;  // stage timing: [cell][5 kMaxDegree]
   int stamp_steps = 0;
 };
@@ -78,6 +79,15 @@ static void drop_graph(pw_batch* b) {
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   b->gexec = nullptr;
   b->gkey = b->gwarm = -1;
+}
+
+// Sum of the cells' epochs: another value than at the capture means that a
+// buffer the graph's nodes point to has moved (a product of another shape grew
+// a cell's partial sums, say), and the graph must not run again.
+static long epochs(const pw_batch* b) {
+  long n = 0;
+  for (const pw_ctx* c : b->ctx) n += c->epoch;
+  return n;
 }
 
 // Cells onto lanes: the largest first, each to the lane with the least work.
@@ -165,10 +175,12 @@ static int batch_steps(pw_batch* b, int degree) {
   float2* HX = degree == 0 ? b->d_HY : nullptr;
   if (b->d_stamps) b->stamp_steps = std::max(degree, 1);
   if (!b->use_graphs || b->d_stamps) return batch_body(b, b->stream, b->d_X, HX, degree);
+  if (b->gexec && b->gepoch != epochs(b)) drop_graph(b);
   if (b->gexec && b->gkey == degree) return batch_replay(b);
   if (b->gwarm != degree) {
-    b->gwarm = degree;
-    return batch_body(b, b->stream, b->d_X, HX, degree);
+    const int rc = batch_body(b, b->stream, b->d_X, HX, degree);
+    b->gwarm = rc == PW_OK ? degree : -1;  // (a failed call may have left buffers unsized)
+    return rc;
   }
   if (!b->gstream) PW_HIP(hipStreamCreateWithFlags(&b->gstream, hipStreamNonBlocking));
   for (auto& e : b->gev)
@@ -188,8 +200,12 @@ static int batch_steps(pw_batch* b, int degree) {
       rc = fail(PW_ERR_HIP, "batch: hipGraphInstantiate failed");
   }
   if (g) (void)hipGraphDestroy(g);
-  if (rc != PW_OK) return rc;
+  if (rc != PW_OK) {
+    b->gwarm = -1;
+    return rc;
+  }
   b->gkey = degree;
+  b->gepoch = epochs(b);
   return batch_replay(b);
 }
 

@@ -954,7 +954,10 @@ int gemm_tn_ws(pw_ctx* c, int K, int n1, int n2, const T* A, int lda, const T* B
   int nsplit = 0;
   const TnShape s = tn_shape<T>(K, n1, n2, 1, pl.tn_cap, max_split, sizeof(T) == 4 && split >= 2 ? 128 : 64);
   nsplit = s.nsplit;
-  if (!ws) PW_TRY(grow_gemm_ws(c, per_split * nsplit));
+  // The buffer is sized by the shape, not by the kind of product: the native
+  // product's 64-row splits are at least as many as the 128-row ones, and a
+  // filter and an H X of the same bands then never move it under each other.
+  if (!ws) PW_TRY(grow_gemm_ws(c, per_split * tn_shape<T>(K, n1, n2, 1, pl.tn_cap, max_split, 64).nsplit));
   P = (T*)(ws ? ws : c->d_gemm_ws);
   bool done = false;
   if constexpr (sizeof(T) == 4) {

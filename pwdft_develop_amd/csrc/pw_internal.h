@@ -348,6 +348,7 @@ struct pw_ctx {
   hipEvent_t gev[2] = {nullptr, nullptr};
   hipGraphExec_t fg_exec = nullptr;
   long fg_key = -1, fg_warm = -1;
+  long epoch = 0;  // counts invalidate_graph: a graph captured elsewhere (a batch's) holds for one value of it
   void* fg_result = nullptr;
   hipGraphExec_t lz_exec = nullptr;  // Lanczos steps, keyed by their count
   long lz_key = -1, lz_warm = -1;
@@ -364,6 +365,10 @@ struct pw_ctx {
 namespace pw {
 // A captured filter graph holds raw device pointers and the shape of the
 // operator (potential, projectors, exchange): it is dropped whenever any of
-// them is reallocated or switched on or off.
-inline void invalidate_graph(pw_ctx* c) { c->fg_key = c->fg_warm = c->lz_key = c->lz_warm = -1; }
+// them is reallocated or switched on or off.  A batch's graph holds the
+// pointers of all its contexts and compares their epochs.
+inline void invalidate_graph(pw_ctx* c) {
+  c->fg_key = c->fg_warm = c->lz_key = c->lz_warm = -1;
+  c->epoch++;
+}
 }  // namespace pw

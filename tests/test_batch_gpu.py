@@ -106,6 +106,35 @@ def test_batch_graph_replays_match_eager(cells):
     B.close()
 
 
+def test_batch_graph_after_other_calls(cells):
+    """H X between replays of a filter's graph: at these shapes its native
+    projector product splits K more often (52 and 53 times) than the filter's
+    split-BF16 one (39 and 44), whose partial sums' buffer the graph's nodes
+    hold.  Filter, filter (captured), H X, filter, and the other way round,
+    each equal to the eager result bit for bit."""
+    import torch
+    from pwdft_develop_amd.ops import Batch
+    side = np.pi / np.sqrt(80.0)
+    sub = []
+    for n, natom, nb in ((54, 16, 77), (64, 32, 128)):
+        atoms = np.random.default_rng(natom).uniform(0, n * side * 0.99, (natom, 3))
+        sub.append(W.Problem(f"cell{n}", (n, n, n), np.eye(3) * n * side * 0.99, 10.0, atoms, nb).build())
+    print("case: batch graph after other calls " + str([(c.npw, c.nbeta, c.nb) for c in sub]), flush=True)
+    bounds = np.array([_bounds(c) for c in sub])
+    E = Batch(sub)
+    E.set_graphs(False)
+    X0 = E.to_device([c.psi for c in sub])
+    F = E.cheb_filter(X0.clone(), 3, bounds)
+    H = E.apply_h(X0)
+    E.close()
+    for order in ("ffhfhff", "hhfhffhh"):
+        B = Batch(sub)
+        for c in order:
+            got = B.apply_h(X0) if c == "h" else B.cheb_filter(X0.clone(), 3, bounds)
+            assert torch.equal(got, H if c == "h" else F), (order, c)
+        B.close()
+
+
 @pytest.mark.parametrize("rp,zc,nwg", [(5, 1, 0), (7, 3, 96), (0, 0, 256)])
 def test_batch_tuning_knobs(cells, rp, zc, nwg):
     """The autotuner's knobs (x row pairs per slab job, stick chunks per z
