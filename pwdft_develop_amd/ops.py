@@ -74,6 +74,8 @@ class Context:
         assert x.is_contiguous() and x.dim() == 2 and x.shape[1] == self.prob.npw
         if out is None:
             out = t.zeros_like(x) if zero_out else t.empty_like(x)
+            if zero_out:
+                self._after_current(x, out)
         check(getattr(_lib.lib(), name)(self.h, _dtype_code(x), x.shape[0], C.c_void_p(x.data_ptr()),
                                         C.c_void_p(out.data_ptr())))
         return out
@@ -170,12 +172,13 @@ class Context:
         v = np.ascontiguousarray(np.asarray(vtot, dtype=np.float64).reshape(-1))
         check(_lib.lib().pw_set_vtot(self.h, v))
 
-    def _after_current(self, v):
-        """Work of the context's stream on v comes after what made v."""
+    def _after_current(self, *tensors):
+        """Work of the context's stream on these comes after what made them."""
         cur = self.torch.cuda.current_stream(self.device)
         if cur != self.stream:
             self.stream.wait_stream(cur)
-            v.record_stream(self.stream)
+            for v in tensors:
+                v.record_stream(self.stream)
 
     def set_atoms(self, pos):
         """Rebuild the Gaussian projector block at new atom positions (same
@@ -189,7 +192,10 @@ class Context:
     def density(self, x, f, out=None, accumulate=False):
         t = self.torch
         if out is None:
-            out = t.zeros(int(np.prod(self.prob.grid)), dtype=t.float64, device=self.device)
+            # (written whole unless accumulated to)
+            make = t.zeros if accumulate else t.empty
+            out = make(int(np.prod(self.prob.grid)), dtype=t.float64, device=self.device)
+        self._after_current(x, out)
         check(_lib.lib().pw_density(self.h, _dtype_code(x), x.shape[0], C.c_void_p(x.data_ptr()),
                                     np.ascontiguousarray(f, np.float64), C.c_void_p(out.data_ptr()),
                                     1 if accumulate else 0))
@@ -237,6 +243,7 @@ class Context:
 
     def nonlocal_force(self, x, f, natom, npa):
         F = np.zeros(3 * natom)
+        self._after_current(x)
         check(_lib.lib().pw_nonlocal_force(self.h, _dtype_code(x), x.shape[0], C.c_void_p(x.data_ptr()),
                                            np.ascontiguousarray(f, np.float64), natom, npa, F))
         return F.reshape(natom, 3)

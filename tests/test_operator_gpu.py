@@ -90,3 +90,78 @@ def test_density_tiles(grid, nb):
         ctx.density(X, f, out=rho, accumulate=True)
         assert _rel(rho.cpu().numpy(), 2 * ref) < 256 * eps
     ctx.close()
+
+
+def _busy():
+    """Some 20 ms of work on the current stream."""
+    import torch
+    a = torch.full((4096, 4096), 1.0 / 4096, device="cuda")
+    for _ in range(20):
+        a = a @ a
+    return a
+
+
+@pytest.mark.parametrize("current", ["null", "other"])
+def test_density_force_exchange_on_a_stream_of_their_own(current):
+    """A context with its own stream, while the current stream is busy: blocks
+    just made there (psi, an accumulated density) are waited for, and no fill
+    of an output queued there lands on a result."""
+    import torch
+    from pwdft_develop_amd.ops import Context
+    print(f"case: density and force, own stream, current {current}", flush=True)
+    prob = _problem((32, 30, 24), 5, natom=3)
+    f = np.linspace(0.5, 2.0, 5)
+    ref = Context(prob)
+    X = ref.to_device(prob.psi)
+    rho, F = ref.density(X, f), ref.nonlocal_force(X, f, 3, 4)
+    twice = ref.density(X, f, out=rho.clone(), accumulate=True)
+    ref.set_exx(prob.ecut, 0.2, 0.25, X[:2].contiguous(), np.ones(2))
+    V = ref.add_exx(X)
+    torch.cuda.synchronize()
+    ctx = Context(prob, stream=torch.cuda.Stream())
+    ctx.set_exx(prob.ecut, 0.2, 0.25, X[:2].contiguous(), np.ones(2))
+    torch.cuda.synchronize()
+    keep = []
+    cur = torch.cuda.Stream() if current == "other" else torch.cuda.default_stream()
+    with torch.cuda.stream(cur):
+        keep.append(_busy())
+        got = ctx.density(X, f)
+        assert torch.equal(got, rho)
+        keep.append(_busy())
+        acc = ctx.density(X * 1.0, f, out=rho * 1.0, accumulate=True)
+        assert torch.equal(acc, twice)
+        keep.append(_busy())
+        assert np.array_equal(ctx.nonlocal_force(X * 1.0, f, 3, 4), F)
+        keep.append(_busy())
+        vx = ctx.add_exx(X * 1.0)
+        torch.cuda.synchronize()
+        assert torch.equal(vx, V)
+    ctx.close()
+    ref.close()
+
+
+def test_band_energy_gradient_on_a_stream_of_its_own():
+    """E, dE/dV and dE/dR of a context with its own stream, the default stream
+    busy before each: equal to those of a context on the default stream."""
+    import torch
+    from pwdft_develop_amd.adjoint import band_energy
+    from pwdft_develop_amd.ops import Context
+    print("case: band-energy gradient, own stream", flush=True)
+    prob = _problem((24, 30, 25), 4, natom=3)
+    f = np.linspace(0.5, 2.0, 4)
+    out = []
+    for stream in (None, torch.cuda.Stream()):
+        ctx = Context(prob, stream=stream)
+        X = ctx.to_device(prob.psi)
+        torch.cuda.synchronize()
+        a = _busy()
+        V = (torch.from_numpy(prob.vtot).cuda() * 0.5).requires_grad_(True)
+        R = torch.from_numpy(np.array(prob.atoms)).cuda().requires_grad_(True)
+        E = band_energy(V, R, ctx, X, f)
+        a = _busy() + a
+        E.backward()
+        torch.cuda.synchronize()
+        out.append((E.detach().clone(), V.grad.clone(), R.grad.clone()))
+        ctx.close()
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
