@@ -1267,6 +1267,13 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
   }
   PW_HIP(hipStreamSynchronize(rs->stream));
   free_nonlocal(rs);
+  // (without projectors the whole of V is the forward transform's factor)
+  auto none = [&](int code) {
+    free_nonlocal(rs);
+    (void)hipGetLastError();  // a refused allocation's
+    (void)forward_factors(rs);
+    return code;
+  };
   int rc;
   if ((rc = upload_rs(&rs->d_atab, atab.data(), atab.size())) != PW_OK ||
       (rc = upload_rs(&rs->d_apt_off, apt_off.data(), apt_off.size())) != PW_OK ||
@@ -1276,15 +1283,11 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
       (rc = upload_rs(&rs->d_rowptr, rowptr.data(), rowptr.size())) != PW_OK ||
       (rc = upload_rs(&rs->d_ent, ent.data(), ent.size())) != PW_OK ||
       (rc = upload_rs(&rs->d_clist, clist.data(), clist.size())) != PW_OK ||
-      (rc = upload_rs(&rs->d_pts, pts.data(), pts.size())) != PW_OK) {
-    free_nonlocal(rs);
-    return rc;
-  }
+      (rc = upload_rs(&rs->d_pts, pts.data(), pts.size())) != PW_OK)
+    return none(rc);
   if (tot_proj > 0 &&
-      hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * rs->chunk * kNlSplits) != hipSuccess) {
-    free_nonlocal(rs);
-    return fail(PW_ERR_NOMEM, "pw_rs_set_nonlocal: cannot allocate projector weights");
-  }
+      hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * rs->chunk * kNlSplits) != hipSuccess)
+    return none(fail(PW_ERR_NOMEM, "pw_rs_set_nonlocal: cannot allocate projector weights"));
   rs->natom = natom;
   rs->nproj_tot = tot_proj;
   rs->npmax = npmax;

@@ -53,3 +53,27 @@ def test_matrix_core_transforms_against_oracle(grid, fine, natom, nb):
     R.check(lib.pw_rs_set_vtot(ctx.h, p.vtot))
     assert np.array_equal(ctx.mult_spinor(x).cpu().numpy(), got)
     ctx.close()
+
+
+def test_refused_projectors_leave_the_potential():
+    """Projector weights of more bytes than any card has (atoms without points,
+    32 projectors each) are refused, and the handle then has no projectors:
+    the whole of V psi, also on the old ones' points."""
+    import torch
+    p = _problem((12, 12, 12), (24, 24, 24), 2, 3)
+    x = torch.from_numpy(p.psi).cuda()
+    bare = R.RealSpaceContext(p, nonlocal_=False)
+    want = bare.mult_spinor(x)
+    ctx = R.RealSpaceContext(p, max_bands=1 << 20)
+    print(f"case: refused projectors, chunk {ctx.info()['chunk']}", flush=True)
+    assert not torch.equal(ctx.mult_spinor(x), want)
+    natom = (1 << 42) // (8 * 32 * ctx.info()["chunk"])  # 4 TiB and more
+    zero = np.zeros(natom, np.int32)
+    with pytest.raises(RuntimeError, match="cannot allocate"):
+        ctx.set_nonlocal(zero, zero + 32, np.zeros(0, np.int32), np.zeros(0), np.zeros(32 * natom))
+    assert torch.equal(ctx.mult_spinor(x), want)
+    ctx.set_nonlocal(p.npts, p.nproj, p.idx, p.val, p.wgt)
+    ref = O.rs_mult_spinor(p.grid, p.grid_fine, p.volume, p.ekin, p.vtot, p.npts, p.nproj, p.idx, p.val, p.wgt, p.psi)
+    assert np.abs(ctx.mult_spinor(x).cpu().numpy() - ref).max() < 512 * 2.0 ** -53 * np.abs(ref).max()
+    ctx.close()
+    bare.close()
