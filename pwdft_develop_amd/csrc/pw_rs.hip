@@ -1185,6 +1185,21 @@ extern "C" int pw_rs_set_vtot(pw_rs* rs, const double* vtot) {
   return forward_factors(rs);
 }
 
+namespace {
+// Bands a k_rs_weights workgroup takes, and splits of an atom's points that
+// bring `blocks` workgroups to about 2048, each with a point per thread at least.
+int weight_bands(int npmax) { return npmax <= 8 ? 8 : npmax <= 16 ? 4 : 2; }
+int point_splits(const pw_rs* rs, long blocks, int cap) {
+  const int most = (rs->ptmax + 255) / 256;
+  return (int)std::max<long>(1, std::min<long>({2048 / std::max<long>(blocks, 1), (long)most, (long)cap}));
+}
+// Splits of the weights' sums for nbc bands (the point-major kernel reads one).
+int weight_splits(const pw_rs* rs, int nbc) {
+  const int BB = weight_bands(rs->npmax);
+  return rs->ncolor > 0 ? point_splits(rs, (long)rs->natom * ((nbc + BB - 1) / BB), kNlSplits) : 1;
+}
+}  // namespace
+
 extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const int* nproj,
                                   const int* idx, const double* val, const double* wgt) {
   if (!rs || natom < 0) return fail(PW_ERR_ARG, "pw_rs_set_nonlocal: bad argument");
@@ -1285,15 +1300,17 @@ extern "C" int pw_rs_set_nonlocal(pw_rs* rs, int natom, const int* npts, const i
       (rc = upload_rs(&rs->d_clist, clist.data(), clist.size())) != PW_OK ||
       (rc = upload_rs(&rs->d_pts, pts.data(), pts.size())) != PW_OK)
     return none(rc);
-  if (tot_proj > 0 &&
-      hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * rs->chunk * kNlSplits) != hipSuccess)
-    return none(fail(PW_ERR_NOMEM, "pw_rs_set_nonlocal: cannot allocate projector weights"));
   rs->natom = natom;
   rs->nproj_tot = tot_proj;
   rs->npmax = npmax;
   rs->ptmax = natom > 0 ? *std::max_element(npts, npts + natom) : 0;
   rs->ncolor = ncolor;
   rs->color_off = color_off;
+  // one value per split, projector and band: few bands come in more splits
+  size_t cols = 1;
+  for (int b = 1; b <= rs->chunk; b++) cols = std::max(cols, (size_t)b * weight_splits(rs, b));
+  if (tot_proj > 0 && hipMalloc((void**)&rs->d_coef, sizeof(double) * (size_t)tot_proj * cols) != hipSuccess)
+    return none(fail(PW_ERR_NOMEM, "pw_rs_set_nonlocal: cannot allocate projector weights"));
   return forward_factors(rs);
 }
 
@@ -1530,19 +1547,11 @@ int own_to_coarse(pw_rs* rs, const double* fine, const double* vloc, double* a3,
 int local_terms(pw_rs* rs, int nbc, const double** vloc) {
   const bool nl = rs->natom > 0 && rs->nproj_tot > 0;
   *vloc = !nl || rs->ncolor > 0 ? rs->d_vfwd : nullptr;
-  // splits of an atom's points that bring `blocks` workgroups to about 2048,
-  // each with a point per thread at least
-  const int most = (rs->ptmax + 255) / 256;
-  auto splits = [&](long blocks, int cap) {
-    return (int)std::max<long>(1, std::min<long>({2048 / std::max<long>(blocks, 1), (long)most, (long)cap}));
-  };
   const long ldc = (long)rs->nproj_tot * nbc;
-  int nsplit = 1;
+  const int nsplit = nl ? weight_splits(rs, nbc) : 1;
   if (nl) {
     const double scale = rs->vol / (double)rs->Nf;
-    const int BB = rs->npmax <= 8 ? 8 : rs->npmax <= 16 ? 4 : 2, groups = (nbc + BB - 1) / BB;
-    // (the point-major kernel reads one split)
-    if (rs->ncolor > 0) nsplit = splits((long)rs->natom * groups, kNlSplits);
+    const int BB = weight_bands(rs->npmax), groups = (nbc + BB - 1) / BB;
     const dim3 g(rs->natom, groups, nsplit);
 #define RS_LAUNCH(NP, B)                                                                                            \
   hipLaunchKernelGGL((k_rs_weights<NP, B>), g, dim3(256), 0, rs->stream, rs->d_pf, rs->d_atab, rs->d_apt_off,       \
@@ -1558,7 +1567,7 @@ int local_terms(pw_rs* rs, int nbc, const double** vloc) {
       const int na = rs->color_off[c + 1] - rs->color_off[c];
       const int* cl = rs->d_clist + rs->color_off[c];
       const int groups = (nbc + kNlBands - 1) / kNlBands;
-      const dim3 g(na, groups, splits((long)na * groups, most));
+      const dim3 g(na, groups, point_splits(rs, (long)na * groups, 2048));
 #define RS_LAUNCH(NP)                                                                                          \
   hipLaunchKernelGGL(k_rs_nl_apply<NP>, g, dim3(256), 0, rs->stream, rs->d_pf, cl, rs->d_atab, rs->d_apt_off,  \
                      rs->d_pts, rs->d_vtot, rs->d_val, rs->d_coef, nsplit, ldc, nbc, rs->Nf)

@@ -77,3 +77,20 @@ def test_refused_projectors_leave_the_potential():
     assert np.abs(ctx.mult_spinor(x).cpu().numpy() - ref).max() < 512 * 2.0 ** -53 * np.abs(ref).max()
     ctx.close()
     bare.close()
+
+
+def test_projector_weights_take_one_split_of_many_atoms():
+    """48 GiB of projector weights at one value per projector and band (atoms
+    too many to split their points) are accepted: several splits of them would
+    exceed the card.  No atom has points here, so H psi is the bare one."""
+    import torch
+    p = _problem((12, 12, 12), (24, 24, 24), 2, 3)
+    x = torch.from_numpy(p.psi).cuda()
+    ctx = R.RealSpaceContext(p, max_bands=1 << 20, nonlocal_=False)
+    want = ctx.mult_spinor(x)
+    natom = (48 << 30) // (8 * 32 * ctx.info()["chunk"])
+    print(f"case: many projectors, chunk {ctx.info()['chunk']} natom {natom}", flush=True)
+    zero = np.zeros(natom, np.int32)
+    ctx.set_nonlocal(zero, zero + 32, np.zeros(0, np.int32), np.zeros(0), np.zeros(32 * natom))
+    assert torch.equal(ctx.mult_spinor(x), want)
+    ctx.close()
