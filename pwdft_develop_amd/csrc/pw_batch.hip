@@ -62,7 +62,7 @@ struct pw_batch {
   float2 *d_X = nullptr, *d_Y[3] = {nullptr, nullptr, nullptr}, *d_HY = nullptr;
   float* d_coef = nullptr;                // [cell][3 kMaxDegree]
   std::vector<float> h_coef;
-  int rp_force = 0, zc_force = 0, nwg_force = 0;
+  int nwg_force = 0;
   bool use_graphs = true;
   hipStream_t gstream = nullptr;
   hipEvent_t gev[2] = {nullptr, nullptr};
@@ -311,8 +311,6 @@ extern "C" int pw_batch_info(const pw_batch* b, long* xtotal, int* njobs, int* n
 
 extern "C" int pw_batch_tune(pw_batch* b, int rp, int zc, int nwg) {
   if (!b || rp < 0 || zc < 0 || nwg < 0) return fail(PW_ERR_ARG, "pw_batch_tune: bad argument");
-  b->rp_force = rp;
-  b->zc_force = zc;
   b->nwg_force = nwg;
   return batch_plan(b);
 }
@@ -395,9 +393,8 @@ extern "C" int pw_batch_set_stream(pw_batch* b, void* stream) {
 
 // Autotuner of the batched launch (see pw_tune.cpp for the single-cell
 // plans): the number of lanes, timed on the batch's own H X over every cell;
-// the fastest is kept and recorded in cache_path under a key of the device and
-// the batch's shapes (the two zeros of a line stand where other choices once
-// did; such lines are read for their lanes alone).
+// the fastest is kept and recorded in cache_path ("<key> <lanes>") under a key
+// of the device and the batch's shapes.
 extern "C" int pw_batch_autotune(pw_batch* b, const char* cache_path, char* summary, int len) {
   if (!b) return fail(PW_ERR_ARG, "null batch");
   std::string key;
@@ -414,28 +411,24 @@ extern "C" int pw_batch_autotune(pw_batch* b, const char* cache_path, char* summ
     for (int v : b->shapes) h = (h ^ (unsigned long)v) * 1099511628211UL;
     char hb[32];
     snprintf(hb, sizeof(hb), "%016lx", h);
-    key = dev + "|batch" + std::to_string(b->ncell) + "|" + hb;
+    key = dev + "|batch" + std::to_string(b->ncell) + "|" + hb + "|lanes";
   }
   if (cache_path) {
     FILE* f = fopen(cache_path, "r");
     if (f) {
       char line[512];
-      int r = 0, z = 0, n = 0, found = 0;
+      int n = 0;
       while (fgets(line, sizeof(line), f)) {
         char k[400];
-        int r2, z2, n2;
-        if (sscanf(line, "%399s %d %d %d", k, &r2, &z2, &n2) == 4 && key == k) {
-          r = r2; z = z2; n = n2; found = 1;
-        }
+        int lanes;
+        if (sscanf(line, "%399s %d", k, &lanes) == 2 && key == k && lanes >= 1 && lanes <= kMaxLanes) n = lanes;
       }
       fclose(f);
-      if (found) {
-        b->rp_force = r;
-        b->zc_force = z;
+      if (n > 0) {
         b->nwg_force = n;
         PW_TRY(batch_plan(b));
         char s[160];
-        snprintf(s, sizeof(s), "batch rp %d zc %d nwg %d (cached)", r, z, n);
+        snprintf(s, sizeof(s), "batch lanes %d (cached)", n);
         if (summary && len > 0) snprintf(summary, (size_t)len, "%s", s);
         return PW_OK;
       }
@@ -457,6 +450,7 @@ extern "C" int pw_batch_autotune(pw_batch* b, const char* cache_path, char* summ
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
     return done(fail(PW_ERR_HIP, "pw_batch_autotune: event creation failed"));
   double tbest = 1e30;
+  const int was = b->nwg_force;
   int bn = 0, tried = 0;
   int rc = PW_OK;
   for (int lanes : {1, 2, 3, 4, 6, 8}) {
@@ -482,19 +476,18 @@ extern "C" int pw_batch_autotune(pw_batch* b, const char* cache_path, char* summ
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  if (rc != PW_OK) return done(rc);
-  b->rp_force = b->zc_force = 0;
-  b->nwg_force = bn;
-  PW_TRY(batch_plan(b));
+  b->nwg_force = rc == PW_OK ? bn : was;
+  const int rp = batch_plan(b);  // (the lanes of before where timing failed)
+  if (rc != PW_OK || rp != PW_OK) return done(rc != PW_OK ? rc : rp);
   if (cache_path) {
     FILE* f = fopen(cache_path, "a");
     if (f) {
-      fprintf(f, "%s 0 0 %d\n", key.c_str(), bn);
+      fprintf(f, "%s %d\n", key.c_str(), bn);
       fclose(f);
     }
   }
   char s[200];
-  snprintf(s, sizeof(s), "batch rp 0 zc 0 nwg %d (%.3f ms H X over %d layouts)", bn, tbest, tried);
+  snprintf(s, sizeof(s), "batch lanes %d (%.3f ms H X over %d layouts)", bn, tbest, tried);
   if (summary && len > 0) snprintf(summary, (size_t)len, "%s", s);
   return done(PW_OK);
 }

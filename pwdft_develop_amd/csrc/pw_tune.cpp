@@ -11,7 +11,9 @@
 //
 // Cache file: one line per tuned shape, "<key> <choice...>", keys made of the
 // device name and CU count, grid, sphere size, band count, precision and the
-// stage ("slab" or "tn<nbeta>").  Lines are appended; the last line of a key
+// stage ("xy": the slab kernel, "tn-cap<nbeta>").  A stage whose choices
+// change gets a new name, so that lines made among other choices are not read
+// ("slab" lines know no matrix-core kernel, "tn" lines a tile shape).  Lines are appended; the last line of a key
 // wins.  A shape found in the cache is applied without timing.
 #include <hip/hip_runtime.h>
 
@@ -113,8 +115,7 @@ static void apply_slab(pw_ctx::Plan& pl, const SlabChoice& ch) {
   pl.threads = lds ? ch.threads : 0;
 }
 
-// A line of the cache ("reg <ly> <n>": files written with other band groups
-// of the register kernel in the second number are read as that kernel).
+// A line of the cache.
 static bool parse_slab(const std::string& v, SlabChoice* ch) {
   int cg = 0, rp = 0, th = 0, ly = 0, sb = 0;
   if (v == "mm") {
@@ -146,7 +147,7 @@ extern "C" int pw_autotune(pw_ctx* c, int dtype, int nb, const char* cache_path,
   const std::string base = device_tag(c->device) + "|" + std::to_string(c->n1) + "x" + std::to_string(c->n2) + "x" +
                            std::to_string(c->n3) + "|npw" + std::to_string(c->npw) + "|nb" + std::to_string(nb) +
                            (dtype == PW_F64 ? "|f64" : "|f32");
-  const std::string kslab = base + "|slab", ktn = base + "|tn-cap" + std::to_string(c->nbeta);
+  const std::string kslab = base + "|xy", ktn = base + "|tn-cap" + std::to_string(c->nbeta);
   auto cache = read_cache(cache_path);
   std::string out;
   // blocks to time on (deterministic content)

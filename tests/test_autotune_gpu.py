@@ -36,3 +36,20 @@ def test_autotune_keeps_parity_and_caches(name, nb, tmp_path):
         ctx2.close()
     lines = open(cache).read().splitlines()
     assert len(lines) == 4 and all("|" + f"{prob.grid[0]}x" in l for l in lines)
+
+
+@pytest.mark.parametrize("value", ["reg 1 0", "reg 1 8 p", "lds 0 4 256"])
+def test_slab_lines_of_other_choices_are_not_read(value, tmp_path):
+    """A "slab" line, written by a tuner that knew no matrix-core kernel, does
+    not keep a context from it: the slab is timed anew."""
+    import torch
+    from pwdft_develop_amd.ops import Context
+    print(f"case: old cache line {value}", flush=True)
+    prob = W.si8_32(nb=8).build()
+    cache = tmp_path / "tune.txt"
+    ctx = Context(prob)
+    ctx.autotune(8, torch.complex64, str(cache))
+    key, stage = cache.read_text().split()[0].rsplit("|", 1)
+    cache.write_text(f"{key}|slab {value}\n")
+    assert stage == "xy" and "(cached)" not in ctx.autotune(8, torch.complex64, str(cache))
+    ctx.close()

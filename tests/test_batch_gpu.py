@@ -178,3 +178,21 @@ def test_batch_autotune_and_cache(cells, tmp_path):
     import torch
     assert torch.equal(B2.apply_h(X), H1)
     B2.close()
+
+
+@pytest.mark.parametrize("line", ["{old} 5 1 512", "{old} 0 0 4", "{key} 17", "{key} 0"])
+def test_batch_cache_lines_of_other_choices(cells, tmp_path, line):
+    """Lines of the persistent grid's knobs (row pairs, z chunks, workgroups)
+    and lane counts out of range are not taken for lanes."""
+    from pwdft_develop_amd.ops import Batch
+    sub = cells[:3]
+    cache = tmp_path / "tune.txt"
+    B = Batch(sub)
+    B.autotune(str(cache))
+    key = cache.read_text().split()[0]
+    line = line.format(key=key, old=key.removesuffix("|lanes"))
+    print(f"case: batch cache line {line}", flush=True)
+    cache.write_text(line + "\n")
+    assert "cached" not in B.autotune(str(cache))
+    assert 1 <= B.info()["workgroups"] <= len(sub)
+    B.close()
