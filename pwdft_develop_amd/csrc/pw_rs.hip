@@ -629,7 +629,9 @@ __global__ __launch_bounds__(256) void k_rs_x_c2r(const double2* __restrict__ in
       if (k >= 0) {
         const double sg = e < hw ? 1.0 : -1.0;
         const double2 a0 = r0[k], a1 = r1[k];
-        z = make_double2(a0.x - sg * a1.y, sg * a0.y + a1.x);
+        // a row's own Nyquist entry counts by its real part alone (IP_c2f leaves
+        // that column without its mirror where x is not refined and y or z is)
+        z = 2 * e == n ? make_double2(a0.x, a1.x) : make_double2(a0.x - sg * a1.y, sg * a0.y + a1.x);
       }
     }
     vt[it] = z;

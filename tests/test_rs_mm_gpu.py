@@ -27,7 +27,9 @@ def _problem(grid, fine, natom, nb):
     ((12, 14, 16), (24, 28, 32), 2, 1), ((16, 16, 16), (16, 16, 16), 3, 2), ((30, 32, 18), (60, 64, 36), 9, 5),
     ((62, 12, 16), (124, 24, 32), 4, 3), ((12, 62, 20), (24, 126, 40), 1, 6), ((16, 20, 62), (24, 34, 124), 0, 2),
     ((12, 16, 20), (24, 32, 20), 1, 6), ((12, 16, 20), (24, 16, 40), 1, 2),
-    ((34, 34, 14), (68, 68, 28), 12, 9), ((64, 12, 12), (128, 24, 24), 3, 2)])
+    ((34, 34, 14), (68, 68, 28), 12, 9), ((64, 12, 12), (128, 24, 24), 3, 2),
+    ((12, 16, 20), (12, 32, 40), 2, 3), ((64, 12, 14), (64, 24, 28), 2, 3), ((64, 12, 14), (64, 24, 14), 1, 2),
+    ((12, 64, 14), (12, 64, 28), 2, 1), ((16, 64, 12), (32, 64, 24), 1, 2), ((14, 12, 64), (28, 24, 64), 2, 3)])
 def test_matrix_core_transforms_against_oracle(grid, fine, natom, nb):
     import torch
     print(f"case: real-space transforms {grid} / {fine} natom={natom} nb={nb}", flush=True)
