@@ -645,6 +645,11 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
       // "reg[:<ly>...]": the transforms held in registers (on matrix cores or
       // as register FFTs with ly lanes per y column), as by default
       if (sl && std::string(sl).compare(0, 4, "reg:") == 0) pl.ly = std::max(1, atoi(sl + 4));
+      // "fft[:<ly>]": the register FFTs alone
+      if (sl && std::string(sl).compare(0, 3, "fft") == 0) {
+        pl.mm = false;
+        if (sl[3] == ':') pl.ly = std::max(1, atoi(sl + 4));
+      }
       // "lds:<g>[:<r>]": the LDS kernel with its large-plane layout, g y
       // columns per group (and r x row pairs per step)
       if (sl && std::string(sl).compare(0, 4, "lds:") == 0) {

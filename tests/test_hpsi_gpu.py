@@ -54,9 +54,9 @@ def test_apply_h_fp32(ctx8, si8):
 
 @pytest.mark.parametrize("name,nb", [("si8_32", 13), ("rand16_48", 8), ("si64_60", 24)])
 def test_fp32_register_slab_kernel(name, nb, monkeypatch):
-    """The FP32 register slab kernel (one z plane of 8 bands per workgroup,
-    ragged last group) against the oracle and against the LDS slab kernel
-    (same arithmetic; agreement to FP32 rounding)."""
+    """The default FP32 slab kernel (on matrix cores at these sizes; ragged band
+    groups) against the oracle and against the LDS slab kernel (agreement to
+    FP32 rounding)."""
     import torch
     from pwdft_develop_amd.ops import Context
     prob = W.WORKLOADS[name](nb=nb).build()
@@ -77,9 +77,9 @@ def test_fp32_register_slab_kernel(name, nb, monkeypatch):
 
 @pytest.mark.parametrize("name,nb", [("si8_32", 13), ("rand16_48", 21), ("si64_60", 40)])
 def test_fp32_wide_register_slab_kernel(name, nb, monkeypatch):
-    """The 16-band, 512-thread FP32 register slab variant (PW_SLAB=reg:1:16;
-    ragged last group) against the oracle and against the 8-band kernel
-    (same arithmetic)."""
+    """PW_SLAB=reg:1:16 (once a 16-band variant, now the register-held
+    transforms as by default) is still taken: against the oracle and equal to
+    the default."""
     import torch
     from pwdft_develop_amd.ops import Context
     prob = W.WORKLOADS[name](nb=nb).build()
@@ -100,12 +100,10 @@ def test_fp32_wide_register_slab_kernel(name, nb, monkeypatch):
 
 @pytest.mark.parametrize("name,nb", [("si8_32", 13), ("rand16_48", 21), ("si64_60", 5), ("si64_60", 203)])
 def test_fp32_persistent_register_slab_kernel(name, nb, monkeypatch):
-    """The FP32 register slab kernel on a persistent grid (PW_SLAB=reg:1:8:p:
-    one workgroup per resident slot, looping over (plane, band group) items
-    with the next item's sticks and V plane prefetched; 203 bands at 60
-    points give several items per workgroup and a ragged last group)
-    against the oracle and against the one-item grid (same arithmetic).
-    FP64 has no persistent variant and keeps the one-item kernel."""
+    """PW_SLAB=reg:1:8:p (once a persistent grid of the register kernel, now
+    the default's) is still taken: against the oracle and equal to
+    PW_SLAB=reg:1:8; 203 bands at 60 points give several items per workgroup of
+    the matrix-core kernel and a ragged last group."""
     import torch
     from pwdft_develop_amd.ops import Context
     prob = W.WORKLOADS[name](nb=nb).build()
@@ -128,6 +126,39 @@ def test_fp32_persistent_register_slab_kernel(name, nb, monkeypatch):
         assert _rel(a64, ref) < 1e-12
     cp.close()
     c1.close()
+
+
+@pytest.mark.parametrize("ly", [1, 2, 4])
+@pytest.mark.parametrize("n,nb", [(24, 3), (30, 9), (32, 13), (36, 4), (40, 17), (48, 8), (60, 5), (64, 3), (72, 9)])
+def test_register_fft_slab_kernels(n, nb, ly, monkeypatch):
+    """The register-FFT slab kernel of every compiled plane (PW_SLAB=fft:<ly>:
+    ly lanes per y column, 4 where 4 divides n; 8 bands a workgroup in FP32, 4
+    in FP64, ragged last groups) against the oracle; it is another kernel than
+    the default, so not every bit agrees with that.
+
+    Tolerance: two radix-2/3/5 transforms of n and two of 24 points, and the
+    pointwise V, at most 12 passes of a few roundings each: 64 eps of max
+    |H psi|."""
+    import torch
+    from pwdft_develop_amd.ops import Context
+    if ly == 4 and n % 4:
+        pytest.skip("four lanes need a multiple of 4")
+    print(f"case: register FFT slab n={n} nb={nb} ly={ly}", flush=True)
+    sides = np.array([n, n, 24]) * np.pi / np.sqrt(80.0) * 0.99
+    prob = W.Problem("fft", (n, n, 24), np.diag(sides), 10.0, np.array([[0.1, 0.2, 0.3]]) * sides, nb).build()
+    ref = O.Hamiltonian(prob).mult_spinor(prob.psi)
+    monkeypatch.setenv("PW_SLAB", f"fft:{ly}")
+    cf = Context(prob)
+    monkeypatch.setenv("PW_SLAB", "mm")
+    cm = Context(prob)
+    monkeypatch.delenv("PW_SLAB")
+    for dt, eps in ((torch.complex128, 2.0 ** -53), (torch.complex64, 2.0 ** -24)):
+        X = cf.to_device(prob.psi, dt)
+        a = cf.mult_spinor(X).cpu().numpy()
+        assert _rel(a, ref) < 64 * eps
+        assert not np.array_equal(a, cm.mult_spinor(X).cpu().numpy())
+    cf.close()
+    cm.close()
 
 
 @pytest.mark.parametrize("name,nb", [("si8_32", 13), ("rand16_48", 5), ("si64_60", 9)])
@@ -156,9 +187,8 @@ def test_register_z_kernels(name, nb, monkeypatch):
 
 @pytest.mark.parametrize("name,nb", [("si8_32", 32), ("si8_32", 7), ("rand16_48", 9), ("si64_60", 5)])
 def test_fp64_register_slab_kernel(name, nb, monkeypatch):
-    """The FP64 register slab kernel (one z plane of 4 bands per workgroup,
-    ragged last group; one wave per SIMD at 60 points) against the oracle
-    (FP64 parity) and against the LDS slab kernel (same arithmetic)."""
+    """The default FP64 slab kernel (on matrix cores at these sizes; ragged band
+    groups) against the oracle (FP64 parity) and against the LDS slab kernel."""
     from pwdft_develop_amd.ops import Context
     prob = W.WORKLOADS[name](nb=nb).build()
     print(f"case: {name} fp64 slab kernels nb={nb}", flush=True)
