@@ -668,10 +668,13 @@ struct ExxRegKernels {
 template <typename T>
 static ExxRegKernels<T> exx_reg_kernels(int n1, int n2) {
   ExxRegKernels<T> k;
-  // The register kernels wherever the plane has one; us for 32 x 32 pairs, LDS
-  // / register kernels: 96 x 96 x 40 FP32 4732 / 2465, FP64 7938 / 6655; 48^3
-  // 1115 / 634, 2305 / 1387; 30^3 330 / 236, 451 / 395; 24^3 246 / 149, 309 /
-  // 207.  PW_EXX_PAIR (for comparisons): "lds" both LDS kernels, "fwd" the
+  // The register kernels wherever the plane has one.  us for 32 x 32 pairs (72
+  // and 96 points: 16 x 16) on 24 planes, LDS / register kernels:
+  //   FP32 24: 236 / 140  32: 301 / 177  40: 457 / 282  48: 615 / 344
+  //        60: 1009 / 523  64: 1280 / 580  72: 569 / 263  96: 768 / 411
+  //   FP64 24: 298 / 199  32: 411 / 272  40: 703 / 423  48: 1081 / 587
+  //        60: 1687 / 1100  64: 1835 / 1272  72: 773 / 547  96: 1429 / 1193
+  // PW_EXX_PAIR (for comparisons): "lds" both LDS kernels, "fwd" the
   // register forward kernel only.
   const char* f = getenv("PW_EXX_PAIR");
   const std::string mode = f ? f : "";

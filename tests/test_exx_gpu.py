@@ -96,10 +96,10 @@ def test_add_exx_forced_grouped_layouts(pair, wfn, monkeypatch):
 def test_register_pair_kernels(name, nb, nocc, monkeypatch):
     """The register-FFT pair kernels (k_exx_pair_fwd_reg / _acc_reg: 4 lanes
     per 1D transform, the accumulator in registers over the occupied bands;
-    PW_EXX_PAIR=reg forces them in FP64 too) against the LDS pair kernels
-    (PW_EXX_PAIR=lds) on square planes of 32, 48 and 96 points, FP64 and
-    FP32; parity of the defaults (FP32 register, FP64 LDS) with the oracle
-    is the other tests'."""
+    the default in both precisions, any PW_EXX_PAIR but "lds" and "fwd") against
+    the LDS pair kernels (PW_EXX_PAIR=lds) on square planes of 32, 48 and 96
+    points, FP64 and FP32; the default's parity with the oracle is the other
+    tests'."""
     import torch
     from pwdft_develop_amd.ops import Context
     prob = W.WORKLOADS[name](nb=nb).build()

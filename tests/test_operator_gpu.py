@@ -73,7 +73,8 @@ def test_device_potential_is_the_host_potential(other_stream):
 @pytest.mark.parametrize("grid,nb", [((24, 24, 24), 1), ((32, 30, 25), 17), ((60, 24, 24), 3), ((45, 64, 24), 5),
                                      ((72, 72, 24), 2), ((144, 24, 24), 3)])
 def test_density_tiles(grid, nb):
-    """(144 points: 36 columns, beyond the matrix-core plan.)  psi(r) passes
+    """(144 points: 36 columns, nine k-steps, beyond the matrix-core density
+    kernel.)  psi(r) passes
     two sums of at most 32 + 32 terms: 64 eps of its largest value, twice that
     of its square, taken as 256 eps of the largest density."""
     import torch
