@@ -1,9 +1,9 @@
-"""Many uneven cells in one persistent launch (pw_batch_*): the 48-cell
+"""Many uneven cells in one call (pw_batch_*): the 48-cell
 workload (grids 24..72 cubed, 2..32 atoms, 16..128 bands) through the
 batched FP32 H*psi and degree-8 Chebyshev filter, each cell against the FP64
 oracle on its first and last band (the filter acts on every band by itself,
 so a band subset is an exact check; the last band sits in each cell's
-ragged last item), the batched filter against the same filter run cell by
+ragged last group), the batched filter against the same filter run cell by
 cell, and graph replays against the eager launch."""
 import numpy as np
 import pytest
@@ -84,7 +84,7 @@ def test_batch_filter_each_cell_and_serial(cells):
 def test_batch_graph_replays_match_eager(cells):
     """First call eager, second captured, then replays: every result equal to
     the eager one bit for bit (each item's arithmetic does not depend on
-    which workgroup takes it), with eager torch work between replays."""
+    which lane takes it), with eager torch work between replays."""
     import torch
     from pwdft_develop_amd.ops import Batch
     print("case: batch48 graph replays", flush=True)
@@ -137,10 +137,10 @@ def test_batch_graph_after_other_calls(cells):
 
 @pytest.mark.parametrize("rp,zc,nwg", [(5, 1, 0), (7, 3, 96), (0, 0, 256)])
 def test_batch_tuning_knobs(cells, rp, zc, nwg):
-    """The autotuner's knobs (x row pairs per slab job, stick chunks per z
-    job, grid size) change the LDS layout and the schedule, not the result:
-    FP32 parity with the oracle on a subset of cells, for H X and a degree-8
-    filter."""
+    """Lane counts (the default, and more than the cells and the most lanes
+    there are) change the schedule, not the result: FP32 parity with the oracle
+    on a subset of cells, for H X and a degree-8 filter.  rp and zc are taken and
+    have no effect."""
     from pwdft_develop_amd.ops import Batch
     print(f"case: batch tune rp={rp} zc={zc} nwg={nwg}", flush=True)
     sub = [cells[i] for i in (0, 5, 11, 17, 23)]
@@ -156,6 +156,24 @@ def test_batch_tuning_knobs(cells, rp, zc, nwg):
     for c, g in zip(sub, B.split(X)):
         ref = O.Hamiltonian(c).cheb_filter(c.psi[[c.nb - 1]], DEGREE, *_bounds(c))
         assert _rel(g[[c.nb - 1]].astype(np.complex128), ref) < 2e-5, c.name
+    B.close()
+
+
+def test_batch_lanes_are_bit_equal(cells):
+    """1, 2, 3 and all lanes, eager, captured and replayed: the same bits."""
+    import torch
+    from pwdft_develop_amd.ops import Batch
+    print("case: batch lanes", flush=True)
+    sub = [cells[i] for i in (0, 5, 11, 17, 23)]
+    B = Batch(sub)
+    X0 = B.to_device([c.psi for c in sub])
+    bounds = np.array([_bounds(c) for c in sub])
+    F = B.cheb_filter(X0.clone(), DEGREE, bounds)
+    for lanes in (1, 2, 3, 5, 9):
+        B.tune(nwg=lanes)
+        assert B.info()["workgroups"] == min(lanes, len(sub))
+        for _ in range(3):
+            assert torch.equal(B.cheb_filter(X0.clone(), DEGREE, bounds), F), lanes
     B.close()
 
 

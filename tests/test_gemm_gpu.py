@@ -1,11 +1,17 @@
 """The projector products on matrix cores at the edges of their tiles: 1 to 64
 atoms' projectors and 2 to 130 bands around multiples of 16 (tiles of 32, 48
 and 64), ragged last rows, K with remainders to 16 and too short for one
-split; FP64 and FP32.
+split; FP64, FP32 and, inside the FP32 filter, products of split BF16 terms;
+every tile shape of the split-K product.
 
 Tolerance: W = w beta^T x sums K products and beta W sums nbeta, in any order
 within (K + nbeta) eps of the sums of the terms' absolute values; the local
-part is within 360 eps of max |H psi| (four chained transforms).
+part is within 360 eps of max |H psi| (four chained transforms).  Rounding
+errors of both signs add up as the root of their number: the 2-norm of the error
+is within 2 eps sqrt(K + nbeta + 360) of that of H psi, where a lost row of K or
+a column in the wrong place would be 1 / sqrt(K) of beta W.  Three BF16 terms
+hold 24 bits and drop products of 2^-27; two hold 18 (operands rounded by 2^-18,
+the product of the small terms dropped): 6 2^-18 more over the two products.
 """
 import numpy as np
 import pytest
@@ -22,7 +28,7 @@ SIDE = np.pi / np.sqrt(80.0)
                                              (24, 0.985, 5, 31), (24, 0.97, 8, 33), (25, 0.99, 12, 48),
                                              (27, 0.98, 13, 49), (30, 0.96, 16, 65), (48, 0.99, 33, 100),
                                              (48, 0.97, 64, 130)])
-def test_projector_products_against_oracle(n, fill, natom, nb):
+def test_projector_products_against_oracle(n, fill, natom, nb, monkeypatch):
     import torch
     from pwdft_develop_amd.ops import Context
     side = n * SIDE * fill
@@ -39,3 +45,56 @@ def test_projector_products_against_oracle(n, fill, natom, nb):
         err = np.abs((got - ref).view(np.float64)).reshape(terms.shape)
         assert (err <= eps * ((beta.shape[1] + prob.nbeta) * terms + 360 * np.abs(ref).max())).all()
     ctx.close()
+    _check_filter_products(prob, ref, monkeypatch)
+
+
+def _norm_bound(prob, ref, eps):
+    return 2 * eps * np.sqrt(2 * prob.npw + prob.nbeta + 360) * np.linalg.norm(ref)
+
+
+def _check_filter_products(prob, ref, monkeypatch):
+    """One step of the FP32 filter, (H - c) psi s, on three and on two BF16
+    terms and on the native product, from H psi = ref."""
+    import torch
+    from pwdft_develop_amd.ops import Context
+    a, b, aL = 0.5, 30.0, -2.0
+    step = O.Hamiltonian(prob).cheb_filter(prob.psi[:1], 1, a, b, aL)
+    c = (a + b) / 2
+    s = np.vdot(ref[0] - c * prob.psi[0], step[0]).real / np.linalg.norm(ref[0] - c * prob.psi[0]) ** 2
+    want = s * (ref - c * prob.psi)
+    assert np.abs(step[0] - want[0]).max() < 1e-12 * np.abs(step).max()
+    for split, loss in (("3", 0.0), ("2", 6 * 2.0 ** -18), ("0", 0.0)):
+        monkeypatch.setenv("PW_BF16", split)
+        ctx = Context(prob, max_bands=prob.nb)
+        X = ctx.cheb_filter(ctx.to_device(prob.psi, torch.complex64), 1, a, b, aL).cpu().numpy()
+        ctx.close()
+        # (H psi's error, and three roundings of the step)
+        bound = abs(s) * (_norm_bound(prob, ref, 2.0 ** -24) + loss * np.linalg.norm(ref)) \
+            + 3 * 2.0 ** -24 * np.linalg.norm(want)
+        err = np.linalg.norm(X - want)
+        print(f"  filter split {split}: {err / bound:.3f} of the bound", flush=True)
+        assert err < bound, split
+    monkeypatch.delenv("PW_BF16")
+
+
+# (atoms of four projectors, bands) for every pair of 2, 3 and 4 16-wide tiles
+# per workgroup: enough rows at 54^3 that none falls back to 32 x 32
+@pytest.mark.parametrize("natom,nb", [(8, 144), (8, 196), (33, 31), (33, 143), (33, 49), (64, 18), (64, 47), (61, 63)])
+def test_tile_shapes_against_oracle(natom, nb, monkeypatch):
+    import torch
+    from pwdft_develop_amd.ops import Context
+    side = 54 * SIDE * 0.99
+    atoms = np.random.default_rng(natom).uniform(0, side, (natom, 3))
+    prob = W.Problem("nl", (54, 54, 54), np.eye(3) * side, 10.0, atoms, nb).build()
+    prob.wgt = 300 * prob.wgt  # beta W leads H psi
+    print(f"case: tile shapes nbeta={prob.nbeta} nb={nb} npw={prob.npw}", flush=True)
+    ref = O.Hamiltonian(prob).apply_h(prob.psi)
+    ctx = Context(prob, max_bands=nb)
+    for dt, eps in ((torch.complex128, 2.0 ** -53), (torch.complex64, 2.0 ** -24)):
+        got = ctx.apply_h(ctx.to_device(prob.psi, dt)).cpu().numpy()
+        err, bound = np.linalg.norm(got - ref), _norm_bound(prob, ref, eps)
+        print(f"  H psi {dt}: {err / bound:.3f} of the bound, nonlocal share "
+              f"{np.linalg.norm(ctx.nonlocal_multx(ctx.to_device(prob.psi)).cpu().numpy()) / np.linalg.norm(ref):.2f}", flush=True)
+        assert err < bound
+    ctx.close()
+    _check_filter_products(prob, ref, monkeypatch)
