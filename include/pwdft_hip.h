@@ -197,6 +197,10 @@ int pw_chebfsi_sweep(pw_ctx* ctx, int mode, int nb, int m, int k,
                      const void* v0, const double* prev_eig, void* X,
                      double* eig, double* res, double* bounds);
 
+/* Frees the eigensolvers' scratch and that of pw_band_energy, pw_density and
+ * pw_nonlocal_force, which is kept at the largest size asked for: one block of
+ * bands for the energy, up to 16 grids for the density, up to 256 MiB of
+ * projector columns for the force. */
 int pw_free_workspace(pw_ctx* ctx);
 
 /* Graph capture of the Chebyshev filter and of the Lanczos steps (default
@@ -347,6 +351,9 @@ int pw_get_timing(pw_ctx* ctx, double* ms4, int* ncalls);
  * The band blocks of all cells live in one device buffer of complex floats
  * (FP32, the PW_F32 layout per cell): cell c's npw[c] x nb[c] block starts
  * at complex offset xoff[c] = sum_{c' < c} npw[c'] nb[c'].
+ * The filter's projector products run on split BF16 terms, as those of
+ * pw_cheb_filter in FP32 (three terms hold FP32's 24 bits; PW_BF16=0 when the
+ * batch is made: FP32 products); pw_batch_apply_h's are FP32.
  * The cells run on lanes (streams) whose kernels overlap; every step of every
  * cell is captured into a hipGraph on the second call of a degree and replayed
  * afterwards.  Calls return after the work has finished. */

@@ -110,9 +110,11 @@ static int batch_plan(pw_batch* b) {
   }
   while ((int)b->lstream.size() < n) {
     hipStream_t s = nullptr;
-    hipEvent_t e = nullptr;
     PW_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     b->lstream.push_back(s);
+  }
+  while ((int)b->ljoin.size() < n) {
+    hipEvent_t e = nullptr;
     PW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     b->ljoin.push_back(e);
   }

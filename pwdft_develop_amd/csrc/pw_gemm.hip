@@ -12,8 +12,9 @@
 //        other terms or forms a Chebyshev step.
 //
 // Both use the 16x16x4 MFMA (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32)
-// on operands in registers, or split-BF16 products on tiles in LDS.  Lane layout of the
-// 16x16x4 MFMA: A operand lane l = (row l%16, k l/16), B operand lane l =
+// on operands in registers, or products of split BF16 terms: in registers
+// (TN, and NN on an operand split ahead of time) or on tiles in LDS (NN on
+// operands that are not).  Lane layout of the 16x16x4 MFMA: A operand lane l = (row l%16, k l/16), B operand lane l =
 // (k l/16, col l%16).  Accumulator lane l register i holds column l%16 and
 // row 4(l/16)+i for the FP32 MFMA but row 4i + l/16 for the FP64 one
 // (checked on gfx950 with a known 16x16x4 product).
@@ -1062,8 +1063,8 @@ int gemm_nn_ep(pw_ctx* c, int m, int n, int k, const T* A, int lda, const T* B, 
   return PW_OK;
 }
 
-// A (m x k, column-major, ld lda) split ahead of time into *out (the tile
-// layout of k_gemm_nn_pre; allocated here, freed by the caller).
+// A (m x k, column-major, ld lda) split ahead of time into the caller's
+// split_a_bytes(m, k) bytes at out (the tile layout of k_gemm_nn_pre).
 size_t split_a_bytes(int m, int k) {
   return sizeof(unsigned short) * (size_t)((m + 15) / 16) * ((k + 31) / 32) * kSplitTerms * 512;
 }

@@ -705,7 +705,6 @@ extern "C" int pw_ctx_create(pw_ctx** out, const int grid[3], const double super
     }
   }
   build_stick_plan(c, idx);
-  c->h_idx.assign(idx, idx + npw);
   c->f1 = radix_plan(c->n1);
   c->f2 = radix_plan(c->n2);
   c->f3 = radix_plan(c->n3);
@@ -855,12 +854,14 @@ static int mark(pw_ctx* c, int k) {
   return PW_OK;
 }
 
-// LDS bytes of k_slab_xy: twiddles, y-space (two copies when cg == 0, one
-// plus a cg-column scratch shared with the x rows otherwise), x rows.
+// LDS bytes of the z kernels: twiddles and two buffers of sticks.
 template <typename T>
 static size_t z_lds(const pw_ctx* c) {
   return sizeof(typename cx<T>::t) * (c->n3 + 2 * (size_t)kStickChunk * z_ld<T>(c->n3));
 }
+
+// LDS bytes of k_slab_xy: twiddles, y-space (two copies when cg == 0, one
+// plus a cg-column scratch shared with the x rows otherwise), x rows.
 static size_t slab_lds(const pw_ctx* c, int esz, int rp, int cg) {
   const size_t nk = c->sp.kxmax + 1, n1 = c->n1, n2 = c->n2;
   if (cg == 0) return esz * (n1 + n2 + 2 * nk * n2 + 2 * (size_t)rp * n1);
@@ -1064,7 +1065,6 @@ template int sticks_to_sphere_add<float>(pw_ctx*, int, const void*, void*);
 template <typename T>
 static int nonlocal(pw_ctx* c, int nb, const void* X, void* Y, bool accumulate) {
   const int m = 2 * c->npw;
-  const T one = 1, zero = 0, b2 = accumulate ? (T)1 : (T)0;
   if (c->nbeta == 0) {
     if (!accumulate) PW_HIP(hipMemsetAsync(Y, 0, sizeof(T) * (size_t)m * nb, c->stream));
     return PW_OK;
@@ -1072,11 +1072,9 @@ static int nonlocal(pw_ctx* c, int nb, const void* X, void* Y, bool accumulate) 
   const T* beta = (const T*)(sizeof(T) == 8 ? (const void*)c->d_beta : (const void*)c->d_beta_f);
   const T* betaw = (const T*)(sizeof(T) == 8 ? (const void*)c->d_betaw : (const void*)c->d_betaw_f);
   T* W = (T*)(sizeof(T) == 8 ? (void*)c->d_W : (void*)c->d_W_f);
-  PW_TRY(gemm_tn<T>(c, m, c->nbeta, nb, beta, m, (const T*)X, m, W, c->nbeta, nullptr, zero));
+  PW_TRY(gemm_tn<T>(c, m, c->nbeta, nb, beta, m, (const T*)X, m, W, c->nbeta, nullptr, (T)0));
   if (!accumulate) PW_HIP(hipMemsetAsync(Y, 0, sizeof(T) * (size_t)m * nb, c->stream));
   // Y += (beta w) W on the MFMA kernel (FP64 / FP32)
-  (void)one;
-  (void)b2;
   PW_TRY(gemm_nn_ep<T>(c, m, nb, c->nbeta, betaw, m, W, c->nbeta, (const T*)Y, nullptr, nullptr, (T*)Y, m, nullptr,
                        0, false));
   return PW_OK;

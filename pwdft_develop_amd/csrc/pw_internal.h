@@ -100,12 +100,6 @@ std::vector<int> radix_plan(int n);
 // so a graph capture (which always follows an eager call) never makes it.
 int ensure_lds(const void* kern, size_t bytes);
 
-// A device buffer owned by the context.
-struct DevBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-};
-
 constexpr int kStickChunk = 16;  // sticks a workgroup of the z kernels takes
 
 // Stick decomposition of the half sphere: the distinct (kx, ky) columns of
@@ -274,7 +268,6 @@ struct pw_ctx {
   double supercell[9], recip[9];
   int npw, npad, max_bands;
   pw::StickPlan sp;
-  std::vector<int> h_idx;       // idxCoarseCut, host copy
   std::vector<int> f1, f2, f3;  // radix plans
   // device arrays (d_pt_idx ... d_tw32 lie in d_tables)
   void* d_tables = nullptr;
@@ -332,10 +325,11 @@ struct pw_ctx {
   bool zreg = false;  // PW_ZREG=1: the register z kernels where the z length has one
   // Plans per precision ([PW_F64], [PW_F32]), set by PW_SLAB or pw_autotune:
   //   mm, reg: the matrix-core slab kernel, else the register-FFT one where
-  //   compiled (PW_SLAB=lds: the LDS kernel); cg / rp / threads: the LDS kernel's y column groups (0 = two
-  //   y buffers), x row pairs per step, threads per workgroup (0 = the
-  //   built-in rule; PW_SLAB=lds:<cg>:<rp>:<threads>); tn_cap: the
-  //   number of partial workgroups a TN product aims at (0 = the built-in rule)
+  //   compiled (PW_SLAB=fft[:<ly>]: that one, PW_SLAB=lds: the LDS kernel);
+  //   cg / rp / threads: the LDS kernel's y column groups (0 = two y buffers),
+  //   x row pairs per step, threads per workgroup (0 = the built-in rule;
+  //   PW_SLAB=lds:<cg>:<rp>:<threads>); tn_cap: the number of partial
+  //   workgroups a TN product aims at (0 = the built-in rule)
   struct Plan {
     bool reg = true;
     bool mm = true;        // the matrix-core slab kernel where it wins

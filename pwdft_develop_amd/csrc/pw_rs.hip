@@ -1091,7 +1091,8 @@ extern "C" int pw_rs_create(pw_rs** out, const int grid[3], const int grid_fine[
   }
   rs->vol = vol;
   rs->stream = (hipStream_t)stream;
-  // bands per chunk: chunk buffers within about 8 GiB of the 288 GB HBM
+  // bands per chunk: chunk buffers within 8 GiB of the 288 GB HBM, counted as
+  // the LDS path's (the matrix-core one has no d_cw and d_tf and stays below)
   const double hc = rs->hc0, ny = grid[1] + 1, nz = grid[2] + 1;
   const double per_band = 48.0 * rs->Hc + 16.0 * rs->Nf +
                           16.0 * hc * ((double)grid_fine[2] * ny + (double)grid_fine[2] * grid_fine[1] + nz * ny);
