@@ -1153,12 +1153,16 @@ static int adjoint_ws(pw_ctx* c, size_t bytes) {
 }
 static size_t pad256(size_t b) { return (b + 255) / 256 * 256; }
 
-// Host occupations into that scratch.  A blocking copy, and on the null stream
-// rather than the context's: it returns when the null stream's earlier work is
-// done, and callers whose context has a stream of its own have their blocks
-// (psi, an accumulated rho) made there.
-static int upload_occ(double* d, const double* f, int nb) {
-  PW_HIP(hipMemcpy(d, f, sizeof(double) * nb, hipMemcpyHostToDevice));
+// Host occupations into that scratch, after the null stream's earlier work:
+// callers whose context has a stream of its own have their blocks (psi, an
+// accumulated rho) made there, and the blocking copy, which runs on it, waits for
+// them.  A context on the null stream is in order already (a band-energy gradient
+// at 48^3: 505 us with blocking copies there, 467 without).
+static int upload_occ(pw_ctx* c, double* d, const double* f, int nb) {
+  if (c->stream)
+    PW_HIP(hipMemcpy(d, f, sizeof(double) * nb, hipMemcpyHostToDevice));
+  else
+    PW_HIP(hipMemcpyAsync(d, f, sizeof(double) * nb, hipMemcpyHostToDevice, c->stream));
   return PW_OK;
 }
 
@@ -1173,7 +1177,7 @@ static int density_impl(pw_ctx* c, int nb, const void* psi, const double* f, dou
   PW_TRY(adjoint_ws(c, fb + sizeof(double) * N * nsplit));
   double* df = (double*)c->d_adj_ws;
   double* part = (double*)((unsigned char*)c->d_adj_ws + fb);
-  PW_TRY(upload_occ(df, f, nb));
+  PW_TRY(upload_occ(c, df, f, nb));
   PW_TRY(sphere_to_sticks<T>(c, nb, psi, c->d_t1));
   if (mm > 0) {
     PW_TRY(mm_density<T>(c, nb, c->d_t1, df, nsplit, part));
@@ -1310,7 +1314,7 @@ static int nonlocal_force_impl(pw_ctx* c, int nb, const void* X, const double* f
   unsigned char* ws = (unsigned char*)c->d_adj_ws;
   double *dfv = (double*)ws, *dF = (double*)(ws + fb);
   T *dP = (T*)(ws + fb + Fb), *dB = (T*)(ws + fb + Fb + Pb);
-  PW_TRY(upload_occ(dfv, f, nb));
+  PW_TRY(upload_occ(c, dfv, f, nb));
   GVectors v;
   for (int i = 0; i < 9; i++) v.recip[i] = c->recip[i];
   v.n1 = c->n1; v.n2 = c->n2; v.n3 = c->n3; v.h1 = c->h1; v.npw = npw;
