@@ -868,49 +868,31 @@ static size_t slab_lds(const pw_ctx* c, int esz, int rp, int cg) {
   return esz * (n1 + n2 + nk * n2 + std::max((size_t)cg * n2, 2 * (size_t)rp * n1));
 }
 
-// Whether the matrix-core slab kernel is the faster one for nb bands; it is
-// against the LDS kernel (no register FFT for the plane) on every plane tried:
-// 45 x 45 FP32 207 -> 47 us, FP64 259 -> 81 us at 256 bands.  Against the
-// register FFT (us at 256 / 32 / 8 bands, FFT -> matrix cores):
-//   FP32 24: 19 -> 15 / - / 16 -> 7      FP64 38 -> 22 / - / 17 -> 8
-//        32: 24 -> 27 / 17 -> 9 / 17 -> 8     66 -> 44 / 18 -> 11 / 18 -> 10
-//        36: 30 -> 35 / 17 -> 12 / 17 -> 9    83 -> 55 / 22 -> 16 / 18 -> 11
-//        40: 40 -> 42                        103 -> 69
-//        48: 58 -> 49 / 22 -> 13 / 20 -> 10  141 -> 82 / 29 -> 20 / 22 -> 12
-//        60: 94 -> 71 / 26 -> 17 / 24 -> 11  348 -> 124 / 54 -> 26 / 28 -> 14
-//        64: 201 -> 117                      438 -> 209
-//        72: 309 -> 250 / 72 -> 51 / 39 -> 22   655 -> 675 / 117 -> 125 / 41 -> 46
-// The quarter plane is padded to 16-row tiles: 32..40 points (17..21 rows)
-// pay most for it, which only FP32 with the whole chip busy loses, and at 72
-// FP64 points (37 rows, 18 columns) one wave per SIMD holds the tiles.
+// The LDS slab kernel's layout for nb bands: y columns per group (0: two y
+// buffers), x row pairs per step, threads, LDS bytes.
+struct LdsLayout {
+  int cg, rp, threads;
+  size_t lds;
+  bool few;  // chosen for one or two bands
+};
 template <typename T>
-static bool mm_wins(const pw_ctx* c, int nb) {
-  if (!slab_reg_kernel<T>(c->n1, c->n2)) return true;
-  if (sizeof(T) == 4) return !(c->n1 >= 32 && c->n1 <= 40 && (long)nb * c->n3 >= 5000);
-  return c->n1 < 72;
-}
-
-template <typename T>
-static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
-  typedef typename cx<T>::t C;
-  const int esz = sizeof(C);
-  const T* tw = (const T*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32);
-  const C* tw1 = (const C*)tw;
-  const C* tw2 = tw1 + c->n1;
-  const C* tw3 = tw2 + c->n2;
-  const T* vt = (const T*)(sizeof(T) == 8 ? (const void*)c->d_vtot : (const void*)c->d_vtot_f);
-  const T* ek = (const T*)(sizeof(T) == 8 ? (const void*)c->d_ekin : (const void*)c->d_ekin_f);
-  C* t1 = (C*)c->d_t1;
-  C* t2 = (C*)c->d_t2;
-  // x-pass row-pair chunk: as many pairs as fit next to the y buffers in 64 KiB
+static LdsLayout lds_layout(const pw_ctx* c, int nb, bool few_ok) {
+  const int esz = sizeof(typename cx<T>::t), nk = c->sp.kxmax + 1, npair = (c->n2 + 1) / 2;
   const pw_ctx::Plan& pl = c->plan[sizeof(T) == 8 ? PW_F64 : PW_F32];
+  // one or two bands (the Lanczos steps): all y columns in one group and all x
+  // row pairs in one step at 512 threads spreads each plane's transforms over
+  // the workgroup, where the register kernel leaves most of its threads idle
+  // (si64_60, one band: FP32 13.6 us against 24.0, FP64 15.7 against 29.3)
+  if (few_ok && nb <= 2 && slab_lds(c, esz, npair, nk) <= 160 * 1024)
+    return LdsLayout{nk, npair, 512, slab_lds(c, esz, npair, nk), true};
+  // x-pass row-pair chunk: as many pairs as fit next to the y buffers in 64 KiB
   int rp = 8, cg = 0;
   while (rp > 1 && slab_lds(c, esz, rp, 0) > 64 * 1024) rp /= 2;
   if (pl.cg == 0 && pl.rp > 0) {
     // double-buffered layout with a chosen row-pair count (the autotuner's)
-    rp = std::min(pl.rp, (c->n2 + 1) / 2);
+    rp = std::min(pl.rp, npair);
   } else if (pl.cg > 0) {
-    cg = std::min(c->sp.kxmax + 1, pl.cg);
+    cg = std::min(nk, pl.cg);
     if (pl.rp > 0) rp = pl.rp;
   } else if (slab_lds(c, esz, rp, 0) > 64 * 1024) {
     // large planes: the double-buffered layout would hold one workgroup per
@@ -918,12 +900,11 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
     // scratch (the x rows' space) instead: one group of all columns when it
     // fits, else the most row pairs (<= 8) that leave room for two
     // workgroups per CU, else for one.
-    const int nk = c->sp.kxmax + 1;
     bool found = false;
     // first choice: all nk columns in one group (the scratch is a second y
     // buffer) and as many x row pairs as that scratch holds (FP32 180 x 180,
     // 22 row pairs: 13.1 ms; 16: 13.3; 8-column groups with 4 row pairs: 14.8)
-    const int r = std::max(1, std::min((c->n2 + 1) / 2, nk * c->n2 / (2 * c->n1)));
+    const int r = std::max(1, std::min(npair, nk * c->n2 / (2 * c->n1)));
     if (slab_lds(c, esz, r, nk) <= 160 * 1024) {
       rp = r;
       cg = nk;
@@ -940,22 +921,82 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
     }
     if (!found) { rp = 1; cg = 1; }
   }
+  const size_t lds = slab_lds(c, esz, rp, cg);
+  // large planes (one or two workgroups per CU): more waves per workgroup
+  // to cover the LDS latency of the transform passes
+  // (180 x 180 planes, 1024 bands: 1024 threads 15.0 / 33.3 ms FP32 / FP64,
+  // 256 threads 18.9 / 43.2 ms)
+  const int threads = pl.threads > 0 ? pl.threads : cg > 0 ? (lds > 80 * 1024 ? 1024 : 512) : 256;
+  return LdsLayout{cg, rp, threads, lds, false};
+}
+
+// The LDS kernel's time, as mm_slab_us: its transform steps, each of which the
+// workgroup waits for, and its work, per round of the workgroups that the CUs
+// hold at once.
+template <typename T>
+static double lds_slab_us(const pw_ctx* c, int nb) {
+  const LdsLayout l = lds_layout<T>(c, nb, true);
+  const int nk = c->sp.kxmax + 1, npair = (c->n2 + 1) / 2;
+  const double p1 = (double)c->f1.size(), p2 = (double)c->f2.size();
+  const int groups = l.cg == 0 ? 1 : (nk + l.cg - 1) / l.cg, xsteps = (npair + l.rp - 1) / l.rp;
+  const double steps = 2 * groups * p2 + xsteps * (2 * p1 + 3);
+  const double work = 2.0 * nk * c->n2 * p2 + 2.0 * npair * c->n1 * p1, planes = (double)nb * c->n3;
+  const int per_cu = std::max(1, std::min((int)(160 * 1024 / l.lds), 2048 / l.threads));
+  const double r = planes / (256.0 * per_cu), rounds = r < 4 ? std::ceil(r) : r;
+  return sizeof(T) == 4 ? rounds * (0.318 * steps + 0.100 * work / l.threads) + 0.098e-3 * planes / 256 * work
+                        : rounds * (0.347 * steps + 0.108 * work / l.threads) + 0.166e-3 * planes / 256 * work;
+}
+
+// Whether the matrix-core slab kernel is the faster one for nb bands.
+// Up to 16 columns it is, but for some of the planes with a register FFT (us at
+// 256 / 32 / 8 bands, FFT -> matrix cores):
+//   FP32 24: 19 -> 15 / - / 16 -> 7      FP64 38 -> 22 / - / 17 -> 8
+//        32: 24 -> 27 / 17 -> 9 / 17 -> 8     66 -> 44 / 18 -> 11 / 18 -> 10
+//        36: 30 -> 35 / 17 -> 12 / 17 -> 9    83 -> 55 / 22 -> 16 / 18 -> 11
+//        40: 40 -> 42                        103 -> 69
+//        48: 58 -> 49 / 22 -> 13 / 20 -> 10  141 -> 82 / 29 -> 20 / 22 -> 12
+//        60: 94 -> 71 / 26 -> 17 / 24 -> 11  348 -> 124 / 54 -> 26 / 28 -> 14
+//        64: 201 -> 117                      438 -> 209
+//        72: 309 -> 250 / 72 -> 51 / 39 -> 22   655 -> 675 / 117 -> 125 / 41 -> 46
+//            (FP32, one band: LDS kernel 19, matrix cores 24)
+// The quarter plane is padded to 16-row tiles: 32..40 points (17..21 rows)
+// pay most for it, which only FP32 with the whole chip busy loses, and at 72
+// FP64 points (37 rows, 18 columns) one wave per SIMD holds the tiles.
+// Beyond 16 columns the LDS kernel can be the faster one, above all where the
+// axes differ: both are padded to the longer one's columns, and a short y axis
+// leaves few wavefronts a plane (us at 24 bands of 24 planes, LDS / matrix
+// cores, FP32: 180 x 24 40 / 109, 180 x 45 82 / 86, 180 x 90 203 / 118, 45 x 180
+// 87 / 105, 120 x 120 323 / 47; FP64 108 x 24 40 / 92, 108 x 60 120 / 76), and for
+// one or two bands (FP64 75 x 75 27 / 44, 96 x 96 36 / 26).  The two estimates
+// decide; fitted to 11084 pairs of timings (831 grids of 12 to 225 points an axis,
+// 1 to 200 bands), they leave 1.0 % on average to the faster of the two in FP32,
+// 0.6 % in FP64, and more than 5 % in 434 of 7020 and 150 of 4064; matrix cores
+// wherever they can run left up to a factor of 6.8.
+template <typename T>
+static bool mm_wins(const pw_ctx* c, int nb) {
+  if (!slab_reg_kernel<T>(c->n1, c->n2))
+    return mm_ksteps(c) <= 4 || mm_slab_us<T>(c, nb) < 0.95 * lds_slab_us<T>(c, nb);
+  if (sizeof(T) == 8) return c->n1 < 72;
+  return !(c->n1 >= 32 && c->n1 <= 40 && (long)nb * c->n3 >= 5000) && !(c->n1 >= 72 && nb <= 2);
+}
+
+template <typename T>
+static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
+  typedef typename cx<T>::t C;
+  const T* tw = (const T*)(sizeof(T) == 8 ? (const void*)c->d_tw64 : (const void*)c->d_tw32);
+  const C* tw1 = (const C*)tw;
+  const C* tw2 = tw1 + c->n1;
+  const C* tw3 = tw2 + c->n2;
+  const T* vt = (const T*)(sizeof(T) == 8 ? (const void*)c->d_vtot : (const void*)c->d_vtot_f);
+  const T* ek = (const T*)(sizeof(T) == 8 ? (const void*)c->d_ekin : (const void*)c->d_ekin_f);
+  C* t1 = (C*)c->d_t1;
+  C* t2 = (C*)c->d_t2;
+  const pw_ctx::Plan& pl = c->plan[sizeof(T) == 8 ? PW_F64 : PW_F32];
   const bool mm = pl.mm && mm_slab_ready<T>(c) && (pl.mm_only || mm_wins<T>(c, nb));
-  // one or two bands (the Lanczos steps) where the plane has no matrix-core
-  // kernel: the LDS kernel with all y columns in one group and all x row
-  // pairs in one step at 512 threads spreads each plane's transforms over the
-  // workgroup, where the register kernel leaves most of its threads idle
-  // (si64_60, one band: FP32 13.6 us against 24.0, FP64 15.7 against 29.3)
-  const int nkc = c->sp.kxmax + 1, npr = (c->n2 + 1) / 2;
-  const bool few = !mm && nb <= 2 && slab_lds(c, esz, npr, nkc) <= 160 * 1024;
-  if (few) {
-    cg = nkc;
-    rp = npr;
-  }
-  const size_t lds2 = slab_lds(c, esz, rp, cg);
-  const slab_reg_fn<T> kreg = pl.reg && !few ? slab_reg_kernel<T>(c->n1, c->n2, pl.ly) : nullptr;
-  if (lds2 > 160 * 1024)
-    return fail(PW_ERR_UNSUPPORTED, "H*psi slab needs %zu bytes of LDS (> 160 KiB)", lds2);
+  const LdsLayout ll = lds_layout<T>(c, nb, !mm);
+  const slab_reg_fn<T> kreg = pl.reg && !ll.few ? slab_reg_kernel<T>(c->n1, c->n2, pl.ly) : nullptr;
+  if (ll.lds > 160 * 1024)
+    return fail(PW_ERR_UNSUPPORTED, "H*psi slab needs %zu bytes of LDS (> 160 KiB)", ll.lds);
   PW_TRY(mark(c, 0));
   PW_TRY(launch_inv_z<T>(c, nb, (const C*)psi, t1, tw3));
   PW_TRY(mark(c, 1));
@@ -971,16 +1012,9 @@ static int local_kinetic(pw_ctx* c, int nb, const void* psi, void* a3) {
                        c->sp.nstick, c->sp.kxmax, nb, c->d_pos, c->d_mpos, (const T*)vt);
   } else {
     auto kslab = slab_kernel<T>(c->n1, c->n2);
-    PW_TRY(ensure_lds((const void*)kslab, lds2));
-    // large planes (one or two workgroups per CU): more waves per workgroup
-    // to cover the LDS latency of the transform passes
-    // (180 x 180 planes, 1024 bands: 1024 threads 15.0 / 33.3 ms FP32 / FP64,
-    // 256 threads 18.9 / 43.2 ms)
-    int threads = cg > 0 ? (lds2 > 80 * 1024 ? 1024 : 512) : 256;
-    if (pl.threads > 0) threads = pl.threads;
-    if (few) threads = 512;
-    hipLaunchKernelGGL(kslab, dim3(c->n3, nb), dim3(threads), lds2, c->stream, (const C*)t1, t2, c->n1,
-                       c->n2, c->n3, c->sp.nstick, c->sp.kxmax, c->d_pos, c->d_mpos, vt, tw1, tw2, rp, cg);
+    PW_TRY(ensure_lds((const void*)kslab, ll.lds));
+    hipLaunchKernelGGL(kslab, dim3(c->n3, nb), dim3(ll.threads), ll.lds, c->stream, (const C*)t1, t2, c->n1,
+                       c->n2, c->n3, c->sp.nstick, c->sp.kxmax, c->d_pos, c->d_mpos, vt, tw1, tw2, ll.rp, ll.cg);
   }
   PW_HIP(hipGetLastError());
   PW_TRY(mark(c, 2));

@@ -231,6 +231,10 @@ template <typename T>
 bool mm_slab_ready(const pw_ctx* c);
 template <typename T>
 int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2);
+// k-steps (of four columns) of the plan, 0 without one; estimated us of a launch.
+int mm_ksteps(const pw_ctx* c);
+template <typename T>
+double mm_slab_us(const pw_ctx* c, int nb);
 // part[split] (N doubles each) = sum over the split's bands of f r^2 / N from
 // the sticks t1; splits: how many, 0 where the context has no plan.
 int mm_density_splits(const pw_ctx* c, int nb);

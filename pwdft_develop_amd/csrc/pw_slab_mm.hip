@@ -193,6 +193,16 @@ static WgShape wg_shape(const SlabMm* m) {
   }
   return w;
 }
+// Bands too few to fill the chip: one a workgroup, in more workgroups.
+static bool wg_few(const pw_ctx* c, const WgShape& w, int nb) {
+  return (long)c->n3 * ((nb + w.nb - 1) / w.nb) < 256;
+}
+template <typename T>
+static WgShape wg_one(const SlabMm* m, WgShape w) {
+  w.lds -= (w.nb - 1) * mm_wg_band<T>(m->KS, m->TY);
+  w.nb = 1;
+  return w;
+}
 template <typename T>
 using wg_fn = decltype(&k_slab_mm_wg<T, 2, 512>);
 template <typename T>
@@ -235,6 +245,38 @@ bool mm_slab_ready(const pw_ctx* c) {
          (m->KS > 4 && wg_shape<T>(m).nb > 0);
 }
 
+int mm_ksteps(const pw_ctx* c) { return c->mm ? c->mm->KS : 0; }
+
+// The matrix-core kernel's time in us beyond launch and stick traffic, which the
+// LDS kernel has too: a wavefront's products (32 cycles each in FP32, 64 in
+// FP64), the first round and the further ones of what the CUs hold at once; in
+// the workgroup kernel the fourth product, two chains long, and a cost per item
+// by themselves.  Planes of one or two y tiles give the workgroup kernel as few
+// wavefronts a band: never the faster with one (180 x 24 FP32, 24 bands of 24
+// planes, 109 us for 40 in LDS), 1.6 times the estimate in FP32 with two.
+template <typename T>
+double mm_slab_us(const pw_ctx* c, int nb) {
+  const SlabMm* m = c->mm;
+  const int KS = m->KS, TK = (KS + 3) / 4, TX = m->TX, TY = m->TY;
+  const double cyc = (sizeof(T) == 8 ? 64.0 : 32.0) / 2400.0;
+  auto rounds = [](double r) { return r < 8 ? std::max(1.0, std::ceil(r)) : r; };
+  if (!use_wg<T>(c, nb)) {
+    const double w = 4.0 * cyc * (TY * (TK * KS + TX * KS + m->XS * TK) + m->YS * TK * TK);
+    const double r = rounds((double)c->n3 * ((nb + 3) / 4) / 256);
+    return sizeof(T) == 4 ? w * (1.48 + 0.934 * (r - 1)) : w * (1.75 + 1.76 * (r - 1));
+  }
+  if (TY == 1) return 1e30;
+  WgShape w = wg_shape<T>(m);
+  if (wg_few(c, w, nb)) w = wg_one<T>(m, w);
+  const double items = (double)c->n3 * ((nb + w.nb - 1) / w.nb);
+  const int per_cu = std::max(1, std::min((int)(160 * 1024 / w.lds), w.maxt / (64 * w.nb * TY)));
+  const double q = (w.nb * TY + 3) / 4, r = rounds(items / (256.0 * per_cu));
+  const double p3 = 4.0 * cyc * q * (TK * KS + TX * KS + m->XS * TK);
+  const double p4 = 4.0 * cyc * q * m->YS * ((TK * TK + TY - 1) / TY);
+  if (sizeof(T) == 8) return p3 * (1.0 + 1.15 * (r - 1)) + 9.6 * r;
+  return (TY == 2 ? 1.6 : 1.0) * (p3 * (1.31 + 1.49 * (r - 1)) + 2.51 * p4 * r + 4.4 * r);
+}
+
 template <typename T>
 static MmArgs<T> mm_args(const pw_ctx* c, int nb) {
   typedef typename cx<T>::t C;
@@ -253,11 +295,8 @@ int mm_slab(pw_ctx* c, int nb, const void* t1, void* t2) {
   if (use_wg<T>(c, nb)) {
     const auto kwg = wg_kernel<T>(m->KS);
     WgShape w = wg_shape<T>(m);
-    const bool few = (long)c->n3 * ((nb + w.nb - 1) / w.nb) < 256;  // one band each: more workgroups
-    if (few) {
-      w.lds -= (w.nb - 1) * mm_wg_band<T>(m->KS, m->TY);
-      w.nb = 1;
-    }
+    const bool few = wg_few(c, w, nb);
+    if (few) w = wg_one<T>(m, w);
     const int threads = 64 * w.nb * m->TY;
     PW_TRY(ensure_lds((const void*)kwg, w.lds));
     SlabMm::Grid& gw = c->mm->wgrid[d][few];
@@ -328,6 +367,8 @@ template int mm_density<float>(pw_ctx*, int, const void*, const double*, int, do
 template bool mm_slab_ready<double>(const pw_ctx*);
 template bool mm_slab_ready<float>(const pw_ctx*);
 template int mm_slab<double>(pw_ctx*, int, const void*, void*);
+template double mm_slab_us<double>(const pw_ctx*, int);
+template double mm_slab_us<float>(const pw_ctx*, int);
 template int mm_slab<float>(pw_ctx*, int, const void*, void*);
 
 }  // namespace pw

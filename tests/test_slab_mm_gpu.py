@@ -50,6 +50,37 @@ def test_matrix_core_slab_against_oracle(grid, nb):
     ctx.close()
 
 
+@pytest.mark.parametrize("grid,nb", [((72, 24, 24), 5), ((96, 96, 24), 2), ((108, 30, 24), 3), ((30, 108, 12), 3),
+                                     ((150, 32, 10), 30), ((180, 180, 10), 2), ((225, 160, 10), 1),
+                                     ((225, 16, 10), 2), ((16, 225, 10), 5)])
+def test_matrix_core_slab_where_it_is_not_the_faster_one(grid, nb, monkeypatch):
+    """PW_SLAB=mm: the planes that the dispatch leaves to the LDS kernel."""
+    monkeypatch.setenv("PW_SLAB", "mm")
+    test_matrix_core_slab_against_oracle(grid, nb)
+
+
+@pytest.mark.parametrize("grid,nb,dt,kernel", [
+    ((180, 24, 24), 24, "complex64", "lds"), ((180, 32, 24), 24, "complex64", "lds"),
+    ((108, 24, 24), 24, "complex128", "lds"), ((75, 75, 24), 1, "complex128", "lds"),
+    ((72, 72, 24), 2, "complex64", "lds"), ((72, 72, 24), 3, "complex64", "mm"),
+    ((120, 120, 24), 24, "complex64", "mm"), ((180, 90, 24), 24, "complex64", "mm"),
+    ((108, 90, 24), 24, "complex128", "mm"), ((45, 50, 24), 1, "complex128", "mm"),
+    ((16, 60, 24), 2, "complex64", "mm")])
+def test_the_faster_slab_kernel_is_taken(grid, nb, dt, kernel, monkeypatch):
+    """Of two kernels that differ by a quarter or more, by the bits of the result."""
+    import torch
+    from pwdft_develop_amd.ops import Context
+    prob = _problem(grid, nb)
+    out = {}
+    for name in ("", "mm", "lds"):
+        monkeypatch.setenv("PW_SLAB", name)
+        ctx = Context(prob)
+        out[name] = ctx.mult_spinor(ctx.to_device(prob.psi, getattr(torch, dt)))
+        ctx.close()
+    assert not torch.equal(out["mm"], out["lds"])
+    assert torch.equal(out[""], out[kernel])
+
+
 def test_other_half_of_the_kx0_column():
     """Storing (0, -ky, -kz) with the conjugate coefficient in place of
     (0, ky, kz) is the same band: H psi comes back conjugated there alone."""
